@@ -127,6 +127,22 @@ def test_wolff_lds_and_global_paths(vg, orc, ctx):
         assert np.array_equal(b.get_ising(0), st)
 
 
+@pytest.mark.parametrize("kind,dims,pbc,T", [
+    ("fcc", (52, 51, 51), (1, 1, 0), 9.79),  # 541008 sites, open z, at T_c
+    ("fcc", (52, 51, 51), (1, 1, 1), 2.0),   # a cluster of most sites: many pairs a level
+    ("bcc", (66, 64, 63), (0, 1, 1), 6.35),  # 532224 sites, open x
+])
+def test_wolff_global_memory_every_lattice(vg, orc, ctx, kind, dims, pbc, T):
+    OL = orc.lattice(kind, *dims, pbc=pbc)
+    OM = orc.model(terms=("exchange",), temperature=T)
+    st = orc.ising_init(OL, 51)
+    with vg.Batch(ctx, [_chain(vg, kind, dims, pbc, 51)]) as b:
+        b.randomize()
+        b.set_thermostat(0, T)
+        assert np.array_equal(b.run_sums(12)[0], orc.wolff_steps(OL, OM, 51, 0, 12, st))
+        assert np.array_equal(b.get_ising(0), st)
+
+
 def test_wolff_observables_follow_reference_total_energy(vg, orc, ctx):
     """E and |M| per step are the reference's Compound total energy and
     magnetization of the state (the field enters E, not the moves)."""

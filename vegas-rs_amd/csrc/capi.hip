@@ -529,6 +529,30 @@ void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint3
     }
 }
 
+// The Wolff steps of the group's chains of one lattice kind: chains of at
+// most kWolffLdsSites sites in LDS, the rest in global memory; each kernel's
+// blocks skip the other kernels' chains.
+template <uint32_t KIND>
+void launch_wolff(const Group& G, hipStream_t st, uint32_t nsw, int64_t* records) {
+    uint32_t lds_words = 0;
+    bool large = false;
+    for (const ChainDev& d : G.host) {
+        if (d.kind != KIND) continue;
+        if (d.nsites <= vg::kWolffLdsSites)
+            lds_words = std::max(lds_words,
+                                 2u * (uint32_t)((d.nsites + 31) / 32) + vg::kWolffLdsQueue);
+        else
+            large = true;
+    }
+    const dim3 grid((uint32_t)G.members.size()), block(vg::kWolffBlock);
+    if (lds_words)
+        hipLaunchKernelGGL(vg::wolff_run_lds<KIND>, grid, block, lds_words * 4u, st, G.d_chains,
+                           (uint8_t*)G.arena, nsw, records);
+    if (large)
+        hipLaunchKernelGGL(vg::wolff_run<KIND>, grid, block, 0, st, G.d_chains, (uint8_t*)G.arena,
+                           nsw, records);
+}
+
 // Enqueues the sweeps of one block (nsw sweeps, every colour of every group,
 // then the per-chain reductions) on the batch stream.
 int enqueue_block(vg_batch* B, uint32_t nsw) {
@@ -590,24 +614,9 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
         if (G.members.empty()) continue;
         dim3 grid((uint32_t)G.members.size(), nsw);
         if (g == kIsingWolff) {
-            // chains of at most kWolffLdsSites sites in LDS, the rest in
-            // global memory; each kernel's blocks skip the other's chains
-            uint32_t lds_words = 0;
-            bool large = false;
-            for (const ChainDev& d : G.host) {
-                if (d.nsites <= vg::kWolffLdsSites)
-                    lds_words = std::max(lds_words, 2u * (uint32_t)((d.nsites + 31) / 32) +
-                                                        vg::kWolffLdsQueue);
-                else
-                    large = true;
-            }
-            const dim3 chains_grid((uint32_t)G.members.size());
-            if (lds_words)
-                hipLaunchKernelGGL(vg::wolff_run_lds, chains_grid, dim3(256), lds_words * 4u, st,
-                                   G.d_chains, (uint8_t*)G.arena, nsw, B->d_records);
-            if (large)
-                hipLaunchKernelGGL(vg::wolff_run, chains_grid, dim3(256), 0, st, G.d_chains,
-                                   (uint8_t*)G.arena, nsw, B->d_records);
+            launch_wolff<0>(G, st, nsw, B->d_records);
+            launch_wolff<1>(G, st, nsw, B->d_records);
+            launch_wolff<2>(G, st, nsw, B->d_records);
         }
         else if (is_ising(g) && !is_graph(g))
             hipLaunchKernelGGL(vg::ising_reduce, grid, dim3(vg::kBlock), 0, st, G.d_chains,
@@ -1036,9 +1045,13 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
         }
         if (g == kIsingWolff) {
             // the LDS Wolff kernel's dynamic LDS goes past the 64 KiB default
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(vg::wolff_run_lds),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)(vg::kWolffLdsWordsMax * 4u));
+            const void* fns[3] = {reinterpret_cast<const void*>(vg::wolff_run_lds<0>),
+                                  reinterpret_cast<const void*>(vg::wolff_run_lds<1>),
+                                  reinterpret_cast<const void*>(vg::wolff_run_lds<2>)};
+            for (const void* fn : fns)
+                if (e == hipSuccess)
+                    e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)(vg::kWolffLdsWordsMax * 4u));
             if (e != hipSuccess) {
                 free_batch(B);
                 return fail(VG_ERR_DEVICE, "Wolff LDS size: %s", hipGetErrorString(e));

@@ -51,7 +51,10 @@ __global__ void ising_fcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32
 template <uint32_t A>
 __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t);
+// Wolff steps of the chains of one lattice kind (0 sc, 1 bcc, 2 fcc).
+template <uint32_t KIND>
 __global__ void wolff_run(const ChainDev*, uint8_t*, uint32_t, int64_t*);
+template <uint32_t KIND>
 __global__ void wolff_run_lds(const ChainDev*, uint8_t*, uint32_t, int64_t*);
 __global__ void wolff_init(const ChainDev*, uint8_t*);
 __global__ void heis_clear(const ChainDev*, float*);

@@ -186,6 +186,7 @@ constexpr uint32_t kNumXcd = 8;        // MI355X: 8 XCDs, workgroups dealt round
 // first kWolffLdsQueue entries of the cluster queue (31 KiB).
 constexpr uint32_t kWolffLdsSites = 1u << 19;
 constexpr uint32_t kWolffLdsQueue = 7936;
+constexpr uint32_t kWolffBlock = 1024;  // threads per workgroup of the Wolff kernels
 constexpr uint32_t kWolffLdsWordsMax = 2u * (kWolffLdsSites / 32u) + kWolffLdsQueue;
 
 // Exact unsigned division by a per-chain constant d for n < 2^31:
