@@ -40,9 +40,9 @@ CSRC = ROOT / "vegas-rs_amd" / "csrc"
 # The sources each pass kernel is compiled from (the file and the headers it
 # includes): a counter row applies to the build only while they are unchanged.
 KERNEL_SOURCES = {
-    "ising_sc_pass": ["ising_sc.hip", "ising_swar.hpp", "vg_device.hpp"],
-    "ising_bcc_pass": ["ising_bcc.hip", "ising_swar.hpp", "vg_device.hpp"],
-    "ising_fcc_pass": ["ising_fcc.hip", "fcc_common.hpp", "ising_swar.hpp", "vg_device.hpp"],
+    "ising_sc_pass": ["ising_sc.hip", "ising_word.hpp", "vg_device.hpp"],
+    "ising_bcc_pass": ["ising_bcc.hip", "ising_word.hpp", "vg_device.hpp"],
+    "ising_fcc_pass": ["ising_fcc.hip", "fcc_common.hpp", "ising_word.hpp", "vg_device.hpp"],
     "heis_sc_pass": ["heis_sc.hip", "heis_common.hpp", "vg_device.hpp"],
     "heis_bcc_pass": ["heis_bcc.hip", "heis_common.hpp", "vg_device.hpp"],
     "heis_fcc_pass": ["heis_fcc.hip", "fcc_common.hpp", "heis_common.hpp", "vg_device.hpp"],
@@ -104,20 +104,20 @@ def with_counters(roofline, workload, kernels, mads_per_launch=None):
     """Adds the counter-measured traffic (bytes per launch, null when not
     profiled at this tile) and, given the v_mad_u64_u32 count of the launch,
     its VALU ceiling: the time the measured VALU instructions take to issue
-    on every SIMD at the peak clock (4 cycles per wave64 instruction, 16 for
-    v_mad_u64_u32), as a fraction of the measured launch time."""
+    on every SIMD at the peak clock (4 cycles per wave64 instruction; measured
+    4.2, v_mad_u64_u32 4.4, and 2.2 in runs of simple operations with four or
+    more waves on the SIMD), as a fraction of the measured launch time."""
     c = pass_counters(workload, kernels)
     roofline["traffic"] = c["traffic"] if c else None
     roofline["traffic_source"] = c["source"] if c else None
     if c and mads_per_launch is not None:
-        busy_us = (4.0 * c["valu"] + 12.0 * mads_per_launch) / (SIMDS * CLOCK_GHZ * 1e3)
+        busy_us = 4.0 * c["valu"] / (SIMDS * CLOCK_GHZ * 1e3)
         roofline["valu_ceiling"] = {
             "valu_instructions_per_launch": c["valu"],
             "mad_u64_per_launch": mads_per_launch,
             "busy_us": busy_us,
             "frac": busy_us / roofline["mean_launch_us"],
-            "peak": f"{SIMDS} SIMDs x {CLOCK_GHZ} GHz, one wave64 VALU instruction per 4 cycles "
-                    f"(v_mad_u64_u32: 16)",
+            "peak": f"{SIMDS} SIMDs x {CLOCK_GHZ} GHz, one wave64 VALU instruction per 4 cycles",
         }
     return roofline
 
@@ -126,8 +126,8 @@ def ising_mads(attempts_per_launch):
     """v_mad_u64_u32 (wave instructions) of an Ising pass launch with flip
     proposals: one Philox4x32-10 call (20 of them) per 16 sites, 64 lanes per
     wave instruction (tie draws, a few per 10^3 sites, left out).  An upper
-    bound for the sc pass: the multiplies of the first two rounds that do not
-    depend on the row are computed once per z march, not once per plane."""
+    bound: the multiplies of the first two rounds that do not depend on the
+    row are computed once per z march, not once per plane."""
     return 20.0 * attempts_per_launch / 1024.0
 
 
@@ -362,15 +362,14 @@ def run_bitpacked(vg, ctx, side, sweeps):
             {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
              "frac": achieved / HBM_PEAK_GBS, "kernel": "ising_sc_pass<bits>",
              "algorithmic_bytes_per_launch": per_launch // 4, "mean_launch_us": avg_ms * 1e3},
-            "bitpacked", [f"ising_sc_pass<{tile},1>"], ising_mads(per_launch)),
+            "bitpacked", [f"ising_sc_pass<{tile},2>"], ising_mads(per_launch)),
     }
 
 
 def run_resident(vg, ctx, side, sweeps):
     """One int8 Ising chain of sc side^3 at T_c = 4.5115 (J = 1, h = 0, seed
-    7): at 1024^3 the two colour planes (1.07 GB) are far larger than the
-    256 MB Infinity Cache, so every pass streams from HBM.  Attempts/s and
-    the pass kernel's roofline at 2 B per attempt."""
+    7), held one bit per site like every Ising chain: 134 MB at 1024^3.
+    Attempts/s and the pass kernel's roofline at 2 B per attempt."""
     L = vg.lattice(vg.SC, side, side, side)
     n = side ** 3
     with vg.Batch(ctx, [vg.chain(L, vg.ISING, vg.FLIP, vg.hamiltonian(exchange=1.0), 7)]) as b:
@@ -391,7 +390,8 @@ def run_resident(vg, ctx, side, sweeps):
     achieved = 2 * per_launch / (avg_ms * 1e-3) / 1e9
     log(f"resident sc {side}^3: {value:.4e} attempts/s, pass {avg_ms * 1e3:.1f} us, tile {tile}")
     return {
-        "workload": f"ising-sc{side}-i8: one chain sc {side}^3 at T=4.5115, HBM-resident",
+        "workload": (f"ising-sc{side}-i8: one chain sc {side}^3 at T=4.5115 (int8 chain, one bit "
+                     f"per site on the device)"),
         "value": value,
         "unit": "spin-flip attempts/s",
         "sweeps": sweeps,
@@ -462,13 +462,12 @@ def run_heisenberg(vg, ctx, side, sweeps):
 
 def pass_kernels(lattice, spin, tile):
     """The colour-pass kernels of a bcc or fcc line as the counter table names
-    them (fcc: one instantiation per colour)."""
-    bits = 1 if spin == "ising_bits" else 0
-    if lattice == "bcc":
-        return ["heis_bcc_pass"] if spin == "heisenberg" else [f"ising_bcc_pass<{tile},{bits}>"]
+    them: one instantiation per colour (bcc Heisenberg: one kernel for both).
+    Both Ising spin kinds run the periodic bit-plane pass."""
+    colours = range(2 if lattice == "bcc" else 4)
     if spin == "heisenberg":
-        return [f"heis_fcc_pass<{a}>" for a in range(4)]
-    return [f"ising_fcc_pass<{a},{tile},{bits}>" for a in range(4)]
+        return ["heis_bcc_pass"] if lattice == "bcc" else [f"heis_fcc_pass<{a}>" for a in colours]
+    return [f"ising_{lattice}_pass<{a},{tile},2>" for a in colours]
 
 
 def run_fcc(vg, ctx, cells, heis_cells, sweeps, kind=None):
@@ -899,8 +898,9 @@ def main():
         "data": "synthetic (Philox random +-1 start, seed 7)",
         "config": {
             "workload": (f"ising-sc{side}-i8: {len(temps)} chains sc {side}x{side}x{side}, full "
-                         f"PBC, J=1, h=0, int8 spins, seed 7, T={temps}, checkerboard flip "
-                         f"sweeps; one step = one sweep of every chain"),
+                         f"PBC, J=1, h=0, int8 spins (held one bit per site on the device), "
+                         f"seed 7, T={temps}, checkerboard flip sweeps; one step = one sweep "
+                         f"of every chain"),
             "lattice": f"sc {side}^3",
             "chains": len(temps),
             "attempts_per_step": attempts_per_step,

@@ -120,8 +120,8 @@ typedef struct vg_hamiltonian {
 /* ------------------------------------------------------------------ */
 /* Chain = lattice + spin kind + proposal + Hamiltonian + seed.          */
 /* ------------------------------------------------------------------ */
-#define VG_SPIN_ISING 0          /* IsingSpin (state.rs:61-130), int8 arena */
-#define VG_SPIN_ISING_BITS 1     /* IsingSpin, 1 bit per site arena (every lattice) */
+#define VG_SPIN_ISING 0          /* IsingSpin (state.rs:61-130), set and got as int8 */
+#define VG_SPIN_ISING_BITS 1     /* IsingSpin; both kinds are held 1 bit per site */
 #define VG_SPIN_HEISENBERG 2     /* HeisenbergSpin (state.rs:134-192), fp32 xyz */
 
 #define VG_PROPOSAL_FLIP 0       /* MetropolisFlipIntegrator (integrator.rs:100-138) */
@@ -247,20 +247,19 @@ int vg_batch_set_graph(vg_batch* batch, int enabled);
  * autotune) drops the captured graphs. */
 int vg_batch_prepare(vg_batch* batch, uint64_t sweeps);
 /* Tile of the Ising sc, bcc and fcc passes (int8 and bit-packed): z
- * planes marched by one work item (1, 2, 4 or 8; default 4), set for all
- * six groups; get_tile reports the first of them that has chains.  Results
- * do not depend on it. */
+ * planes marched by one work item (1, 2, 4 or 8; by default chosen from the
+ * amount of work in the batch), set for all three groups; get_tile reports
+ * the first of them that has chains.  Results do not depend on it. */
 int vg_batch_set_tile(vg_batch* batch, uint32_t tile);
 int vg_batch_get_tile(const vg_batch* batch, uint32_t* tile);
 /* Times `trial_sweeps` sweeps with every tile (replays of graphs captured
  * beforehand, five rounds over the tiles, the median of each) and keeps the
- * fastest, for each of the six groups.  The chains' spins and sweep counters are
+ * fastest, for each of the three groups.  The chains' spins and sweep counters are
  * restored after every trial, so tuning does not change any trajectory. */
 int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen_tile);
 /* Records (0..128, default 128) the per-wave tie queue of the Ising sc, bcc
  * and fcc passes may hold before a wave settles further tied rows in the
- * lane that found them (each pass holds at most its own queue: 128 records
- * in the sc pass, 64 in the bcc and fcc passes).  No counterpart in the reference; a test hook, so
+ * lane that found them.  No counterpart in the reference; a test hook, so
  * that the queue-overflow path can be checked against the oracle: results
  * do not depend on it.  Drops captured graphs. */
 int vg_batch_set_tie_capacity(vg_batch* batch, uint32_t records);
@@ -278,7 +277,7 @@ int vg_batch_pass_stats(const vg_batch* batch, int32_t spin, double* total_ms, u
 /* that cannot allocate device memory (code under HIP graph capture,     */
 /* tight serving loops, harnesses that forbid hipMalloc).  The sweeps of  */
 /* vg_batch_run_sums for one Metropolis Ising chain (int8 or bit-packed;  */
-/* sc, bcc or fcc; tile 4) on caller-owned device buffers, enqueued on    */
+/* sc, bcc or fcc) on caller-owned device buffers, enqueued on    */
 /* `stream` (a hipStream_t; NULL = the null stream) of the calling        */
 /* thread's current device; the call returns once the work is enqueued.  */
 /*   spins: the chain's colour planes, plane c (c < 2, or < 4 on fcc) at  */
@@ -288,7 +287,9 @@ int vg_batch_pass_stats(const vg_batch* batch, int32_t spin, double* total_ms, u
 /*     x = i on bcc and fcc; w = lx / 2 (sc) or lx positions.  int8: one  */
 /*     byte per position, 1 = Up, 0 = Down, pitch = round_up(w, 64).      */
 /*     Bit-packed: bit (i & 7) of byte i >> 3, pitch = round_up(2 *       */
-/*     ceil(w / 16), 16).  Padding bytes zero.  Updated in place.          */
+/*     ceil(w / 16), 16).  Padding bytes zero.  Updated in place; while    */
+/*     the call's sweeps run, int8 rows hold their bits in their first w/8 */
+/*     bytes.                                                              */
 /*   sums: sweeps * 5 int64, per sweep {bond, 0, 0, mag, 0} as in          */
 /*     vg_sweep_sums (the batch path reports N as the fifth).             */
 /*   sweep0: the chain's sweep counter before the first sweep (Philox).   */

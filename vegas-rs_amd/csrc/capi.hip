@@ -110,28 +110,29 @@ void ising_thresholds(const ChainHost& ch, ChainDev& d) {
                 d.thr[b][S] = (uint32_t)th;
         }
     }
-    // Class plans of the multispin sc pass (z = 6): for a site with g absent
-    // neighbour slots, p = 6 - g present and a of them aligned with its bit b,
-    // the up-neighbour count is c = a (b = 1) or p - a (b = 0) and the class
+    // Class plans of the multispin passes: for a site with g absent neighbour
+    // slots, p = z - g present and a of them aligned with its bit b, the
+    // up-neighbour count is c = a (b = 1) or p - a (b = 0) and the class
     // S = 2c + g.  Classes always accepted are left out.
     std::memset(d.plan, 0, sizeof d.plan);
-    if (z == 6)
-        for (uint32_t g = 0; g < vg::kPlanG; ++g)
-            for (uint32_t a = 0; a <= 6 - g; ++a) {
-                uint32_t slot[2] = {0, 0};
-                for (uint32_t b = 0; b < 2; ++b) {
-                    const uint32_t S = 2 * (b ? a : 6 - g - a) + g;
-                    if ((d.always[b] >> S) & 1u) continue;
-                    const uint32_t th = d.thr[b][S];
-                    slot[b] = (1u << (3 + b)) | ((th != 0 ? 1u : 0u) << 5) | ((th >> 24) << 8);
-                }
-                if (slot[0] && slot[1] && (slot[0] >> 5) == (slot[1] >> 5)) {
-                    d.plan[g][a][0] = slot[0] | slot[1];
-                } else {
-                    d.plan[g][a][0] = slot[0] ? slot[0] : slot[1];
-                    d.plan[g][a][1] = slot[0] ? slot[1] : 0;
-                }
+    for (int g = 0; g <= z; ++g)
+        for (int a = 0; a <= z - g; ++a) {
+            uint32_t slot[2] = {0, 0};
+            for (int b = 0; b < 2; ++b) {
+                const int S = 2 * (b ? a : z - g - a) + g;
+                if ((d.always[b] >> S) & 1u) continue;
+                slot[b] = (1u << (8 + b)) | (d.thr[b][S] >> 24);
             }
+            if (slot[0] && slot[1] && (slot[0] & 0xFFu) == (slot[1] & 0xFFu))
+                d.plan[g][a] = slot[0] | slot[1];
+            else if (slot[0])
+                d.plan[g][a] = slot[0] | (slot[1] << 16);
+            else
+                d.plan[g][a] = slot[1];
+        }
+    d.plain = 1;
+    for (int a = 0; a <= z; ++a)
+        if (2 * a > z ? (d.plan[0][a] >> 8) != 3u : d.plan[0][a] != 0u) d.plain = 0;
 }
 
 // m, s with n / d == (n * m) >> s for every n < 2^31: s = 31 + ceil(log2 d),
@@ -237,26 +238,27 @@ int init_chain_dev(const ChainHost& ch, int g, uint32_t slot, ChainDev& d) {
         }
         return VG_OK;
     }
-    const uint32_t seg = (g == kIsingSc || g == kIsingBits) ? vg::kScSeg
-                         : is_ising(g)                        ? vg::kIsingSeg
-                                                              : vg::kHeisSeg;
-    const uint32_t align = is_ising(g) ? 64u : 16u;  // 64-byte aligned rows
-    if (is_bits(g))  // bytes: whole segments (2 or 4 bytes), 16-byte aligned rows
+    const uint32_t seg = is_ising(g) ? vg::kIsingSeg : vg::kHeisSeg;
+    if (!is_ising(g))
+        d.pitch = (uint32_t)round_up(d.w, 16);  // floats: 64-byte aligned rows
+    else if (ch.byte_planes)
+        d.pitch = (uint32_t)round_up(d.w, 64);
+    else  // bytes: whole words, 16-byte aligned rows
         d.pitch = (uint32_t)round_up((d.w + seg - 1) / seg * (seg / 8), 16);
-    else
-        d.pitch = (uint32_t)round_up(d.w, align);
     d.segs = (d.w + seg - 1) / seg;
-    d.hy = (d.ly + 1) / 2;
-    if ((uint64_t)d.rows * d.segs > 0x7FFFFFFFull - vg::kBlock || (uint64_t)d.rows > 0x7FFFFFFFull)
+    // the seg-16 count bounds what is accepted, as it did for 16-site items
+    const uint64_t halves = is_ising(g) && L.kind != VG_LATTICE_SC ? (d.w + 15) / 16 : d.segs;
+    if ((uint64_t)d.rows * halves > 0x7FFFFFFFull - vg::kBlock || (uint64_t)d.rows > 0x7FFFFFFFull)
         return fail(VG_ERR_INVALID_ARGUMENT, "chain %u too large", slot);
     magic_div(d.segs, d.segs_m, d.segs_s);
     magic_div(d.ly, d.ly_m, d.ly_s);
-    magic_div(d.hy, d.hy_m, d.hy_s);
     d.plane = (uint64_t)d.rows * d.pitch;
-    if (is_ising(g) && d.plane > 0xFFFFF000ull)
+    // int8 chains keep the limit of a byte per site
+    const uint64_t charged = ch.desc.spin == VG_SPIN_ISING ? byte_plane(d) : d.plane;
+    if (is_ising(g) && charged > 0xFFFFF000ull)
         return fail(VG_ERR_UNSUPPORTED_LATTICE,
                     "chain %u: an Ising colour plane of %llu bytes exceeds 4 GiB", slot,
-                    (unsigned long long)d.plane);
+                    (unsigned long long)charged);
     if ((g == kHeisSc || g == kHeisBcc || g == kHeisFcc) && 4 * d.plane > 0xFFFFF000ull)
         return fail(VG_ERR_UNSUPPORTED_LATTICE,
                     "chain %u: a Heisenberg colour plane component of %llu bytes exceeds 4 GiB",
@@ -275,24 +277,10 @@ uint64_t colour_elems(int g, const ChainDev& d) { return (is_ising(g) ? 1 : 3) *
 uint32_t quantities(int group) { return is_ising(group) && !is_graph(group) ? 8u : 5u; }
 uint32_t quantity_bytes(int group) { return is_ising(group) && !is_graph(group) ? 4u : 8u; }
 
-// After the int8 planes of an sc chain with shadows were written: rebuild
-// its shadows (one thread per shadow word).
-void launch_shadow_build(const Group& G, const ChainDev& d, const ChainDev* dp, hipStream_t st) {
-    if (!d.shadow) return;
-    const uint64_t n = 2ull * d.rows * (d.spitch / 4);
-    hipLaunchKernelGGL(vg::ising_shadow_build, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st,
-                       dp, (uint8_t*)G.arena);
-}
-
-void launch_ising_init(int g, const Group& G, const ChainDev& d, const ChainDev* dp,
-                       hipStream_t st) {
+void launch_ising_init(const Group& G, const ChainDev& d, const ChainDev* dp, hipStream_t st) {
     const uint64_t n = (uint64_t)d.ncol * d.plane;  // one thread per plane byte
-    const dim3 grid((uint32_t)((n + 255) / 256));
-    if (is_bits(g))
-        hipLaunchKernelGGL(vg::ising_init_bits, grid, dim3(256), 0, st, dp, (uint8_t*)G.arena);
-    else
-        hipLaunchKernelGGL(vg::ising_init, grid, dim3(256), 0, st, dp, (uint8_t*)G.arena);
-    if (g == kIsingSc) launch_shadow_build(G, d, dp, st);
+    hipLaunchKernelGGL(vg::ising_init, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, dp,
+                       (uint8_t*)G.arena);
 }
 
 int upload_descriptors(vg_batch* B, int g, int slot) {
@@ -305,29 +293,61 @@ int upload_descriptors(vg_batch* B, int g, int slot) {
     return VG_OK;
 }
 
-constexpr uint32_t kDefaultTile = 4;
+// The tile a new batch's Ising group starts with: the largest that leaves the
+// pass at least 7/4 waves per SIMD (1792 on 256 CUs).  Fewer leave SIMDs with
+// one wave or none, which issues an instruction every 8 cycles at best; more
+// planes per wave share its start-up, its tie round and its neighbour rows.
+// Measured, us a pass at tiles 1/2/4/8 and waves at tile 1 (waves at the tile
+// picked): sc 128^3 512: 4.0/4.5/5.5/7.3 (512); sc 256^3 4096: 5.9/5.1/5.7/7.5
+// (2048); two of them 8.9/7.0/6.3/7.7 (2048); three 11.2/9.5/7.4/8.9 (3072);
+// sc 512^3 32768: 25.0/20.8/16.4/13.4 (4096); bcc 161^3 2430: 5.6/5.6/6.2/8.8
+// (2430), three 9.6/8.0/7.5/9.0 (1822); fcc 161^3 2430: 6.0/6.3/6.9/10.4
+// (2430), two 8.1/7.7/8.4/10.5 (2430).  (Tile 4 whatever the size, before.)
+uint32_t default_tile(const ChainDev* chains, size_t n) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        cus = 256;
+    for (uint32_t tile : {8u, 4u, 2u}) {
+        uint64_t items = 0;
+        for (size_t k = 0; k < n; ++k)
+            items += (uint64_t)((chains[k].lz + tile - 1) / tile) * chains[k].ly * chains[k].segs;
+        if (items / 64 >= (uint64_t)cus * 7) return tile;
+    }
+    return 1;
+}
 
-template <uint32_t K>
-const void* zmarch_fn(int g) {
-    switch (g) {
-        case kIsingBits: return (const void*)&vg::ising_sc_pass<K, vg::kScBits>;
-        case kIsingBcc: return (const void*)&vg::ising_bcc_pass<K, false>;
-        case kIsingBccBits: return (const void*)&vg::ising_bcc_pass<K, true>;
-        case kIsingFcc: return (const void*)&vg::ising_fcc_pass<0, K, false>;
-        case kIsingFccBits: return (const void*)&vg::ising_fcc_pass<0, K, true>;
-        default: return (const void*)&vg::ising_sc_pass<K, vg::kScShadow>;
+// The pass kernel of an Ising lattice group for colour c, a tile and a mode.
+template <uint32_t K, uint32_t MODE>
+const void* zmarch_fn_mode(int g, uint32_t c) {
+    if (g == kIsingSc) return (const void*)&vg::ising_sc_pass<K, MODE>;
+    if (g == kIsingBcc)
+        return c ? (const void*)&vg::ising_bcc_pass<1, K, MODE>
+                 : (const void*)&vg::ising_bcc_pass<0, K, MODE>;
+    switch (c) {
+        case 0: return (const void*)&vg::ising_fcc_pass<0, K, MODE>;
+        case 1: return (const void*)&vg::ising_fcc_pass<1, K, MODE>;
+        case 2: return (const void*)&vg::ising_fcc_pass<2, K, MODE>;
+        default: return (const void*)&vg::ising_fcc_pass<3, K, MODE>;
+    }
+}
+
+const void* zmarch_fn(int g, uint32_t tile, uint32_t mode, uint32_t c) {
+    const bool per = mode == 2;
+    switch (tile) {
+        case 1: return per ? zmarch_fn_mode<1, 2>(g, c) : zmarch_fn_mode<1, 1>(g, c);
+        case 2: return per ? zmarch_fn_mode<2, 2>(g, c) : zmarch_fn_mode<2, 1>(g, c);
+        case 8: return per ? zmarch_fn_mode<8, 2>(g, c) : zmarch_fn_mode<8, 1>(g, c);
+        default: return per ? zmarch_fn_mode<4, 2>(g, c) : zmarch_fn_mode<4, 1>(g, c);
     }
 }
 
 // Whether `grid` workgroups of group g's z-marching Ising pass with this tile
 // are all resident at once on the current device.
-bool all_resident(int g, uint32_t tile, uint32_t grid) {
-    const void* fn = tile == 1   ? zmarch_fn<1>(g)
-                     : tile == 2 ? zmarch_fn<2>(g)
-                     : tile == 8 ? zmarch_fn<8>(g)
-                                 : zmarch_fn<4>(g);
+bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid) {
     int nb = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, vg::kBlock, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, zmarch_fn(g, tile, G.mode, 0), vg::kBlock,
+                                                     0) != hipSuccess ||
         hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return false;
@@ -349,10 +369,7 @@ int layout_work(vg_batch* B, int g, uint32_t tile) {
             items = d.items;  // one thread per site of the largest colour class (set at creation)
         } else if (is_zmarch(g)) {
             d.nzc = (d.lz + tile - 1) / tile;
-            // sc: rows in natural order; bcc, fcc: the rows of one y parity,
-            // then the other (2 * hy rows, the last one past an odd ly idle)
-            const bool sc = g == kIsingSc || g == kIsingBits;
-            items = (uint64_t)d.nzc * (sc ? d.ly : 2 * d.hy) * d.segs;
+            items = (uint64_t)d.nzc * d.ly * d.segs;
         } else {
             items = (uint64_t)d.rows * d.segs;
         }
@@ -375,10 +392,16 @@ int layout_work(vg_batch* B, int g, uint32_t tile) {
     G.tile = tile;
     G.total_blocks = (uint32_t)block_chain.size();
     G.grid = (uint32_t)round_up(G.total_blocks, vg::kNumXcd);
-    G.uniform_nb = G.host.empty() ? 0u : G.host[0].nblocks;
-    for (const ChainDev& d : G.host)
-        if (d.nblocks != G.uniform_nb) G.uniform_nb = 0;
-    if (is_zmarch(g)) G.prio = all_resident(g, tile, G.grid) ? 1u : 0u;
+    bool uniform = !G.host.empty();
+    for (const ChainDev& d : G.host) uniform = uniform && d.nblocks == G.host[0].nblocks;
+    G.chain_m = G.chain_s = 0;
+    if (uniform) magic_div(G.host[0].nblocks, G.chain_m, G.chain_s);
+    if (is_zmarch(g)) {
+        G.mode = 2;  // vg::kPeriodic when every chain is, else vg::kOpen
+        for (const ChainDev& d : G.host)
+            if ((d.pbc & 7u) != 7u) G.mode = 1;
+        G.prio = all_resident(g, G, tile, G.grid) ? 1u : 0u;
+    }
     G.partial_bytes_per_sweep = std::max<uint64_t>(
         256, (uint64_t)passes_of(G, g) * G.total_blocks * quantities(g) * quantity_bytes(g));
     for (auto& kv : B->graphs) quiet(hipGraphExecDestroy(kv.second));
@@ -407,126 +430,28 @@ int free_batch(vg_batch* B) {
     return VG_OK;
 }
 
-template <uint32_t MODE>
-void launch_sc_mode(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
-    const dim3 grid(G.grid), block(vg::kBlock);
-    uint8_t* arena = (uint8_t*)G.arena;
-    int32_t* part = (int32_t*)G.partials;
-    const uint32_t opts = G.prio | (G.tie_cap << 8);
-    switch (G.tile) {
-        case 1:
-            hipLaunchKernelGGL((vg::ising_sc_pass<1, MODE>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid, opts,
-                               G.uniform_nb);
-            break;
-        case 2:
-            hipLaunchKernelGGL((vg::ising_sc_pass<2, MODE>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid, opts,
-                               G.uniform_nb);
-            break;
-        case 8:
-            hipLaunchKernelGGL((vg::ising_sc_pass<8, MODE>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid, opts,
-                               G.uniform_nb);
-            break;
-        default:
-            hipLaunchKernelGGL((vg::ising_sc_pass<4, MODE>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid, opts,
-                               G.uniform_nb);
-            break;
-    }
-}
-
-// One colour pass of an sc Ising group: bit-packed planes, or int8 planes
-// with or without shadows.
-template <bool BITS>
-void launch_ising_pass(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
-    if (BITS)
-        launch_sc_mode<vg::kScBits>(G, st, c, s);
-    else if (G.shadow)
-        launch_sc_mode<vg::kScShadow>(G, st, c, s);
-    else
-        launch_sc_mode<vg::kScInt8>(G, st, c, s);
-}
-
-template <bool BITS>
-void launch_bcc_pass(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
-    const dim3 grid(G.grid), block(vg::kBlock);
-    uint8_t* arena = (uint8_t*)G.arena;
-    int32_t* part = (int32_t*)G.partials;
-    switch (G.tile) {
-        case 1:
-            hipLaunchKernelGGL((vg::ising_bcc_pass<1, BITS>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid,
-                               G.prio | (G.tie_cap << 8));
-            break;
-        case 2:
-            hipLaunchKernelGGL((vg::ising_bcc_pass<2, BITS>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid,
-                               G.prio | (G.tie_cap << 8));
-            break;
-        case 8:
-            hipLaunchKernelGGL((vg::ising_bcc_pass<8, BITS>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid,
-                               G.prio | (G.tie_cap << 8));
-            break;
-        default:
-            hipLaunchKernelGGL((vg::ising_bcc_pass<4, BITS>), grid, block, 0, st, G.d_chains,
-                               G.d_block_chain, arena, part, c, s, G.total_blocks, G.grid,
-                               G.prio | (G.tie_cap << 8));
-            break;
-    }
-}
-
-template <uint32_t A, uint32_t K, bool BITS>
-void launch_ising_fcc(const Group& G, hipStream_t st, uint32_t s) {
-    hipLaunchKernelGGL((vg::ising_fcc_pass<A, K, BITS>), dim3(G.grid), dim3(vg::kBlock), 0, st,
-                       G.d_chains, G.d_block_chain, (uint8_t*)G.arena, (int32_t*)G.partials, s,
-                       G.total_blocks, G.grid, G.prio | (G.tie_cap << 8));
-}
-
-template <uint32_t A, bool BITS>
-void launch_ising_fcc_tile(const Group& G, hipStream_t st, uint32_t s) {
-    switch (G.tile) {
-        case 1: launch_ising_fcc<A, 1, BITS>(G, st, s); break;
-        case 2: launch_ising_fcc<A, 2, BITS>(G, st, s); break;
-        case 8: launch_ising_fcc<A, 8, BITS>(G, st, s); break;
-        default: launch_ising_fcc<A, 4, BITS>(G, st, s); break;
-    }
-}
-
-// kind: 0 Ising int8, 1 Ising bit-packed, 2 Heisenberg.
-template <uint32_t A>
-void launch_fcc_colour(const Group& G, hipStream_t st, uint32_t s, int kind) {
-    const dim3 grid(G.grid), block(vg::kBlock);
-    if (kind == 0)
-        launch_ising_fcc_tile<A, false>(G, st, s);
-    else if (kind == 1)
-        launch_ising_fcc_tile<A, true>(G, st, s);
-    else
-        hipLaunchKernelGGL(vg::heis_fcc_pass<A>, grid, block, 0, st, G.d_chains, G.d_block_chain,
-                           (float*)G.arena, (int64_t*)G.partials, s, G.total_blocks, G.grid);
-}
-
-void launch_fcc_pass(const Group& G, hipStream_t st, uint32_t c, uint32_t s, int kind) {
-    switch (c) {
-        case 0: launch_fcc_colour<0>(G, st, s, kind); break;
-        case 1: launch_fcc_colour<1>(G, st, s, kind); break;
-        case 2: launch_fcc_colour<2>(G, st, s, kind); break;
-        default: launch_fcc_colour<3>(G, st, s, kind); break;
-    }
-}
-
-// One colour pass of a z-marching Ising group (sc, bcc, fcc; int8 or bits).
+// One colour pass of an Ising lattice group.
 void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s) {
-    switch (g) {
-        case kIsingBits: launch_ising_pass<true>(G, st, c, s); break;
-        case kIsingBcc: launch_bcc_pass<false>(G, st, c, s); break;
-        case kIsingBccBits: launch_bcc_pass<true>(G, st, c, s); break;
-        case kIsingFcc: launch_fcc_pass(G, st, c, s, 0); break;
-        case kIsingFccBits: launch_fcc_pass(G, st, c, s, 1); break;
-        default: launch_ising_pass<false>(G, st, c, s); break;
-    }
+    const ChainDev* chains = G.d_chains;
+    const uint32_t* map = G.d_block_chain;
+    uint8_t* arena = (uint8_t*)G.arena;
+    int32_t* part = (int32_t*)G.partials;
+    uint32_t nb = G.chain_m, total = G.total_blocks, grid = G.grid;
+    uint32_t opts = G.prio | (G.tie_cap << 8) | (G.chain_s << 16);
+    void* sc[] = {&chains, &map, &arena, &part, &c, &s, &total, &grid, &opts, &nb};
+    void* other[] = {&chains, &map, &arena, &part, &s, &total, &grid, &opts, &nb};
+    // an error stays behind for the caller's hipGetLastError
+    quiet(hipLaunchKernel(zmarch_fn(g, G.tile, G.mode, c), dim3(grid), dim3(vg::kBlock),
+                          g == kIsingSc ? sc : other, 0, st));
+}
+
+void launch_heis_fcc(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
+    const auto fn = c == 0   ? vg::heis_fcc_pass<0>
+                    : c == 1 ? vg::heis_fcc_pass<1>
+                    : c == 2 ? vg::heis_fcc_pass<2>
+                             : vg::heis_fcc_pass<3>;
+    hipLaunchKernelGGL(fn, dim3(G.grid), dim3(vg::kBlock), 0, st, G.d_chains, G.d_block_chain,
+                       (float*)G.arena, (int64_t*)G.partials, s, G.total_blocks, G.grid);
 }
 
 // The Wolff steps of the group's chains of one lattice kind: chains of at
@@ -572,18 +497,8 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
                     VG_HIP(hipEventRecord(B->pass_events[k], st));
                 }
                 const dim3 grid(G.grid), block(vg::kBlock);
-                if (g == kIsingSc)
-                    launch_ising_pass<false>(G, st, c, s);
-                else if (g == kIsingBits)
-                    launch_ising_pass<true>(G, st, c, s);
-                else if (g == kIsingBcc)
-                    launch_bcc_pass<false>(G, st, c, s);
-                else if (g == kIsingBccBits)
-                    launch_bcc_pass<true>(G, st, c, s);
-                else if (g == kIsingFcc)
-                    launch_fcc_pass(G, st, c, s, 0);
-                else if (g == kIsingFccBits)
-                    launch_fcc_pass(G, st, c, s, 1);
+                if (is_zmarch(g))
+                    launch_zmarch_pass(G, g, st, c, s);
                 else if (g == kHeisSc)
                     hipLaunchKernelGGL(vg::heis_sc_pass, grid, block, 0, st, G.d_chains,
                                        G.d_block_chain, (float*)G.arena, (int64_t*)G.partials,
@@ -601,7 +516,7 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
                                        G.d_chains, G.d_block_chain, (uint8_t*)G.arena,
                                        (int64_t*)G.partials, c, s, G.total_blocks, G.npass);
                 else
-                    launch_fcc_pass(G, st, c, s, 2);
+                    launch_heis_fcc(G, st, c, s);
                 if (timed) {
                     VG_HIP(hipEventRecord(B->pass_events[B->pass_events_used + 1], st));
                     B->pass_events_used += 2;
@@ -1019,16 +934,6 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
                 d.off[c] = offset;
                 offset += colour_elems(g, d);
             }
-            if (g == kIsingSc) {  // bit-packed shadows of the two planes
-                d.spitch = (uint32_t)round_up((d.w + 31) / 32 * 4, 16);
-                for (uint32_t c = 0; c < 2; ++c) {
-                    offset = round_up(offset, elem_align);
-                    d.soff[c] = offset;
-                    offset += (uint64_t)d.rows * d.spitch;
-                }
-                d.shadow = 1;
-                G.shadow = true;
-            }
         }
         G.arena_bytes = std::max<uint64_t>(offset * elem_bytes(g), 256);
         hipError_t e = hipMalloc(&G.arena, G.arena_bytes);
@@ -1087,7 +992,7 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             return fail(VG_ERR_OUT_OF_MEMORY, "allocating partial sums: %s", hipGetErrorString(e));
         }
         if (is_zmarch(g)) {
-            int rc = layout_work(B, g, kDefaultTile);
+            int rc = layout_work(B, g, default_tile(G.host.data(), G.host.size()));
             if (rc) {
                 free_batch(B);
                 return rc;
@@ -1216,7 +1121,7 @@ int vg_batch_randomize(vg_batch* batch) {
             hipLaunchKernelGGL(vg::graph_heis_init, dim3((uint32_t)((d.nsites + 255) / 256)),
                                dim3(256), 0, st, dp, (uint8_t*)G.arena);
         } else if (is_ising(ch.group)) {
-            launch_ising_init(ch.group, G, d, dp, st);
+            launch_ising_init(G, d, dp, st);
         } else {
             const uint64_t n = (uint64_t)d.ncol * d.rows * d.w;
             hipLaunchKernelGGL(vg::heis_init, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st,
@@ -1262,17 +1167,9 @@ int vg_batch_set_ising(vg_batch* batch, uint32_t chain, const int8_t* spins) {
     VG_HIP(hipMalloc(&tmp, ch.n_sites));
     hipError_t e = hipMemcpyAsync(tmp, spins, ch.n_sites, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {
-        if (is_bits(ch.group)) {
-            const uint64_t nb = (uint64_t)G.host[ch.index].ncol * G.host[ch.index].plane;
-            hipLaunchKernelGGL(vg::ising_scatter_bits, dim3((uint32_t)((nb + 255) / 256)),
-                               dim3(256), 0, st, G.d_chains + ch.index, (uint8_t*)G.arena, tmp);
-        } else {
-            hipLaunchKernelGGL(vg::ising_scatter, dim3((uint32_t)((ch.n_sites + 255) / 256)),
-                               dim3(256), 0, st, G.d_chains + ch.index, (uint8_t*)G.arena, tmp,
-                               ch.n_sites);
-            if (ch.group == kIsingSc)
-                launch_shadow_build(G, G.host[ch.index], G.d_chains + ch.index, st);
-        }
+        const uint64_t nb = (uint64_t)G.host[ch.index].ncol * G.host[ch.index].plane;
+        hipLaunchKernelGGL(vg::ising_scatter, dim3((uint32_t)((nb + 255) / 256)), dim3(256), 0, st,
+                           G.d_chains + ch.index, (uint8_t*)G.arena, tmp);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1308,14 +1205,8 @@ int vg_batch_get_ising(vg_batch* batch, uint32_t chain, int8_t* spins) {
     }
     int8_t* tmp = nullptr;
     VG_HIP(hipMalloc(&tmp, ch.n_sites));
-    if (is_bits(ch.group))
-        hipLaunchKernelGGL(vg::ising_gather_bits, dim3((uint32_t)((ch.n_sites + 255) / 256)),
-                           dim3(256), 0, st, G.d_chains + ch.index, (const uint8_t*)G.arena, tmp,
-                           ch.n_sites);
-    else
-        hipLaunchKernelGGL(vg::ising_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)),
-                           dim3(256), 0, st, G.d_chains + ch.index, (const uint8_t*)G.arena, tmp,
-                           ch.n_sites);
+    hipLaunchKernelGGL(vg::ising_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256), 0,
+                       st, G.d_chains + ch.index, (const uint8_t*)G.arena, tmp, ch.n_sites);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(spins, tmp, ch.n_sites, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1473,7 +1364,7 @@ int vg_batch_set_tile(vg_batch* batch, uint32_t tile) {
     if (tile != 1 && tile != 2 && tile != 4 && tile != 8)
         return fail(VG_ERR_INVALID_ARGUMENT, "tile must be 1, 2, 4 or 8 (got %u)", tile);
     VG_HIP(hipSetDevice(batch->ctx->device));
-    for (int g : {kIsingSc, kIsingBits, kIsingBcc, kIsingBccBits, kIsingFcc, kIsingFccBits}) {
+    for (int g : kZmarchGroups) {
         if (batch->groups[g].members.empty()) continue;
         int rc = layout_work(batch, g, tile);
         if (rc) return rc;
@@ -1482,10 +1373,9 @@ int vg_batch_set_tile(vg_batch* batch, uint32_t tile) {
 }
 
 // The group whose tile vg_batch_get_tile and vg_batch_autotune report: the
-// first of the z-marching Ising groups (sc, bcc, fcc; int8, then bit-packed)
-// that has chains.
+// first of the Ising lattice groups (sc, bcc, fcc) that has chains.
 static int tile_group(const vg_batch* batch) {
-    for (int g : {kIsingSc, kIsingBits, kIsingBcc, kIsingBccBits, kIsingFcc, kIsingFccBits})
+    for (int g : kZmarchGroups)
         if (!batch->groups[g].members.empty()) return g;
     return kIsingSc;
 }
@@ -1501,7 +1391,7 @@ int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen) 
     uint32_t tile_now = 0;
     vg_batch_get_tile(batch, &tile_now);
     bool any = false;
-    for (int g : {kIsingSc, kIsingBits, kIsingBcc, kIsingBccBits, kIsingFcc, kIsingFccBits})
+    for (int g : kZmarchGroups)
         any = any || !batch->groups[g].members.empty();
     if (!any || trial_sweeps == 0) {
         if (chosen) *chosen = tile_now;
@@ -1544,7 +1434,7 @@ int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen) 
     batch->use_graph = true;
     hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) rc = fail(VG_ERR_DEVICE, "autotune backup: %s", hipGetErrorString(e));
-    for (int g : {kIsingSc, kIsingBits, kIsingBcc, kIsingBccBits, kIsingFcc, kIsingFccBits}) {
+    for (int g : kZmarchGroups) {
         Group& G = batch->groups[g];
         if (G.members.empty() || rc != VG_OK) continue;
         const uint32_t start_tile = G.tile;

@@ -19,35 +19,31 @@
 
 namespace vg {
 // sc pass args: (chains, block -> chain map, arena, partials, colour, sweep,
-// total blocks, grid, options, blocks per chain when uniform else 0).
+// total blocks, grid, options, magic of the blocks per chain or 0).
 template <uint32_t K, uint32_t MODE>
 __global__ void ising_sc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32_t*, uint32_t,
                               uint32_t, uint32_t, uint32_t, uint32_t, uint32_t);
-// Packs the int8 sc planes of one chain into its shadows.
-__global__ void ising_shadow_build(const ChainDev*, uint8_t*);
-__global__ void ising_init_bits(const ChainDev*, uint8_t*);
-__global__ void ising_scatter_bits(const ChainDev*, uint8_t*, const int8_t*);
-__global__ void ising_gather_bits(const ChainDev*, const uint8_t*, int8_t*, uint64_t);
 __global__ void ising_reduce(const ChainDev*, const int32_t*, uint32_t, uint32_t, uint32_t,
                              int64_t*);
 __global__ void ising_init(const ChainDev*, uint8_t*);
-__global__ void ising_scatter(const ChainDev*, uint8_t*, const int8_t*, uint64_t);
+__global__ void ising_scatter(const ChainDev*, uint8_t*, const int8_t*);
 __global__ void ising_gather(const ChainDev*, const uint8_t*, int8_t*, uint64_t);
 __global__ void heis_sc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                              uint32_t, uint32_t, uint32_t);
-template <uint32_t K, bool BITS>
+// bcc and fcc passes: one instantiation per colour A (sublattice), args as
+// the sc pass's without the colour.
+template <uint32_t A, uint32_t K, uint32_t MODE>
 __global__ void ising_bcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32_t*, uint32_t,
                                uint32_t, uint32_t, uint32_t, uint32_t);
 __global__ void heis_bcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t, uint32_t);
 __global__ void heis_reduce(const ChainDev*, const int64_t*, uint32_t, uint32_t, uint32_t,
                             int64_t*);
-// fcc passes: one instantiation per colour A (sublattice), args (chains,
-// block -> chain map, arena, partials, sweep, total blocks, grid[, wave
-// priorities on]).
-template <uint32_t A, uint32_t K, bool BITS>
+template <uint32_t A, uint32_t K, uint32_t MODE>
 __global__ void ising_fcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32_t*, uint32_t,
-                               uint32_t, uint32_t, uint32_t);
+                               uint32_t, uint32_t, uint32_t, uint32_t);
+// One instantiation per colour A, args (chains, block -> chain map, arena,
+// partials, sweep, total blocks, grid).
 template <uint32_t A>
 __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t);
@@ -98,42 +94,34 @@ inline void quiet(hipError_t) {}
 
 // Kernel groups: chains of one group share an arena and one pass kernel.
 enum GroupKind {
-    kIsingSc = 0,
+    kIsingSc = 0,  // Ising lattice groups: both Ising spin kinds, one bit per site
     kHeisSc = 1,
     kIsingBcc = 2,
     kHeisBcc = 3,
-    kIsingBits = 4,  // sc, 1 bit per site
-    kIsingFcc = 5,
-    kHeisFcc = 6,
-    kIsingWolff = 7,  // Wolff cluster steps, any lattice, natural site order
-    kIsingBccBits = 8,  // bcc, 1 bit per site
-    kIsingFccBits = 9,  // fcc, 1 bit per site
-    kIsingGraph = 10,   // arbitrary exchange matrix, int8 Ising, colour classes
-    kHeisGraph = 11,    // arbitrary exchange matrix, fp32 Heisenberg
-    kNumGroups = 12
+    kIsingFcc = 4,
+    kHeisFcc = 5,
+    kIsingWolff = 6,  // Wolff cluster steps, any lattice, natural site order
+    kIsingGraph = 7,  // arbitrary exchange matrix, int8 Ising, colour classes
+    kHeisGraph = 8,   // arbitrary exchange matrix, fp32 Heisenberg
+    kNumGroups = 9
 };
 
 inline bool is_ising(int g) {
-    return g == kIsingSc || g == kIsingBcc || g == kIsingBits || g == kIsingFcc ||
-           g == kIsingWolff || g == kIsingBccBits || g == kIsingFccBits || g == kIsingGraph;
+    return g == kIsingSc || g == kIsingBcc || g == kIsingFcc || g == kIsingWolff ||
+           g == kIsingGraph;
 }
 // Groups of chains whose exchange is a matrix (VG_LATTICE_GRAPH).
 inline bool is_graph(int g) { return g == kIsingGraph || g == kHeisGraph; }
-// Groups whose planes hold one bit per site.
-inline bool is_bits(int g) {
-    return g == kIsingBits || g == kIsingBccBits || g == kIsingFccBits;
-}
-// Groups whose pass marches a tile of z planes per work item.
-inline bool is_zmarch(int g) {
-    return g == kIsingSc || g == kIsingBits || g == kIsingBcc || g == kIsingFcc ||
-           g == kIsingBccBits || g == kIsingFccBits;
-}
+// Ising lattice groups: planes of one bit per site, a pass that marches a
+// tile of z planes per work item.
+inline bool is_zmarch(int g) { return g == kIsingSc || g == kIsingBcc || g == kIsingFcc; }
+constexpr int kZmarchGroups[] = {kIsingSc, kIsingBcc, kIsingFcc};
 // Colours (planes, passes per sweep) of a lattice group's chains; Wolff
 // chains have no colour passes; graph groups keep theirs in Group::npass.
 inline uint32_t colours_of(int g) {
     return g == kIsingWolff || is_graph(g)
                ? 0u
-               : (g == kIsingFcc || g == kHeisFcc || g == kIsingFccBits ? 4u : 2u);
+               : (g == kIsingFcc || g == kHeisFcc ? 4u : 2u);
 }
 
 inline int group_of(const vg_chain_desc& d) {
@@ -142,8 +130,6 @@ inline int group_of(const vg_chain_desc& d) {
     if (d.proposal == VG_PROPOSAL_WOLFF) return kIsingWolff;
     if (d.spin == VG_SPIN_HEISENBERG)
         return k == VG_LATTICE_FCC ? kHeisFcc : (k == VG_LATTICE_BCC ? kHeisBcc : kHeisSc);
-    if (d.spin == VG_SPIN_ISING_BITS)
-        return k == VG_LATTICE_FCC ? kIsingFccBits : (k == VG_LATTICE_BCC ? kIsingBccBits : kIsingBits);
     return k == VG_LATTICE_FCC ? kIsingFcc : (k == VG_LATTICE_BCC ? kIsingBcc : kIsingSc);
 }
 
@@ -161,15 +147,18 @@ struct Group {
     ChainDev* h_staging2 = nullptr;  // second one, for the block after (batches)
     uint32_t* d_block_chain = nullptr;
     uint32_t block_chain_cap = 0;
-    uint32_t tile = 4;  // Ising sc/bcc/fcc (int8, bits): z planes per work item (template parameter)
+    uint32_t tile = 4;  // Ising sc/bcc/fcc: z planes per work item (template parameter)
+    // Ising sc/bcc/fcc: the pass's form (vg::IsingMode) -- one bit per site,
+    // with every chain periodic along every axis or not, or the caller's byte
+    // planes (the allocation-free entry point)
+    uint32_t mode = 1;
     uint32_t total_blocks = 0;
     uint32_t grid = 0;  // total_blocks rounded up to a multiple of 8
-    // blocks per chain when every chain of the group has the same number (a
-    // pass then finds a block's chain without the map), else 0
-    uint32_t uniform_nb = 0;
+    // division by the blocks per chain when every chain of the group has the
+    // same number (a pass then finds a block's chain without the map), else 0
+    uint32_t chain_m = 0, chain_s = 0;
     uint32_t prio = 0;  // z-marching Ising passes: every workgroup resident at once (wave priorities on)
-    // z-marching Ising passes: tie records a wave may queue (each pass holds
-    // at most its own queue: 128 records in the sc pass, 64 in bcc and fcc)
+    // z-marching Ising passes: tie records a wave may queue (at most 128)
     uint32_t tie_cap = 128;
     uint32_t npass = 0;     // graph groups: passes per sweep (the most colours of a member)
     void* arena = nullptr;
@@ -181,9 +170,6 @@ struct Group {
     uint32_t chains_cap = 0;
     uint64_t partial_cap = 0;
     bool shared_arena = false;  // arena is owned by someone else (the server's pool)
-    // int8 sc chains with bit-packed plane shadows (batches; the server's
-    // pooled chains have none)
-    bool shadow = false;
 };
 
 struct ChainHost {
@@ -195,6 +181,9 @@ struct ChainHost {
     double field_dir[3] = {0.0, 0.0, 1.0};
     int group = 0;
     uint32_t index = 0;  // index in its group
+    // The planes are the caller's, with rows of one byte per site (the
+    // allocation-free entry point, which keeps a row's bits at its start).
+    bool byte_planes = false;
     // Graph chains: sum of the matrix's diagonal (a constant -J_ii in every
     // e_i) and the position of each site in the colour-sorted order.
     double diag = 0.0;
@@ -248,6 +237,8 @@ struct GraphBuild {
 };
 int build_graph(const vg_csr& m, GraphBuild& out);
 
+// m, s with n / d == (n * m) >> s for every n < 2^31.
+void magic_div(uint32_t d, uint32_t& m, uint32_t& s);
 int validate_desc(const vg_chain_desc& d);
 int coordination(int kind);
 void refresh_params(vg_batch* B, uint32_t i);
@@ -256,9 +247,8 @@ void refresh_params(vg_batch* B, uint32_t i);
 void ising_thresholds(const ChainHost& ch, ChainDev& d);
 void heis_params(const ChainHost& ch, ChainDev& d);
 int free_batch(vg_batch* B);
-// Random initial state (State::rand_with_size) of an Ising chain of group g.
-void launch_ising_init(int g, const Group& G, const ChainDev& d, const ChainDev* dp,
-                       hipStream_t st);
+// Random initial state (State::rand_with_size) of an Ising lattice chain.
+void launch_ising_init(const Group& G, const ChainDev& d, const ChainDev* dp, hipStream_t st);
 uint32_t quantities(int group);
 uint32_t quantity_bytes(int group);
 // Copies group g's descriptors to the device through pinned staging buffer
@@ -267,7 +257,7 @@ int upload_descriptors(vg_batch* B, int g, int slot = 0);
 int layout_work(vg_batch* B, int g, uint32_t tile);
 // Whether `grid` workgroups of group g's z-marching pass at this tile are all
 // resident at once (the falling wave priorities are used only then).
-bool all_resident(int g, uint32_t tile, uint32_t grid);
+bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid);
 void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s);
 int enqueue_block(vg_batch* B, uint32_t nsw);
 int launch_block(vg_batch* B, uint32_t nsw);
@@ -276,8 +266,15 @@ void observables(const ChainHost& ch, const vg_sweep_sums& r, double* E, double*
 // Geometry and parameters of chain `ch` as member `slot` of group g (sizes,
 // magic divisors, acceptance tables); the plane offsets are set by the caller.
 int init_chain_dev(const ChainHost& ch, int g, uint32_t slot, ChainDev& d);
+// The tile an Ising lattice group of n chains starts with.
+uint32_t default_tile(const ChainDev* chains, size_t n);
 // Elements (bytes for Ising, floats for Heisenberg) of one colour of a chain.
 uint64_t colour_elems(int g, const ChainDev& d);
+// Bytes of one colour plane of an Ising chain at one byte per site: what an
+// int8 chain is charged for and limited by.
+inline uint64_t byte_plane(const ChainDev& d) {
+    return (uint64_t)d.rows * round_up(d.w, 64);
+}
 // Bytes of one element in group g's arena.
 inline uint64_t elem_bytes(int g) { return is_ising(g) || is_graph(g) ? 1 : 4; }
 

@@ -36,46 +36,7 @@ __device__ __forceinline__ Where locate(const ChainDev& C, uint64_t n) {
     return r;
 }
 
-// Ising initial state: position i of row `row` in plane c is Up iff word
-// (i & 3) of Philox(key = seed, ctr = (i >> 2, row, 0, w(0, init, c))) is
-// below 2^31 (Spin::rand draws Up when its uniform is below 1/2).
-__global__ void ising_init(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena) {
-    const ChainDev& C = *chain;
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t per_plane = (uint64_t)C.rows * C.pitch;
-    if (idx >= C.ncol * per_plane) return;
-    const uint32_t c = (uint32_t)(idx / per_plane);
-    const uint64_t e = idx - c * per_plane;
-    const uint32_t row = (uint32_t)(e / C.pitch);
-    const uint32_t i = (uint32_t)(e % C.pitch);
-    uint8_t v = 0;
-    if (i < C.w) {
-        const U4 r = philox(U4{i >> 2, row, 0u, ctr_w(0, kIsingInit, c)}, (uint32_t)C.seed,
-                            (uint32_t)(C.seed >> 32));
-        v = (u4_word(r, i & 3u) >> 31) == 0 ? 1 : 0;
-    }
-    arena[C.off[c] + e] = v;
-}
-
-__global__ void ising_scatter(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena,
-                              const int8_t* __restrict__ natural, uint64_t n_sites) {
-    const ChainDev& C = *chain;
-    const uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= n_sites) return;
-    const Where p = locate(C, n);
-    arena[C.off[p.c] + (uint64_t)p.row * C.pitch + p.i] = natural[n] > 0 ? 1 : 0;
-}
-
-__global__ void ising_gather(const ChainDev* __restrict__ chain, const uint8_t* __restrict__ arena,
-                             int8_t* __restrict__ natural, uint64_t n_sites) {
-    const ChainDev& C = *chain;
-    const uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= n_sites) return;
-    const Where p = locate(C, n);
-    natural[n] = arena[C.off[p.c] + (uint64_t)p.row * C.pitch + p.i] ? 1 : -1;
-}
-
-// Bit-packed Ising planes: position i of a row is bit (i & 7) of byte i >> 3.
+// Ising planes: position i of a row is bit (i & 7) of byte i >> 3.
 // One thread per plane byte; bits past w stay zero.
 
 // Natural site id of position i of row `row` of colour c: sc x + lx*(y +
@@ -92,9 +53,10 @@ __device__ __forceinline__ uint64_t plane_site(const ChainDev& C, uint32_t c, ui
            c;
 }
 
-// The same draws as ising_init: position i is Up iff word (i & 3) of
-// Philox(key = seed, ctr = (i >> 2, row, 0, w(0, init, c))) is below 2^31.
-__global__ void ising_init_bits(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena) {
+// Initial state: position i of row `row` in plane c is Up iff word (i & 3) of
+// Philox(key = seed, ctr = (i >> 2, row, 0, w(0, init, c))) is below 2^31
+// (Spin::rand draws Up when its uniform is below 1/2).
+__global__ void ising_init(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena) {
     const ChainDev& C = *chain;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t per_plane = (uint64_t)C.rows * C.pitch;
@@ -117,7 +79,7 @@ __global__ void ising_init_bits(const ChainDev* __restrict__ chain, uint8_t* __r
     arena[C.off[c] + e] = (uint8_t)v;
 }
 
-__global__ void ising_scatter_bits(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena,
+__global__ void ising_scatter(const ChainDev* __restrict__ chain, uint8_t* __restrict__ arena,
                                    const int8_t* __restrict__ natural) {
     const ChainDev& C = *chain;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -133,7 +95,7 @@ __global__ void ising_scatter_bits(const ChainDev* __restrict__ chain, uint8_t* 
     arena[C.off[c] + e] = (uint8_t)v;
 }
 
-__global__ void ising_gather_bits(const ChainDev* __restrict__ chain,
+__global__ void ising_gather(const ChainDev* __restrict__ chain,
                                   const uint8_t* __restrict__ arena, int8_t* __restrict__ natural,
                                   uint64_t n_sites) {
     const ChainDev& C = *chain;

@@ -187,10 +187,15 @@ struct vg_server {
 namespace vgi {
 namespace {
 
-uint64_t job_bytes(const Job& j) {
+// Pool bytes of one colour of a job.  An int8 Ising job is charged a byte per
+// site, as its spin kind says, though its planes hold one bit per site.
+uint64_t colour_bytes(const Job& j) {
     const int g = j.ch.group;
-    return j.dev.ncol * round_up(colour_elems(g, j.dev) * elem_bytes(g), 256);
+    const uint64_t n = j.ch.desc.spin == VG_SPIN_ISING ? byte_plane(j.dev)
+                                                       : colour_elems(g, j.dev) * elem_bytes(g);
+    return round_up(n, 256);
 }
+uint64_t job_bytes(const Job& j) { return j.dev.ncol * colour_bytes(j); }
 
 // Makes the working batch's groups the running jobs and sizes its buffers.
 int rebuild(vg_server* S) {
@@ -300,7 +305,7 @@ int quantum(vg_server* S, uint32_t& nsw_out) {
         Group& G = B.groups[j->ch.group];
         const ChainDev* dp = G.d_chains + j->ch.index;
         if (is_ising(j->ch.group)) {
-            launch_ising_init(j->ch.group, G, j->dev, dp, st);
+            launch_ising_init(G, j->dev, dp, st);
         } else {
             const uint64_t nc = 3ull * j->dev.ncol * j->dev.plane;
             const uint64_t ni = (uint64_t)j->dev.ncol * j->dev.rows * j->dev.w;
@@ -448,7 +453,7 @@ void worker_main(vg_server* S) {
             const int g = j.ch.group;
             const uint64_t e = elem_bytes(g);
             for (uint32_t c = 0; c < j.dev.ncol; ++c)
-                j.dev.off[c] = (off + c * round_up(colour_elems(g, j.dev) * e, 256)) / e;
+                j.dev.off[c] = (off + c * colour_bytes(j)) / e;
             j.state = VG_JOB_RUNNING;
             j.start_s = now_s(S->t0);
             j.fresh = true;

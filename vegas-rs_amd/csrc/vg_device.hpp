@@ -12,10 +12,14 @@
 //   position i holds
 //     sc     : the colour-c site at x = 2*i + ((c+y+z)&1)   (w = lx/2 positions)
 //     bcc/fcc: the sublattice-c site of cell x = i           (w = lx positions)
-//   Rows are `pitch` elements apart (pitch is a multiple of 64 bytes), so a
-//   row is read with aligned 16-byte loads.  Ising planes hold one byte per
-//   site (1 = Up, 0 = Down); Heisenberg chains hold three fp32 planes (x, y,
-//   z components) per colour.  Padding elements past w stay zero.
+//   Rows are `pitch` elements apart (bytes, Ising; floats, Heisenberg), a
+//   multiple of 16 bytes.  Ising planes hold one bit per site (set = Up; bit j
+//   of 32-bit word k of a row is position 32k + j), for both Ising spin
+//   kinds: an int8 chain differs from a bit-packed one only in what the
+//   caller hands over and is charged for.  (Kept as bytes beside bit shadows,
+//   the bytes were only ever written: 31 of the 37.6 MB a pass of sc 256^3 x
+//   3 moved.)  Heisenberg chains hold three fp32 planes (x, y, z components)
+//   per colour.  Padding elements past w stay zero.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -101,8 +105,8 @@ constexpr float kFixScale = 134217728.0f;  // 2^27
 
 // Ising acceptance classes per current bit: S = 0 .. 2z, z <= 12.
 constexpr uint32_t kThrS = 25;
-// Class plans of the multispin sc pass: absent-slot counts 0..5 of a site.
-constexpr uint32_t kPlanG = 6;
+// Class plans of the Ising passes: absent-slot and aligned counts 0..12.
+constexpr uint32_t kPlanG = 13;
 
 // ---------------------------------------------------------------------------
 // Chain descriptor as the kernels see it (one per chain of a kernel group).
@@ -123,32 +127,24 @@ struct ChainDev {
     uint32_t z;            // coordination number: 6 (sc), 8 (bcc) or 12 (fcc)
     uint32_t ncol;         // colours (planes): 2 (sc, bcc) or 4 (fcc)
     uint32_t limit;        // sweeps of the current block this chain runs (the rest skip it)
-    // n / d == (n * m) >> s for n < 2^31 (segs, ly and hy divisors)
+    // n / d == (n * m) >> s for n < 2^31 (segs and ly divisors)
     uint32_t segs_m, segs_s, ly_m, ly_s;
-    // Ising work order (bcc, fcc): rows of one y parity, then the other, a
-    // tile of z planes per lane (the sc pass takes the rows in natural order)
-    uint32_t hy;           // (ly + 1) / 2, rows of one parity class per plane
-    uint32_t hy_m, hy_s;
-    uint32_t nzc;          // z chunks of one tile of planes
-    // int8 sc chains of a batch: bit-packed shadows of the two colour planes
-    // (bit j of word k of a row = position 32k + j; rows of spitch bytes at
-    // byte offsets soff[c] of the arena), equal to the int8 planes after
-    // every kernel that writes those; the colour passes read the neighbour
-    // rows from the other colour's shadow.  shadow = 0: no shadows.
-    uint32_t spitch, shadow;
-    uint64_t soff[2];
+    uint32_t nzc;          // Ising lattice chains: z chunks of one tile of planes
+    // Ising lattice chains: the plan of g = 0 lists every aligned count above
+    // z / 2 with one threshold byte for both bits, and nothing else (a
+    // ferromagnet without a field)
+    uint32_t plain;
     // Ising acceptance: class (b, S) with b the current bit and S the sum over
     // neighbour slots of 2*b_j (present) or 1 (absent), S in [0, 2z].
     uint32_t thr[2][kThrS];  // accept iff draw < thr (32-bit draw)
     uint32_t always[2];    // bit S set: class always accepted
-    // The multispin sc decision's class plans, per absent-slot count g =
-    // 0..5 of a site (p = 6 - g present neighbours) and aligned count a =
-    // 0..p (present neighbours equal to the site's bit b): up to two slots
-    // for the classes (b, a) that are not always accepted, 0 for none.  Slot
-    // bits: 3 covers b = 0, 4 covers b = 1, 5 the threshold is nonzero (a
-    // draw whose high byte equals bits 8-15 is a tie), 8-15 the threshold's
-    // high byte.  One slot covers both bits when those fields agree.
-    uint32_t plan[kPlanG][7][2];
+    // The multispin decision's class plans, per absent-slot count g of a site
+    // (p = z - g present neighbours) and aligned count a = 0..p (present
+    // neighbours equal to the site's bit b): the classes (b, a) that are not
+    // always accepted, up to two 16-bit slots, 0 for none.  Slot bits: 0-7 the
+    // threshold's high byte, 8 covers b = 0, 9 covers b = 1.  One slot covers
+    // both bits when their bytes agree.
+    uint32_t plan[kPlanG][kPlanG];
     // Heisenberg parameters, fp32.
     float jn;              // -J
     float kk;              // K
@@ -174,11 +170,7 @@ struct ChainDev {
 };
 
 constexpr uint32_t kBlock = 256;       // threads per workgroup of a pass
-constexpr uint32_t kIsingSeg = 16;     // positions per Ising row segment (bcc, fcc)
-constexpr uint32_t kScSeg = 32;        // positions per sc Ising work item (one word of site bits)
-// sc pass modes: int8 planes; bit-packed planes; int8 planes whose
-// neighbour rows are read from bit-packed shadows.
-enum ScMode : uint32_t { kScInt8 = 0, kScBits = 1, kScShadow = 2 };
+constexpr uint32_t kIsingSeg = 32;     // positions per Ising work item (one word of site bits)
 constexpr uint32_t kHeisSeg = 4;       // positions per Heisenberg work item
 constexpr uint32_t kNumXcd = 8;        // MI355X: 8 XCDs, workgroups dealt round-robin
 // Wolff chains of at most this many sites keep their spins and visit marks
@@ -308,6 +300,24 @@ __device__ __forceinline__ int32_t wave_sum(int32_t v) {
            __builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48);
 }
 
+// The same total, left in lane 63 only: prefix sums within the rows of 16
+// (row_shr), then the rows' totals passed on (row_bcast): six instructions,
+// no scalar reads.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {  // 0 where nothing comes in
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
+}
+__device__ __forceinline__ int32_t wave_total(int32_t s) {
+    uint32_t v = (uint32_t)s;
+    v += dpp0<0x111, 0xF>(v);  // row_shr:1, 2, 4, 8
+    v += dpp0<0x112, 0xF>(v);
+    v += dpp0<0x114, 0xF>(v);
+    v += dpp0<0x118, 0xF>(v);
+    v += dpp0<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp0<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+    return (int32_t)v;
+}
+
 // Issue priority of the calling wave, 0 (lowest) .. 3; p must fold to a
 // constant.
 __device__ __forceinline__ void set_prio(uint32_t p) {
@@ -321,12 +331,13 @@ __device__ __forceinline__ void set_prio(uint32_t p) {
 
 // Maximum over the 64 lanes of a wave (every lane active).
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
-    v = max(v, dpp<kDppXor1>(v));
-    v = max(v, dpp<kDppXor2>(v));
-    v = max(v, dpp<kDppHalfMirror>(v));
-    v = max(v, dpp<kDppMirror>(v));
-    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+    v = max(v, dpp0<0x111, 0xF>(v));
+    v = max(v, dpp0<0x112, 0xF>(v));
+    v = max(v, dpp0<0x114, 0xF>(v));
+    v = max(v, dpp0<0x118, 0xF>(v));
+    v = max(v, dpp0<0x142, 0xA>(v));
+    v = max(v, dpp0<0x143, 0xC>(v));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // Ising colour planes are read and written through raw buffer resources:
@@ -338,6 +349,14 @@ constexpr uint32_t kNoRow = 0xFFFFFF00u;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const uint8_t* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0, bytes, 0x00020000);
+}
+
+// A value that is the same in every lane, in scalar registers.  (An address
+// the compiler computes in vector registers, uniform or not, makes every
+// buffer access through it a loop over the wave's distinct resources.)
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
 __device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
