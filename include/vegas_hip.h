@@ -249,13 +249,16 @@ int vg_batch_prepare(vg_batch* batch, uint64_t sweeps);
 /* Tile of the Ising sc, bcc and fcc passes (int8 and bit-packed): z
  * planes marched by one work item (1, 2, 4 or 8; by default chosen from the
  * amount of work in the batch), set for all three groups; get_tile reports
- * the first of them that has chains.  Results do not depend on it. */
+ * the first of them that has chains.  Results do not depend on it.  Small
+ * chains run whole sweep blocks in one workgroup each instead of passes,
+ * unless a tile is set. */
 int vg_batch_set_tile(vg_batch* batch, uint32_t tile);
 int vg_batch_get_tile(const vg_batch* batch, uint32_t* tile);
 /* Times `trial_sweeps` sweeps with every tile (replays of graphs captured
  * beforehand, five rounds over the tiles, the median of each) and keeps the
  * fastest, for each of the three groups.  The chains' spins and sweep counters are
- * restored after every trial, so tuning does not change any trajectory. */
+ * restored after every trial, so tuning does not change any trajectory.
+ * Groups of small chains that run without passes are left as they are. */
 int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen_tile);
 /* Records (0..128, default 128) the per-wave tie queue of the Ising sc, bcc
  * and fcc passes may hold before a wave settles further tied rows in the

@@ -54,6 +54,37 @@ def test_words_plans_and_tiles(vg, orc, ctx, kind, w, ly, lz, pbc):
                 step += 3
 
 
+@pytest.mark.parametrize("kind,w,ly,lz,pbc", [
+    ("sc", 8, 4, 2, (1, 1, 1)), ("sc", 13, 5, 1, (1, 0, 0)),       # 64 (one wave) and 65 sites a colour
+    ("sc", 32, 8, 4, (1, 1, 1)), ("bcc", 41, 5, 5, (0, 1, 0)),     # 1024 and 1025: 1 and 2 a lane
+    ("sc", 33, 8, 8, (1, 1, 1)), ("bcc", 16, 16, 8, (1, 1, 1)),    # 2112 and 2048: 4 and 2 a lane
+    ("sc", 64, 8, 8, (1, 1, 1)), ("bcc", 17, 15, 16, (0, 0, 1)),   # 4096 and 4080: the largest
+    ("fcc", 32, 8, 8, (1, 1, 0)), ("fcc", 1, 1, 1, (1, 1, 1)),     # 2048, the largest of fcc, and 1
+    ("fcc", 9, 5, 23, (1, 0, 1)),                                  # 1035
+])
+def test_resident_chains_equal_passes(vg, orc, ctx, kind, w, ly, lz, pbc):
+    """Sweep blocks in one workgroup against colour passes (a set tile) and the
+    oracle, batches of two fields and both proposals, over two blocks and the
+    seams of the batches of draws."""
+    chains = [_chain(vg, orc, kind, w, ly, lz, pbc, f, 81 + k, p, q)
+              for k, (f, p, q) in enumerate([(0.0, "int8", "flip"), (0.4, "bits", "random"),
+                                             (-0.2, "int8", "flip")])]
+    states = [orc.ising_init(c[2], 81 + k) for k, c in enumerate(chains)]
+    want = [orc.ising_sweeps(c[2], c[3], 81 + k, 0, 300, s)
+            for k, (c, s) in enumerate(zip(chains, states))]
+    for tile in (0, 1):
+        with vg.Batch(ctx, [c[1] for c in chains]) as b:
+            b.randomize()
+            for k, f in enumerate((0.0, 0.4, -0.2)):
+                b.set_thermostat(k, T[kind], f)
+            if tile:
+                b.set_tile(tile)
+            got = b.run_sums(300)
+            for k in range(3):
+                assert np.array_equal(got[k], want[k]), (tile, k)
+                assert np.array_equal(b.get_ising(k), states[k]), (tile, k)
+
+
 @pytest.mark.parametrize("kind,w,ly,lz,pbc,field", [
     ("bcc", 7, 5, 9, (1, 1, 1), 0.0),        # an odd number of rows
     ("fcc", 33, 5, 4, (0, 1, 0), 0.2),

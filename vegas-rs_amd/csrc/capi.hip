@@ -293,6 +293,15 @@ int upload_descriptors(vg_batch* B, int g, int slot) {
     return VG_OK;
 }
 
+// Compute units of the current device.
+int num_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        cus = 256;
+    return cus;
+}
+
 // The tile a new batch's Ising group starts with: the largest that leaves the
 // pass at least 7/4 waves per SIMD (1792 on 256 CUs).  Fewer leave SIMDs with
 // one wave or none, which issues an instruction every 8 cycles at best; more
@@ -304,10 +313,7 @@ int upload_descriptors(vg_batch* B, int g, int slot) {
 // (2430), three 9.6/8.0/7.5/9.0 (1822); fcc 161^3 2430: 6.0/6.3/6.9/10.4
 // (2430), two 8.1/7.7/8.4/10.5 (2430).  (Tile 4 whatever the size, before.)
 uint32_t default_tile(const ChainDev* chains, size_t n) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        cus = 256;
+    const int cus = num_cus();
     for (uint32_t tile : {8u, 4u, 2u}) {
         uint64_t items = 0;
         for (size_t k = 0; k < n; ++k)
@@ -352,6 +358,38 @@ bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid) {
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return false;
     return (uint64_t)grid <= (uint64_t)nb * (uint64_t)cus;
+}
+
+// Sites of a colour per lane of the resident kernel for an Ising lattice
+// group, or 0 for colour passes: always those when a chain does not fit, or
+// when the caller has set the tile or the tie queue of the passes.
+//
+// Otherwise the cheaper by the measured cost of a sweep, in ns.  Resident: one
+// workgroup a chain, 300 a colour + n / 1.75 for n sites, and a CU's chains one
+// after the other.  Passes: 3200 each in replays + 1 for 64 words of 32
+// positions, all chains together.  us a sweep, resident and passes, for 1, 256,
+// 512 and 1024 chains: sc 8^3 0.9/5.9, 1.3/7.9, 1.8/9.1, 3.2/10.6; sc 16^3
+// 2.4/7.0, 2.8/8.9, 5.4/10.6, 10.4/14.6; sc 20^3 4.9/7.3, 5.3/9.7, 10.2/13.6,
+// 20.3/19.4; sc 64 x 16 x 8 6.3/7.0, 6.7/9.0, 13.0/10.6, 25.9/12.3; bcc 16^3
+// 4.7/7.8, 5.1/9.8, 9.9/12.1, 19.5/16.9; fcc 12^3 4.0/15.9, 4.4/20.0, 8.6/23.4,
+// 16.9/29.0.
+uint32_t resident_sites(const Group& G, int g) {
+    if (G.tile_set || G.tie_cap != 128 || G.host.empty()) return 0;
+    const double ncol = colours_of(g);
+    double most = 0.0, sum = 0.0, words = 0.0;
+    for (const ChainDev& d : G.host) {
+        const double nc = (double)d.rows * d.w;
+        most = std::max(most, nc);
+        sum += nc;
+        words += (double)d.rows * d.segs * ncol;
+    }
+    if (most > (g == kIsingFcc ? vg::kResidentSites / 2 : vg::kResidentSites)) return 0;
+    const uint64_t cus = (uint64_t)num_cus();
+    const double chains = (double)G.host.size(), rounds = (double)((G.host.size() + cus - 1) / cus);
+    const auto cost = [&](double nc) { return 300.0 * ncol + ncol * nc / 1.75; };
+    const double mean = cost(sum / chains);
+    if ((rounds - 1.0) * mean + cost(most) > 3200.0 * ncol + words / 64.0) return 0;
+    return most <= vg::kResidentBlock ? 1u : (most <= 2 * vg::kResidentBlock ? 2u : 4u);
 }
 
 // Work decomposition of a group for a tile (Ising sc: z planes per work item):
@@ -401,6 +439,7 @@ int layout_work(vg_batch* B, int g, uint32_t tile) {
         for (const ChainDev& d : G.host)
             if ((d.pbc & 7u) != 7u) G.mode = 1;
         G.prio = all_resident(g, G, tile, G.grid) ? 1u : 0u;
+        G.resident = resident_sites(G, g);
     }
     G.partial_bytes_per_sweep = std::max<uint64_t>(
         256, (uint64_t)passes_of(G, g) * G.total_blocks * quantities(g) * quantity_bytes(g));
@@ -445,6 +484,22 @@ void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint3
                           g == kIsingSc ? sc : other, 0, st));
 }
 
+// A block of nsw sweeps of an Ising lattice group in the resident kernel.
+void launch_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_t* records) {
+    const uint32_t r = G.resident;
+    const auto fn = g == kIsingSc    ? (r == 1   ? vg::ising_resident<6, 1>
+                                        : r == 2 ? vg::ising_resident<6, 2>
+                                                 : vg::ising_resident<6, 4>)
+                    : g == kIsingBcc ? (r == 1   ? vg::ising_resident<8, 1>
+                                        : r == 2 ? vg::ising_resident<8, 2>
+                                                 : vg::ising_resident<8, 4>)
+                                     : (r == 1 ? vg::ising_resident<12, 1>
+                                               : vg::ising_resident<12, 2>);
+    hipLaunchKernelGGL(fn, dim3((uint32_t)G.members.size()), dim3(vg::kResidentBlock),
+                       vg::kResidentLds, st, G.d_chains, (uint8_t*)G.arena, nsw, vg::kResidentLds,
+                       records);
+}
+
 void launch_heis_fcc(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
     const auto fn = c == 0   ? vg::heis_fcc_pass<0>
                     : c == 1 ? vg::heis_fcc_pass<1>
@@ -485,12 +540,12 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
     const uint64_t nrec = (uint64_t)B->chains.size() * nsw * 5u;
     hipLaunchKernelGGL(vg::zero_i64, dim3((uint32_t)((nrec + 255) / 256)), dim3(256), 0, st,
                        B->d_records, nrec);
+    const bool timed = B->timing && !B->use_graph;  // an event pair per colour pass
     for (uint32_t s = 0; s < nsw; ++s) {
         for (int g = 0; g < kNumGroups; ++g) {
             Group& G = B->groups[g];
-            if (G.members.empty()) continue;
+            if (G.members.empty() || (G.resident && !timed)) continue;
             for (uint32_t c = 0; c < passes_of(G, g); ++c) {
-                const bool timed = B->timing && !B->use_graph;
                 if (timed) {
                     const uint32_t k = B->pass_events_used;
                     if (k + 2 > B->pass_events.size()) return fail(VG_ERR_DEVICE, "timing events exhausted");
@@ -533,6 +588,8 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
             launch_wolff<1>(G, st, nsw, B->d_records);
             launch_wolff<2>(G, st, nsw, B->d_records);
         }
+        else if (G.resident && !timed)
+            launch_resident(G, g, st, nsw, B->d_records);
         else if (is_ising(g) && !is_graph(g))
             hipLaunchKernelGGL(vg::ising_reduce, grid, dim3(vg::kBlock), 0, st, G.d_chains,
                                (const int32_t*)G.partials, G.total_blocks, colours_of(g), nsw,
@@ -1366,6 +1423,7 @@ int vg_batch_set_tile(vg_batch* batch, uint32_t tile) {
     VG_HIP(hipSetDevice(batch->ctx->device));
     for (int g : kZmarchGroups) {
         if (batch->groups[g].members.empty()) continue;
+        batch->groups[g].tile_set = true;
         int rc = layout_work(batch, g, tile);
         if (rc) return rc;
     }
@@ -1436,7 +1494,8 @@ int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen) 
     if (e != hipSuccess) rc = fail(VG_ERR_DEVICE, "autotune backup: %s", hipGetErrorString(e));
     for (int g : kZmarchGroups) {
         Group& G = batch->groups[g];
-        if (G.members.empty() || rc != VG_OK) continue;
+        // (the tile means nothing to the resident kernel)
+        if (G.members.empty() || G.resident || rc != VG_OK) continue;
         const uint32_t start_tile = G.tile;
         uint32_t best = start_tile;
         const uint32_t tiles[4] = {1, 2, 4, 8};
@@ -1489,7 +1548,11 @@ int vg_batch_set_tie_capacity(vg_batch* batch, uint32_t records) {
     if (!batch) return fail(VG_ERR_INVALID_ARGUMENT, "null batch");
     if (records > 128)
         return fail(VG_ERR_INVALID_ARGUMENT, "tie capacity must be 0..128 (got %u)", records);
-    for (Group& G : batch->groups) G.tie_cap = records;
+    for (int g : kZmarchGroups) {
+        Group& G = batch->groups[g];
+        G.tie_cap = records;
+        if (!G.members.empty()) G.resident = resident_sites(G, g);
+    }
     // captured graphs hold the old kernel arguments
     for (auto& kv : batch->graphs) quiet(hipGraphExecDestroy(kv.second));
     batch->graphs.clear();

@@ -47,6 +47,10 @@ __global__ void ising_fcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32
 template <uint32_t A>
 __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t);
+// Sweep blocks of small chains, one workgroup a chain.  Z: coordination
+// number; R: sites of a colour per lane.
+template <uint32_t Z, uint32_t R>
+__global__ void ising_resident(const ChainDev*, uint8_t*, uint32_t, uint32_t, int64_t*);
 // Wolff steps of the chains of one lattice kind (0 sc, 1 bcc, 2 fcc).
 template <uint32_t KIND>
 __global__ void wolff_run(const ChainDev*, uint8_t*, uint32_t, int64_t*);
@@ -160,6 +164,11 @@ struct Group {
     uint32_t prio = 0;  // z-marching Ising passes: every workgroup resident at once (wave priorities on)
     // z-marching Ising passes: tie records a wave may queue (at most 128)
     uint32_t tie_cap = 128;
+    // Ising sc/bcc/fcc: the caller has set the tile
+    bool tile_set = false;
+    // Ising sc/bcc/fcc: sites of a colour per lane of the resident kernel that
+    // runs the group's sweep blocks, 0 when colour passes do
+    uint32_t resident = 0;
     uint32_t npass = 0;     // graph groups: passes per sweep (the most colours of a member)
     void* arena = nullptr;
     uint64_t arena_bytes = 0;

@@ -1,0 +1,272 @@
+// Whole sweep blocks of small Ising chains, one workgroup a chain, spins in
+// LDS.
+//
+// The same sweeps as the colour passes (MetropolisFlipIntegrator::step /
+// MetropolisIntegrator::step, reference src/integrator.rs:66-138, with the
+// Exchange + Zeeman local energy of src/energy.rs:147-151, 194-206), the same
+// draws and the same sums.  A pass of a small chain lasts about 3 us whatever
+// its size: the launch, a cold descriptor, and a few waves that issue one
+// instruction every 8 cycles through a pass's start-up.  Here a chain's sweeps
+// are a loop of one workgroup, with nothing to launch and nothing to read back
+// between them:
+//   - the draws depend on the site and the sweep only, not on the spins, so
+//     the workgroup makes those of as many sweeps as its LDS holds at once,
+//     all its lanes busy whatever the chain's size, each site's 32 bits whole
+//     (no ties to settle);
+//   - a colour update is then one lane a site: the class sum S from the
+//     neighbours' bytes, at addresses worked out once (two 16-bit ones a
+//     register), a threshold from a table, the new byte.  About 30
+//     instructions and two LDS round trips, and a barrier (a wave's own LDS
+//     order where a colour fits one wave).
+// A spin is a byte 0 (Down) or 2 (Up) and an absent neighbour a byte 1, so S is
+// the plain sum of the neighbours' bytes and S - Z the sum of the present
+// neighbours' spins.
+//
+// us a sweep of one chain, by passes and here: sc 10 x 10 x 2 5.8, 0.8; 8^3
+// 6.0, 0.9; 16^3 7.0, 2.4; 20^3 7.3, 4.9; bcc 8^3 7.0, 1.0; 16^3 7.8, 4.7;
+// fcc 8^3 14.9, 2.0; 12^3 16.1, 4.0.  At 8^3 the two LDS round trips and the
+// barrier of each colour are most of it; from about 12^3 the instructions, of
+// the draws two thirds.
+#include "fcc_common.hpp"
+
+namespace vg {
+
+namespace {
+
+// LDS of a chain, in bytes: its spins with the absent neighbour's byte, the
+// threshold table, then per sweep its sums, draws and proposals.
+__host__ __device__ constexpr uint32_t resident_spins(uint32_t n) { return (n + 16u) & ~15u; }
+
+// Colour, row and position of the d-th neighbour (fcc: lower colours first).
+// Returns its byte's address, `absent` where it lies past an open end.
+template <uint32_t Z>
+__device__ __forceinline__ uint32_t neighbour_at(const ChainDev& C, uint32_t c, uint32_t y,
+                                                 uint32_t z, uint32_t i, uint32_t d, uint32_t nc,
+                                                 uint32_t absent) {
+    const bool px = C.pbc & 1u, py = C.pbc & 2u, pz = C.pbc & 4u;
+    bool okx = true, oky = true, okz = true;
+    uint32_t b = c ^ 1u;
+    if constexpr (Z == 6) {
+        if (d == 1u) i = fcc_move(i, ((c + y + z) & 1u) ? 1 : -1, C.w, px, okx);
+        if (d == 2u || d == 3u) y = fcc_move(y, d == 2u ? -1 : 1, C.ly, py, oky);
+        if (d >= 4u) z = fcc_move(z, d == 4u ? -1 : 1, C.lz, pz, okz);
+    } else if constexpr (Z == 8) {
+        const int st = c ? 1 : -1;
+        if (d & 1u) i = fcc_move(i, st, C.w, px, okx);
+        if (d & 2u) y = fcc_move(y, st, C.ly, py, oky);
+        if (d & 4u) z = fcc_move(z, st, C.lz, pz, okz);
+    } else {
+        b = d >> 2;
+        if (b >= c) ++b;
+        const uint32_t axes = fcc_diff(c, b);
+        // d's two bits along the two axes of the pair
+        const bool first = d & 1u, second = d & 2u;
+        const bool mx = (axes & 1u) && first;
+        const bool my = (axes & 2u) && ((axes & 1u) ? second : first);
+        const bool mz = (axes & 4u) && second;
+        if (mx) i = fcc_move(i, fcc_step(c, b, 0), C.w, px, okx);
+        if (my) y = fcc_move(y, fcc_step(c, b, 1), C.ly, py, oky);
+        if (mz) z = fcc_move(z, fcc_step(c, b, 2), C.lz, pz, okz);
+    }
+    return okx && oky && okz ? b * nc + (y + C.ly * z) * C.w + i : absent;
+}
+
+}  // namespace
+
+// R: sites of a colour per lane.  With one, sc and bcc keep within the
+// registers of two workgroups a CU (512 chains of sc 8^3: 2.31 us a sweep, now
+// 1.76); fcc spills there (8^3 2.0 us a sweep, 2.2).  lds_bytes: the launch's dynamic LDS.
+template <uint32_t Z, uint32_t R>
+__global__ __launch_bounds__(kResidentBlock, Z < 12 && R == 1 ? 8 : 4) void ising_resident(
+    const ChainDev* __restrict__ chains, uint8_t* __restrict__ arena, uint32_t nsw,
+    uint32_t lds_bytes, int64_t* __restrict__ records) {
+    constexpr uint32_t NCOL = Z == 12 ? 4 : 2;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const ChainDev& C = chains[blockIdx.x];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t run = min(nsw, C.limit);
+    if (!run) return;
+    const uint32_t w = C.w, segs = C.segs, nc = C.rows * w, n = NCOL * nc;
+    const uint32_t words = C.rows * segs;  // of a colour
+    const bool rnd = C.proposal != 0;
+    const uint32_t k0 = (uint32_t)C.seed, k1 = (uint32_t)(C.seed >> 32);
+    uint8_t* const spin = lds;
+    uint2* const table = reinterpret_cast<uint2*>(lds + resident_spins(n));
+    int32_t* const sums = reinterpret_cast<int32_t*>(table + 2u * kThrS);
+    // sweeps whose draws are held at once
+    const uint32_t per_sweep = 8u + n * (rnd ? 5u : 4u);
+    const uint32_t room = lds_bytes - resident_spins(n) - 2u * kThrS * 8u;
+    const uint32_t batch = min(run, room / per_sweep);
+    uint32_t* const draw = reinterpret_cast<uint32_t*>(sums + 2u * batch);
+    uint8_t* const prop = reinterpret_cast<uint8_t*>(draw + n * batch);
+
+    // Spins, the absent neighbour, the table {threshold, always accepted}.
+    for (uint32_t k = tid; k < NCOL * words; k += kResidentBlock) {
+        const uint32_t c = k / words, at = k - c * words;
+        const uint32_t row = fast_div(at, C.segs_m, C.segs_s), i0 = (at - row * segs) * kIsingSeg;
+        uint32_t v = *reinterpret_cast<const uint32_t*>(arena + C.off[c] +
+                                                        (uint64_t)row * C.pitch + (i0 >> 3));
+        uint8_t* const out = spin + c * nc + row * w + i0;
+        const uint32_t m = min(kIsingSeg, w - i0);
+        for (uint32_t j = 0; j < m; ++j) out[j] = (uint8_t)(((v >> j) & 1u) << 1);
+    }
+    if (tid == 0) spin[n] = 1;
+    for (uint32_t k = tid; k < 2u * kThrS; k += kResidentBlock) {
+        const uint32_t b = k / kThrS, S = k - b * kThrS;
+        table[k] = make_uint2(C.thr[b][S], (C.always[b] >> S) & 1u);
+    }
+
+    // The lane's sites and their neighbours' addresses.
+    uint32_t nbr[NCOL][R][Z / 2];
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t site = min(tid + r * kResidentBlock, nc - 1u);
+        const uint32_t row = site / w, i = site - row * w;
+        const uint32_t z = fast_div(row, C.ly_m, C.ly_s), y = row - z * C.ly;
+#pragma unroll
+        for (uint32_t c = 0; c < NCOL; ++c)
+#pragma unroll
+            for (uint32_t d = 0; d < Z / 2; ++d)
+                nbr[c][r][d] = neighbour_at<Z>(C, c, y, z, i, 2u * d, nc, n) |
+                               neighbour_at<Z>(C, c, y, z, i, 2u * d + 1u, nc, n) << 16;
+    }
+
+    const uint32_t dw = kResidentBlock % words, dh = kResidentBlock / words;
+    for (uint32_t done = 0; done < run; done += batch) {
+        const uint32_t ns = min(batch, run - done);
+        const uint64_t t0 = C.sweep0 + done;
+        // The draws of ns sweeps, a lane a word of positions.
+        uint32_t half = tid / words, at = tid - half * words;
+        while (half < ns * NCOL) {
+            const uint32_t s = half / NCOL, c = half % NCOL;
+            const uint64_t t = t0 + s;
+            const uint32_t row = fast_div(at, C.segs_m, C.segs_s);
+            const uint32_t i0 = (at - row * segs) * kIsingSeg, m = min(kIsingSeg, w - i0);
+            const uint32_t wA = ctr_w(t, kIsingA, c), wB = ctr_w(t, kIsingB, c);
+            const U4 r0 = philox(U4{i0 >> 4, row, (uint32_t)t, wA}, k0, k1);
+            const U4 r1 = Z == 6 || m > 16u
+                              ? philox(U4{(i0 >> 4) + 1u, row, (uint32_t)t, wA}, k0, k1)
+                              : r0;
+            uint32_t* const dr = draw + half * nc + row * w + i0;
+#pragma unroll
+            for (uint32_t j0 = 0; j0 < kIsingSeg; j0 += 4u) {
+                if (j0 >= m) break;
+                const U4 rb = philox(U4{(i0 + j0) >> 2, row, (uint32_t)t, wB}, k0, k1);
+                // the high bytes of sites j0 .. j0+3, a byte each
+                uint32_t hi = 0;
+                if constexpr (Z == 6) {
+                    // bit j of the calls' word k is bit k of site j's byte
+                    const uint32_t p[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+                    for (uint32_t k = 0; k < 8; ++k) {
+                        const uint32_t nib = (p[k] >> j0) & 15u;
+                        hi |= ((nib * 0x00204081u) & 0x01010101u) << k;
+                    }
+                } else {
+                    hi = u4_word(j0 < 16u ? r0 : r1, (j0 & 15u) >> 2);
+                }
+                const uint32_t q[4] = {rb.x, rb.y, rb.z, rb.w};
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e)
+                    if (j0 + e < m) dr[j0 + e] = (((hi >> (8u * e)) & 255u) << 24) | (q[e] >> 8);
+            }
+            if (rnd) {
+                const U4 rp = philox(U4{i0 >> 7, row, (uint32_t)t, ctr_w(t, kIsingProposal, c)}, k0,
+                                     k1);
+                const uint32_t v = u4_word(rp, (i0 >> 5) & 3u);
+                uint8_t* const pr = prop + half * nc + row * w + i0;
+                for (uint32_t j = 0; j < m; ++j) pr[j] = (uint8_t)((~(v >> j) & 1u) << 1);
+            }
+            half += dh;
+            at += dw;
+            if (at >= words) {
+                at -= words;
+                ++half;
+            }
+        }
+        for (uint32_t k = tid; k < 2u * ns; k += kResidentBlock) sums[k] = 0;
+        __syncthreads();
+
+        const bool solo = nc <= 64u;  // one wave updates: its LDS operations are in order
+        if (!solo || tid < 64u) {
+            for (uint32_t s = 0; s < ns; ++s) {
+                int32_t acc = 0;  // bond sum << 16 + magnetisation (both small)
+#pragma unroll
+                for (uint32_t c = 0; c < NCOL; ++c) {
+                    const uint32_t base = (s * NCOL + c) * nc;
+#pragma unroll
+                    for (uint32_t r = 0; r < R; ++r) {
+                        const uint32_t site = tid + r * kResidentBlock;
+                        if (site >= nc) break;
+                        const uint32_t d = draw[base + site];
+                        const uint32_t own = spin[c * nc + site];
+                        uint32_t S = 0, low = 0;
+#pragma unroll
+                        for (uint32_t k = 0; k < Z / 2; ++k) {
+                            S += spin[nbr[c][r][k] & 0xFFFFu];
+                            S += spin[nbr[c][r][k] >> 16];
+                            if (Z == 12 && 2u * k + 2u == 4u * c) low = S;
+                        }
+                        const uint2 e = table[(own >> 1) * kThrS + S];
+                        bool ok = (d < e.x) | (e.y != 0u);
+                        if (rnd) ok = ok & (prop[base + site] != own);
+                        const uint32_t now = ok ? own ^ 2u : own;
+                        spin[c * nc + site] = (uint8_t)now;
+                        const int32_t v = (int32_t)now - 1;
+                        acc += v;
+                        // the bonds to lower colours
+                        if (Z == 12 ? c > 0 : c == 1)
+                            acc += (v * ((int32_t)(Z == 12 ? low : S) -
+                                         (int32_t)(Z == 12 ? 4u * c : Z))) *
+                                   65536;
+                    }
+                    if (solo) {
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    } else {
+                        __syncthreads();
+                    }
+                }
+                acc = wave_total(acc);
+                if ((tid & 63u) == 63u && tid - 63u < nc) {
+                    const int32_t m = (int16_t)acc;
+                    atomicAdd(&sums[2u * s], m);
+                    atomicAdd(&sums[2u * s + 1u], (acc - m) >> 16);
+                }
+            }
+        }
+        __syncthreads();
+        for (uint32_t s = tid; s < ns; s += kResidentBlock) {
+            int64_t* const rec = records + ((uint64_t)C.slot * nsw + done + s) * 5u;
+            rec[0] = sums[2u * s + 1u];
+            rec[3] = sums[2u * s];
+        }
+        __syncthreads();
+    }
+
+    for (uint32_t k = tid; k < NCOL * words; k += kResidentBlock) {
+        const uint32_t c = k / words, at = k - c * words;
+        const uint32_t row = fast_div(at, C.segs_m, C.segs_s), i0 = (at - row * segs) * kIsingSeg;
+        const uint8_t* const in = spin + c * nc + row * w + i0;
+        const uint32_t m = min(kIsingSeg, w - i0);
+        uint32_t v = 0;
+        for (uint32_t j = 0; j < m; ++j) v |= ((uint32_t)in[j] >> 1) << j;
+        *reinterpret_cast<uint32_t*>(arena + C.off[c] + (uint64_t)row * C.pitch + (i0 >> 3)) = v;
+    }
+}
+
+#define VG_RESIDENT(Z, R)                                                                       \
+    template __global__ void ising_resident<Z, R>(const ChainDev*, uint8_t*, uint32_t, uint32_t, \
+                                                  int64_t*);
+VG_RESIDENT(6, 1)
+VG_RESIDENT(6, 2)
+VG_RESIDENT(6, 4)
+VG_RESIDENT(8, 1)
+VG_RESIDENT(8, 2)
+VG_RESIDENT(8, 4)
+VG_RESIDENT(12, 1)
+VG_RESIDENT(12, 2)
+#undef VG_RESIDENT
+
+}  // namespace vg

@@ -178,6 +178,12 @@ constexpr uint32_t kNumXcd = 8;        // MI355X: 8 XCDs, workgroups dealt round
 // first kWolffLdsQueue entries of the cluster queue (31 KiB).
 constexpr uint32_t kWolffLdsSites = 1u << 19;
 constexpr uint32_t kWolffLdsQueue = 7936;
+// Resident Ising chains (ising_resident): threads and dynamic LDS of a
+// workgroup, sites of a colour at most (sc and bcc; fcc half).
+constexpr uint32_t kResidentBlock = 1024;
+constexpr uint32_t kResidentLds = 65536;
+constexpr uint32_t kResidentSites = 4096;
+
 constexpr uint32_t kWolffBlock = 1024;  // threads per workgroup of the Wolff kernels
 constexpr uint32_t kWolffLdsWordsMax = 2u * (kWolffLdsSites / 32u) + kWolffLdsQueue;
 
