@@ -392,6 +392,66 @@ uint32_t resident_sites(const Group& G, int g) {
     return most <= vg::kResidentBlock ? 1u : (most <= 2 * vg::kResidentBlock ? 2u : 4u);
 }
 
+bool is_heis_lattice(int g) { return g == kHeisSc || g == kHeisBcc || g == kHeisFcc; }
+
+// The same for a Heisenberg lattice group, with its workspace for the draws of
+// at most max_sweeps sweeps and 64 MiB.
+//
+// The cheaper by the measured cost of a sweep, in ns.  Resident: a workgroup's
+// 750 a colour + n / 1.43 for n sites, a CU's chains one after the other; the
+// draws of all chains, 10 for 1000 sites (flip proposals 8.5); two launches for
+// the sweeps that the workspace holds.  Passes, for P sites with rows padded to
+// items of four: 5000 a colour + 8.4 for 1000 of P (fcc 12), at least 6500 a
+// colour; flip proposals 3800, 6.5 (9), 4600.  us a sweep, resident and passes,
+// random proposals, 1, 128, 256 and 512 chains: sc 8^3 2.2/11.6, 2.9/13.7,
+// 3.7/14.7, 5.3/18.8; sc 16^3 4.3/13.0, 9.2/15.6, 14.8/21.2, 34.9/34.9; sc 20^3
+// 7.0/13.1, 18.2/22.3, 31.2/33.4, 80.8/55.9; bcc 16^3 7.4/13.8, 18.4/19.2,
+// 30.6/27.9, 78.4/45.9; fcc 12^3 9.0/27.0, 19.2/30.7, 30.4/41.3, 77.0/73.6.
+// Flip proposals, 1, 128 and 256: sc 16^3 4.3/9.3, 8.3/11.8, 13.0/16.7; bcc
+// 16^3 7.5/10.0, 17.1/14.9, 28.0/22.0; fcc 12^3 9.0/19.0, 17.8/22.7, 27.5/32.4.
+int setup_heis_resident(Group& G, int g, uint32_t max_sweeps) {
+    const double ncol = colours_of(g);
+    uint64_t n = 0, sites = 0, padded = 0;
+    bool random = false;
+    for (const ChainDev& d : G.host) {
+        const uint64_t nk = (uint64_t)d.rows * d.w * d.ncol;
+        n = std::max(n, nk);
+        sites += nk;
+        padded += (uint64_t)d.rows * d.segs * vg::kHeisSeg * d.ncol;
+        random = random || d.proposal;
+    }
+    const uint64_t nc = n / colours_of(g);
+    if (nc > (g == kHeisFcc ? vg::kResidentSites / 2 : vg::kResidentSites)) return VG_OK;
+    const uint64_t chains = G.host.size(), cus = (uint64_t)num_cus();
+    const uint64_t per_sweep = n * chains * sizeof(float4);
+    if (per_sweep > (64ull << 20) || chains > 65535u) return VG_OK;
+    const uint32_t held = (uint32_t)std::min<uint64_t>(max_sweeps, (64ull << 20) / per_sweep);
+    const double one = 750.0 * ncol, mean = (double)sites / (double)chains;
+    const double resident = (double)((chains + cus - 1) / cus - 1) * (one + mean / 1.43) + one +
+                            (double)n / 1.43 + (double)sites * (random ? 10e-3 : 8.5e-3) +
+                            4000.0 / held;
+    const double slope = g == kHeisFcc ? (random ? 12e-3 : 9e-3) : (random ? 8.4e-3 : 6.5e-3);
+    const double passes = std::max((random ? 6500.0 : 4600.0) * ncol,
+                                   (random ? 5000.0 : 3800.0) * ncol + slope * (double)padded);
+    if (resident > passes) return VG_OK;
+    const void* fns[] = {(const void*)&vg::heis_resident<6, 1>, (const void*)&vg::heis_resident<6, 2>,
+                         (const void*)&vg::heis_resident<6, 4>, (const void*)&vg::heis_resident<8, 1>,
+                         (const void*)&vg::heis_resident<8, 2>, (const void*)&vg::heis_resident<8, 4>,
+                         (const void*)&vg::heis_resident<12, 1>,
+                         (const void*)&vg::heis_resident<12, 2>};
+    for (const void* fn : fns)  // past the 64 KiB default
+        VG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
+    if (hipMalloc(&G.draws, per_sweep * held) != hipSuccess) {
+        G.draws = nullptr;  // no room for the workspace: passes
+        quiet(hipGetLastError());
+        return VG_OK;
+    }
+    G.draw_sweeps = held;
+    G.draw_stride = (uint32_t)n;
+    G.resident = nc <= vg::kResidentBlock ? 1u : (nc <= 2 * vg::kResidentBlock ? 2u : 4u);
+    return VG_OK;
+}
+
 // Work decomposition of a group for a tile (Ising sc: z planes per work item):
 // items and blocks per chain, the block -> chain map, the grid.  Replays of
 // captured graphs bake the grid in, so they are dropped.
@@ -459,6 +519,7 @@ int free_batch(vg_batch* B) {
         if (G.d_block_chain) quiet(hipFree(G.d_block_chain));
         if (G.arena && !G.shared_arena) quiet(hipFree(G.arena));
         if (G.partials) quiet(hipFree(G.partials));
+        if (G.draws) quiet(hipFree(G.draws));
     }
     if (B->d_records) quiet(hipFree(B->d_records));
     if (B->h_records) quiet(hipHostFree(B->h_records));
@@ -498,6 +559,31 @@ void launch_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_
     hipLaunchKernelGGL(fn, dim3((uint32_t)G.members.size()), dim3(vg::kResidentBlock),
                        vg::kResidentLds, st, G.d_chains, (uint8_t*)G.arena, nsw, vg::kResidentLds,
                        records);
+}
+
+// The same of a Heisenberg lattice group: draws, then the sweeps on them, as
+// many at a time as the workspace holds.
+void launch_heis_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_t* records) {
+    const uint32_t r = G.resident, z = g == kHeisSc ? 6u : (g == kHeisBcc ? 8u : 12u);
+    const auto fn = g == kHeisSc    ? (r == 1   ? vg::heis_resident<6, 1>
+                                       : r == 2 ? vg::heis_resident<6, 2>
+                                                : vg::heis_resident<6, 4>)
+                    : g == kHeisBcc ? (r == 1   ? vg::heis_resident<8, 1>
+                                       : r == 2 ? vg::heis_resident<8, 2>
+                                                : vg::heis_resident<8, 4>)
+                                    : (r == 1 ? vg::heis_resident<12, 1>
+                                              : vg::heis_resident<12, 2>);
+    const uint32_t ncol = z == 12 ? 4u : 2u, nc = G.draw_stride / ncol;
+    const uint32_t block = std::min<uint32_t>((nc + 63u) / 64u * 64u, vg::kResidentBlock);
+    const uint32_t chains = (uint32_t)G.members.size();
+    for (uint32_t s0 = 0; s0 < nsw; s0 += G.draw_sweeps) {
+        const uint32_t ns = std::min(G.draw_sweeps, nsw - s0);
+        hipLaunchKernelGGL(vg::heis_draws, dim3((nc + 255u) / 256u, ns * ncol, chains), dim3(256),
+                           0, st, G.d_chains, s0, ns, G.draw_stride, G.draws);
+        hipLaunchKernelGGL(fn, dim3(chains), dim3(block), 16u * (G.draw_stride + 1u) + 40u * ns, st,
+                           G.d_chains, (float*)G.arena, s0, ns, G.draw_stride, G.draws, nsw,
+                           records);
+    }
 }
 
 void launch_heis_fcc(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
@@ -588,6 +674,8 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
             launch_wolff<1>(G, st, nsw, B->d_records);
             launch_wolff<2>(G, st, nsw, B->d_records);
         }
+        else if (G.resident && !timed && is_heis_lattice(g))
+            launch_heis_resident(G, g, st, nsw, B->d_records);
         else if (G.resident && !timed)
             launch_resident(G, g, st, nsw, B->d_records);
         else if (is_ising(g) && !is_graph(g))
@@ -1047,6 +1135,13 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
         if (e != hipSuccess) {
             free_batch(B);
             return fail(VG_ERR_OUT_OF_MEMORY, "allocating partial sums: %s", hipGetErrorString(e));
+        }
+        if (is_heis_lattice(g)) {
+            int rc = setup_heis_resident(G, g, B->max_block_sweeps);
+            if (rc) {
+                free_batch(B);
+                return rc;
+            }
         }
         if (is_zmarch(g)) {
             int rc = layout_work(B, g, default_tile(G.host.data(), G.host.size()));

@@ -51,6 +51,11 @@ __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*
 // number; R: sites of a colour per lane.
 template <uint32_t Z, uint32_t R>
 __global__ void ising_resident(const ChainDev*, uint8_t*, uint32_t, uint32_t, int64_t*);
+// Heisenberg: the draws of sweeps s0 .. of a block, and the sweeps on them.
+__global__ void heis_draws(const ChainDev*, uint32_t, uint32_t, uint32_t, float4*);
+template <uint32_t Z, uint32_t R>
+__global__ void heis_resident(const ChainDev*, float*, uint32_t, uint32_t, uint32_t,
+                              const float4*, uint32_t, int64_t*);
 // Wolff steps of the chains of one lattice kind (0 sc, 1 bcc, 2 fcc).
 template <uint32_t KIND>
 __global__ void wolff_run(const ChainDev*, uint8_t*, uint32_t, int64_t*);
@@ -166,7 +171,7 @@ struct Group {
     uint32_t tie_cap = 128;
     // Ising sc/bcc/fcc: the caller has set the tile
     bool tile_set = false;
-    // Ising sc/bcc/fcc: sites of a colour per lane of the resident kernel that
+    // Lattice groups: sites of a colour per lane of the resident kernel that
     // runs the group's sweep blocks, 0 when colour passes do
     uint32_t resident = 0;
     uint32_t npass = 0;     // graph groups: passes per sweep (the most colours of a member)
@@ -174,6 +179,10 @@ struct Group {
     uint64_t arena_bytes = 0;
     void* partials = nullptr;  // [sweep][colour][block][quantity]
     uint64_t partial_bytes_per_sweep = 0;
+    // Resident Heisenberg chains: workspace for the draws of draw_sweeps
+    // sweeps, draw_stride of them a sweep and chain (the largest chain's sites)
+    float4* draws = nullptr;
+    uint32_t draw_sweeps = 0, draw_stride = 0;
     // Capacities of d_chains / h_staging (descriptors) and of partials
     // (bytes), for batches whose membership changes (the job server).
     uint32_t chains_cap = 0;

@@ -27,7 +27,7 @@
 // fcc 8^3 14.9, 2.0; 12^3 16.1, 4.0.  At 8^3 the two LDS round trips and the
 // barrier of each colour are most of it; from about 12^3 the instructions, of
 // the draws two thirds.
-#include "fcc_common.hpp"
+#include "resident.hpp"
 
 namespace vg {
 
@@ -36,40 +36,6 @@ namespace {
 // LDS of a chain, in bytes: its spins with the absent neighbour's byte, the
 // threshold table, then per sweep its sums, draws and proposals.
 __host__ __device__ constexpr uint32_t resident_spins(uint32_t n) { return (n + 16u) & ~15u; }
-
-// Colour, row and position of the d-th neighbour (fcc: lower colours first).
-// Returns its byte's address, `absent` where it lies past an open end.
-template <uint32_t Z>
-__device__ __forceinline__ uint32_t neighbour_at(const ChainDev& C, uint32_t c, uint32_t y,
-                                                 uint32_t z, uint32_t i, uint32_t d, uint32_t nc,
-                                                 uint32_t absent) {
-    const bool px = C.pbc & 1u, py = C.pbc & 2u, pz = C.pbc & 4u;
-    bool okx = true, oky = true, okz = true;
-    uint32_t b = c ^ 1u;
-    if constexpr (Z == 6) {
-        if (d == 1u) i = fcc_move(i, ((c + y + z) & 1u) ? 1 : -1, C.w, px, okx);
-        if (d == 2u || d == 3u) y = fcc_move(y, d == 2u ? -1 : 1, C.ly, py, oky);
-        if (d >= 4u) z = fcc_move(z, d == 4u ? -1 : 1, C.lz, pz, okz);
-    } else if constexpr (Z == 8) {
-        const int st = c ? 1 : -1;
-        if (d & 1u) i = fcc_move(i, st, C.w, px, okx);
-        if (d & 2u) y = fcc_move(y, st, C.ly, py, oky);
-        if (d & 4u) z = fcc_move(z, st, C.lz, pz, okz);
-    } else {
-        b = d >> 2;
-        if (b >= c) ++b;
-        const uint32_t axes = fcc_diff(c, b);
-        // d's two bits along the two axes of the pair
-        const bool first = d & 1u, second = d & 2u;
-        const bool mx = (axes & 1u) && first;
-        const bool my = (axes & 2u) && ((axes & 1u) ? second : first);
-        const bool mz = (axes & 4u) && second;
-        if (mx) i = fcc_move(i, fcc_step(c, b, 0), C.w, px, okx);
-        if (my) y = fcc_move(y, fcc_step(c, b, 1), C.ly, py, oky);
-        if (mz) z = fcc_move(z, fcc_step(c, b, 2), C.lz, pz, okz);
-    }
-    return okx && oky && okz ? b * nc + (y + C.ly * z) * C.w + i : absent;
-}
 
 }  // namespace
 
