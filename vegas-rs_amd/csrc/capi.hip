@@ -650,12 +650,14 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
                                        c, s, G.total_blocks, G.grid);
                 else if (g == kIsingGraph)
                     hipLaunchKernelGGL(vg::graph_ising_pass, dim3(G.total_blocks), block, 0, st,
-                                       G.d_chains, G.d_block_chain, (uint8_t*)G.arena,
-                                       (int64_t*)G.partials, c, s, G.total_blocks, G.npass);
+                                       G.d_chains, G.members.size() > 1 ? G.d_block_chain : nullptr,
+                                       (uint8_t*)G.arena, (int64_t*)G.partials, c, s,
+                                       G.total_blocks, G.npass);
                 else if (g == kHeisGraph)
                     hipLaunchKernelGGL(vg::graph_heis_pass, dim3(G.total_blocks), block, 0, st,
-                                       G.d_chains, G.d_block_chain, (uint8_t*)G.arena,
-                                       (int64_t*)G.partials, c, s, G.total_blocks, G.npass);
+                                       G.d_chains, G.members.size() > 1 ? G.d_block_chain : nullptr,
+                                       (uint8_t*)G.arena, (int64_t*)G.partials, c, s,
+                                       G.total_blocks, G.npass);
                 else
                     launch_heis_fcc(G, st, c, s);
                 if (timed) {
@@ -1061,6 +1063,12 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
                 for (int part = 0; part < 4; ++part) d.off[part] = offs[part];
                 for (int part = 0; part < 3; ++part) d.goff[part] = offs[4 + part];
                 d.ncol = gr.ncol;
+                const uint64_t per = n ? gr.ptr[1] - gr.ptr[0] : 0;
+                d.w = (uint32_t)per;
+                for (uint64_t r = 1; r < n; ++r)
+                    if (gr.ptr[r + 1] - gr.ptr[r] != per) d.w = 0;
+                for (size_t c = 0; c < std::min<size_t>(gr.cstart.size(), vg::kGraphStarts); ++c)
+                    (&d.plan[0][0])[c] = gr.cstart[c];
                 d.items = gr.max_class;
                 G.npass = std::max(G.npass, gr.ncol);
                 continue;

@@ -27,6 +27,68 @@
 
 namespace vg {
 
+// Row entries gathered at once: their neighbours, couplings and then spins are
+// in flight together, so a row of up to eight entries waits for memory twice
+// and not twice an entry.  (Past the row's end the last entry is read again and
+// not added.)  A pass of 64 workgroups is one wave a SIMD and as long as its
+// chain of waits: MEASURED
+constexpr uint32_t kGather = 8;
+
+// What a pass's wave needs of its chain, loaded in one batch before anything
+// is decided: field by field where each is used, the scalar loads were a chain
+// of six waits at the start of a pass that lasts a few thousand cycles.  The
+// class starts come with it from the descriptor; the arena's table serves
+// colours past those that fit there.
+struct GraphHead {
+    uint64_t off[4], goff[2], seed, t, nsites;
+    uint32_t p;  // the lane's position
+    uint32_t proposal, w;
+    bool go;     // a site of this class, in a sweep that the chain runs
+};
+
+__device__ __forceinline__ uint64_t loaded(uint64_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ uint32_t loaded(uint32_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+__device__ __forceinline__ GraphHead graph_head(const ChainDev& C, const uint8_t* arena,
+                                                uint32_t colour, uint32_t s, uint32_t b) {
+    const uint32_t* const held = &C.plan[0][0];
+    const uint32_t at = min(colour, kGraphStarts - 2u);
+    uint32_t first = held[at], end = held[at + 1u], limit = C.limit, ncol = C.ncol;
+    uint32_t block0 = C.block0;
+    uint64_t starts = C.goff[2];
+    GraphHead h{{C.off[0], C.off[1], C.off[2], C.off[3]}, {C.goff[0], C.goff[1]},
+                C.seed,  C.sweep0 + s, C.nsites, 0u, C.proposal, C.w, false};
+    first = loaded(first);
+    end = loaded(end);
+    limit = loaded(limit);
+    ncol = loaded(ncol);
+    block0 = loaded(block0);
+    starts = loaded(starts);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) h.off[k] = loaded(h.off[k]);
+    h.goff[0] = loaded(h.goff[0]);
+    h.goff[1] = loaded(h.goff[1]);
+    h.seed = loaded(h.seed);
+    h.t = loaded(h.t);
+    h.nsites = loaded(h.nsites);
+    h.proposal = loaded(h.proposal);
+    h.w = loaded(h.w);
+    if (colour > kGraphStarts - 2u && colour < ncol) {
+        const uint32_t* const cst = reinterpret_cast<const uint32_t*>(arena + starts);
+        first = cst[colour];
+        end = cst[colour + 1u];
+    }
+    h.p = first + (b - block0) * kBlock + threadIdx.x;
+    h.go = s < limit && colour < ncol && h.p < end;
+    return h;
+}
+
 __global__ __launch_bounds__(256) void graph_ising_pass(const ChainDev* __restrict__ chains,
                                                         const uint32_t* __restrict__ block_chain,
                                                         uint8_t* __restrict__ arena,
@@ -34,52 +96,78 @@ __global__ __launch_bounds__(256) void graph_ising_pass(const ChainDev* __restri
                                                         uint32_t colour, uint32_t s,
                                                         uint32_t total_blocks, uint32_t npass) {
     const uint32_t b = blockIdx.x;
-    const ChainDev& C = chains[block_chain[b]];
-    if (s >= C.limit) return;  // uniform: the workgroup belongs to one chain
-    int64_t acc[5] = {0, 0, 0, 0, 0};
-    if (colour < C.ncol) {
-        const uint32_t* cst = reinterpret_cast<const uint32_t*>(arena + C.goff[2]);
-        const uint32_t p = cst[colour] + (b - C.block0) * kBlock + threadIdx.x;
-        if (p < cst[colour + 1]) {
-            uint8_t* spin = arena + C.off[0];
-            const uint32_t* ptr = reinterpret_cast<const uint32_t*>(arena + C.off[1]);
-            const uint32_t* nbr = reinterpret_cast<const uint32_t*>(arena + C.off[2]);
-            const double* a = reinterpret_cast<const double*>(arena + C.off[3]);
-            const double* w = reinterpret_cast<const double*>(arena + C.goff[0]);
-            const uint32_t site = reinterpret_cast<const uint32_t*>(arena + C.goff[1])[p];
-            const uint64_t t = C.sweep0 + s;
-            const U4 r = philox(U4{site, 0u, (uint32_t)t, ctr_w(t, kGraphIsing, 0)},
-                                (uint32_t)C.seed, (uint32_t)(C.seed >> 32));
-            double sv = spin[p] ? 1.0 : -1.0;
-            // Spin::rand proposes Up when its draw is below 1/2 (state.rs:76-84);
-            // a proposal equal to the current spin changes nothing.
-            const bool change = C.proposal == 0 || ((r.y < 0x80000000u) ? 1.0 : -1.0) != sv;
-            double h = 0.0, hb = 0.0;
-            const uint32_t e1 = ptr[p + 1];
-            for (uint32_t e = ptr[p]; e < e1; ++e) {
-                const double sj = spin[nbr[e]] ? 1.0 : -1.0;
-                h = __dadd_rn(h, __dmul_rn(a[e], sj));
-                hb = __dadd_rn(hb, __dmul_rn(w[e], sj));
-            }
-            // The decision is computed without branches and applied by one
-            // select: written as `if (dE <= 0 || u < p) flip`, the accept
-            // block has two predecessors, and hipcc for gfx950 (ROCm 7.2)
-            // kept the old spin on the second path (the optimised IR is
-            // right).  exp is evaluated for every site; its argument is
-            // clamped to <= 0, which changes nothing where it is used
-            // (dE > 0).
-            const double dE = __dsub_rn(__dmul_rn(__dmul_rn(2.0, sv), h),
-                                        __dmul_rn(__dmul_rn(__dmul_rn(2.0, C.ghm), C.ghz), sv));
-            const double pr = exp_f64_nonpos(fmin(-__dmul_rn(dE, C.gbeta), 0.0));
-            const bool accept =
-                change & ((dE <= 0.0) | (__dmul_rn((double)r.x, 0x1p-32) < pr));
-            if (accept) spin[p] = sv > 0.0 ? 0 : 1;
-            sv = accept ? -sv : sv;
-            acc[3] = sv > 0.0 ? 1 : -1;
-            acc[0] = __double2ll_rn(__dmul_rn(__dmul_rn(sv, hb), 134217728.0));
+    const ChainDev& C = chains[block_chain ? block_chain[b] : 0u];
+    const GraphHead H = graph_head(C, arena, colour, s, b);
+    const double ghm = __longlong_as_double((long long)loaded((uint64_t)__double_as_longlong(C.ghm)));
+    const double ghz = __longlong_as_double((long long)loaded((uint64_t)__double_as_longlong(C.ghz)));
+    const double gbeta = __longlong_as_double((long long)loaded((uint64_t)__double_as_longlong(C.gbeta)));
+    bool up = false, site_here = false;
+    int64_t bsum = 0;
+    const uint32_t p = H.p;
+    const uint64_t t = H.t;
+    if (H.go) {
+        uint8_t* spin = arena + H.off[0];
+        const uint32_t* ptr = reinterpret_cast<const uint32_t*>(arena + H.off[1]);
+        const uint32_t* nbr = reinterpret_cast<const uint32_t*>(arena + H.off[2]);
+        const double* a = reinterpret_cast<const double*>(arena + H.off[3]);
+        const double* w = reinterpret_cast<const double*>(arena + H.goff[0]);
+        const uint32_t site = reinterpret_cast<const uint32_t*>(arena + H.goff[1])[p];
+        const U4 r = philox(U4{site, 0u, (uint32_t)t, ctr_w(t, kGraphIsing, 0)},
+                            (uint32_t)H.seed, (uint32_t)(H.seed >> 32));
+        double sv = spin[p] ? 1.0 : -1.0;
+        // Spin::rand proposes Up when its draw is below 1/2 (state.rs:76-84);
+        // a proposal equal to the current spin changes nothing.
+        const bool change = H.proposal == 0 || ((r.y < 0x80000000u) ? 1.0 : -1.0) != sv;
+        double h = 0.0, hb = 0.0;
+        uint32_t e0 = p * H.w, e1 = e0 + H.w;  // H.w = 0: rows of different lengths
+        if (!H.w) {
+            e0 = ptr[p];
+            e1 = ptr[p + 1];
         }
+        for (; e0 < e1; e0 += kGather) {
+            uint32_t j[kGather], bj[kGather];
+            double aj[kGather], wj[kGather];
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) {
+                const uint32_t e = min(e0 + k, e1 - 1u);
+                j[k] = nbr[e];
+                aj[k] = a[e];
+                wj[k] = w[e];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) bj[k] = spin[j[k]];
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) {
+                const double sj = bj[k] ? 1.0 : -1.0;
+                const double hk = __dadd_rn(h, __dmul_rn(aj[k], sj));
+                const double hbk = __dadd_rn(hb, __dmul_rn(wj[k], sj));
+                h = e0 + k < e1 ? hk : h;
+                hb = e0 + k < e1 ? hbk : hb;
+            }
+        }
+        // The decision is computed without branches and applied by one
+        // select: written as `if (dE <= 0 || u < p) flip`, the accept
+        // block has two predecessors, and hipcc for gfx950 (ROCm 7.2)
+        // kept the old spin on the second path (the optimised IR is
+        // right).  exp is evaluated for every site; its argument is
+        // clamped to <= 0, which changes nothing where it is used
+        // (dE > 0).
+        const double dE = __dsub_rn(__dmul_rn(__dmul_rn(2.0, sv), h),
+                                    __dmul_rn(__dmul_rn(__dmul_rn(2.0, ghm), ghz), sv));
+        const double pr = exp_f64_nonpos(fmin(-__dmul_rn(dE, gbeta), 0.0));
+        const bool accept =
+            change & ((dE <= 0.0) | (__dmul_rn((double)r.x, 0x1p-32) < pr));
+        if (accept) spin[p] = sv > 0.0 ? 0 : 1;
+        sv = accept ? -sv : sv;
+        up = sv > 0.0;
+        site_here = true;
+        bsum = __double2ll_rn(__dmul_rn(__dmul_rn(sv, hb), 134217728.0));
     }
-    heis_partials(acc, partials, colour, npass, s, total_blocks, b);
+    // {bond, 0, 0, magnetisation, 0}
+    const int64_t mag = 2 * (int64_t)__builtin_popcountll(__ballot(up)) -
+                        (int64_t)__builtin_popcountll(__ballot(site_here));
+    const int64_t sums[5] = {wave_sum_any(bsum), 0, 0, mag, 0};
+    heis_block_partials(sums, partials, colour, npass, s, total_blocks, b);
 }
 
 __global__ __launch_bounds__(256) void graph_heis_pass(const ChainDev* __restrict__ chains,
@@ -89,61 +177,75 @@ __global__ __launch_bounds__(256) void graph_heis_pass(const ChainDev* __restric
                                                        uint32_t colour, uint32_t s,
                                                        uint32_t total_blocks, uint32_t npass) {
     const uint32_t b = blockIdx.x;
-    const ChainDev& C = chains[block_chain[b]];
-    if (s >= C.limit) return;
-    int64_t acc[5] = {0, 0, 0, 0, 0};
-    if (colour < C.ncol) {
-        const uint32_t* cst = reinterpret_cast<const uint32_t*>(arena + C.goff[2]);
-        const uint32_t p = cst[colour] + (b - C.block0) * kBlock + threadIdx.x;
-        if (p < cst[colour + 1]) {
-            float* xs = reinterpret_cast<float*>(arena + C.off[0]);
-            float* ys = xs + C.nsites;
-            float* zs = ys + C.nsites;
-            const uint32_t* ptr = reinterpret_cast<const uint32_t*>(arena + C.off[1]);
-            const uint32_t* nbr = reinterpret_cast<const uint32_t*>(arena + C.off[2]);
-            const float* a = reinterpret_cast<const float*>(arena + C.off[3]);
-            const float* w = reinterpret_cast<const float*>(arena + C.goff[0]);
-            const uint32_t site = reinterpret_cast<const uint32_t*>(arena + C.goff[1])[p];
-            const uint64_t t = C.sweep0 + s;
-            float h[3] = {0.0f, 0.0f, 0.0f}, hb[3] = {0.0f, 0.0f, 0.0f};
-            const uint32_t e1 = ptr[p + 1];
-            for (uint32_t e = ptr[p]; e < e1; ++e) {
-                const uint32_t j = nbr[e];
-                const float aj = a[e], wj = w[e];
-                const float sx = xs[j], sy = ys[j], sz = zs[j];
-                h[0] = fa(h[0], fm(aj, sx));
-                h[1] = fa(h[1], fm(aj, sy));
-                h[2] = fa(h[2], fm(aj, sz));
-                hb[0] = fa(hb[0], fm(wj, sx));
-                hb[1] = fa(hb[1], fm(wj, sy));
-                hb[2] = fa(hb[2], fm(wj, sz));
-            }
-            const float o[3] = {xs[p], ys[p], zs[p]};
-            float u, pr[3];
-            if (C.proposal) {
-                if (!proposal_first(C, site, 0u, t, 0u, u, pr)) proposal_rest(C, site, 0u, t, 0u, pr);
-            } else {
-                const U4 fw = philox(U4{site, 0u, (uint32_t)t, ctr_w(t, kHeisStream, 0)},
-                                     (uint32_t)C.seed, (uint32_t)(C.seed >> 32));
-                u = unit24(fw.x);
-                pr[0] = -o[0];
-                pr[1] = -o[1];
-                pr[2] = -o[2];
-            }
-            float n[3];
-            int32_t s32[4] = {0, 0, 0, 0};
-            int64_t bsum = 0;
-            heis_update(C, false, o, h, hb, u, pr, n, s32, bsum);
-            heis_fold(s32, bsum, acc);
-            // the bond share can exceed the int32 fixed-point range of the
-            // lattice sums when couplings are large: 64-bit conversion
-            acc[0] = (int64_t)__float2ll_rn(fm(dot3(n[0], n[1], n[2], hb[0], hb[1], hb[2]), kFixScale));
-            xs[p] = n[0];
-            ys[p] = n[1];
-            zs[p] = n[2];
+    const ChainDev& C = chains[block_chain ? block_chain[b] : 0u];
+    const GraphHead H = graph_head(C, arena, colour, s, b);
+    int32_t s32[4] = {0, 0, 0, 0};
+    int64_t bsum = 0;
+    const uint32_t p = H.p;
+    const uint64_t t = H.t;
+    if (H.go) {
+        float* xs = reinterpret_cast<float*>(arena + H.off[0]);
+        float* ys = xs + H.nsites;
+        float* zs = ys + H.nsites;
+        const uint32_t* ptr = reinterpret_cast<const uint32_t*>(arena + H.off[1]);
+        const uint32_t* nbr = reinterpret_cast<const uint32_t*>(arena + H.off[2]);
+        const float* a = reinterpret_cast<const float*>(arena + H.off[3]);
+        const float* w = reinterpret_cast<const float*>(arena + H.goff[0]);
+        const uint32_t site = reinterpret_cast<const uint32_t*>(arena + H.goff[1])[p];
+        float h[3] = {0.0f, 0.0f, 0.0f}, hb[3] = {0.0f, 0.0f, 0.0f};
+        uint32_t e0 = p * H.w, e1 = e0 + H.w;  // H.w = 0: rows of different lengths
+        if (!H.w) {
+            e0 = ptr[p];
+            e1 = ptr[p + 1];
         }
+        for (; e0 < e1; e0 += kGather) {
+            uint32_t j[kGather];
+            float aj[kGather], wj[kGather], sj[kGather][3];
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) {
+                const uint32_t e = min(e0 + k, e1 - 1u);
+                j[k] = nbr[e];
+                aj[k] = a[e];
+                wj[k] = w[e];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) {
+                sj[k][0] = xs[j[k]];
+                sj[k][1] = ys[j[k]];
+                sj[k][2] = zs[j[k]];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kGather; ++k) {
+                if (e0 + k >= e1) break;
+#pragma unroll
+                for (uint32_t c = 0; c < 3; ++c) {
+                    h[c] = fa(h[c], fm(aj[k], sj[k][c]));
+                    hb[c] = fa(hb[c], fm(wj[k], sj[k][c]));
+                }
+            }
+        }
+        const float o[3] = {xs[p], ys[p], zs[p]};
+        float u, pr[3];
+        if (H.proposal) {
+            if (!proposal_first(C, site, 0u, t, 0u, u, pr)) proposal_rest(C, site, 0u, t, 0u, pr);
+        } else {
+            const U4 fw = philox(U4{site, 0u, (uint32_t)t, ctr_w(t, kHeisStream, 0)},
+                                 (uint32_t)H.seed, (uint32_t)(H.seed >> 32));
+            u = unit24(fw.x);
+            pr[0] = -o[0];
+            pr[1] = -o[1];
+            pr[2] = -o[2];
+        }
+        float n[3];
+        heis_update(C, false, o, h, hb, u, pr, n, s32, bsum);
+        // the bond share can exceed the int32 fixed-point range of the
+        // lattice sums when couplings are large: 64-bit conversion
+        bsum = (int64_t)__float2ll_rn(fm(dot3(n[0], n[1], n[2], hb[0], hb[1], hb[2]), kFixScale));
+        xs[p] = n[0];
+        ys[p] = n[1];
+        zs[p] = n[2];
     }
-    heis_partials(acc, partials, colour, npass, s, total_blocks, b);
+    heis_partials(s32, bsum, partials, colour, npass, s, total_blocks, b);
 }
 
 // Initial states (State::rand_with_size, src/state.rs:260-262) keyed by the

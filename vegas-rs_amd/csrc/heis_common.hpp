@@ -284,19 +284,6 @@ __device__ __forceinline__ void heis_block_partials(const int64_t w[5],
     }
 }
 
-// Workgroup sums of the five quantities of any magnitude (the graph passes,
-// whose couplings enter the bond share): 64-bit shuffle reduction.
-__device__ __forceinline__ void heis_partials(int64_t acc[5], int64_t* __restrict__ partials,
-                                              uint32_t colour, uint32_t ncol, uint32_t s,
-                                              uint32_t total_blocks, uint32_t b) {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) acc[k] += __shfl_xor(acc[k], o, 64);
-    }
-    heis_block_partials(acc, partials, colour, ncol, s, total_blocks, b);
-}
-
 // Sum over the wave (every lane active) of a value below 2^40 in magnitude
 // in every lane: its low 16 bits and the rest (below 2^24) are summed in
 // int32 -- below 2^22 and 2^30 over 64 lanes, so exactly.
@@ -304,6 +291,32 @@ __device__ __forceinline__ int64_t wave_sum_split(int64_t v) {
     const int32_t lo = (int32_t)(v & 0xFFFF);
     const int32_t hi = (int32_t)(v >> 16);
     return (int64_t)wave_sum(hi) * 65536 + (int64_t)wave_sum(lo);
+}
+
+// Sum over the wave (every lane active) of int64 values of any magnitude,
+// modulo 2^64 as any order of additions: the low and middle 20 bits and the
+// rest are summed in int32 (26 bits, 26 bits, and a sum whose low 24 bits are
+// all that reaches the result).
+__device__ __forceinline__ int64_t wave_sum_any(int64_t v) {
+    const int32_t lo = (int32_t)(v & 0xFFFFF), mid = (int32_t)((v >> 20) & 0xFFFFF);
+    const int32_t hi = (int32_t)(v >> 40);
+    return (int64_t)((uint64_t)(uint32_t)wave_sum(hi) << 40) +
+           (int64_t)((uint64_t)(uint32_t)wave_sum(mid) << 20) + (int64_t)wave_sum(lo);
+}
+
+// Workgroup sums of the graph passes, whose couplings enter the bond share: a
+// value of any magnitude, and four below 2^27 a lane.  By DPP: the 64-bit
+// shuffles they replace, thirty in a row of two LDS permutes each, took more
+// of a small pass than its site did.
+__device__ __forceinline__ void heis_partials(const int32_t s32[4], int64_t bsum,
+                                              int64_t* __restrict__ partials, uint32_t colour,
+                                              uint32_t ncol, uint32_t s, uint32_t total_blocks,
+                                              uint32_t b) {
+    int64_t w[5];
+    w[0] = wave_sum_any(bsum);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[1 + k] = wave_sum_split(s32[k]);
+    heis_block_partials(w, partials, colour, ncol, s, total_blocks, b);
 }
 
 // Workgroup sums of the lattice passes (sc, bcc, fcc): a lane holds at most

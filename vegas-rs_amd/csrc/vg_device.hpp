@@ -107,6 +107,7 @@ constexpr float kFixScale = 134217728.0f;  // 2^27
 constexpr uint32_t kThrS = 25;
 // Class plans of the Ising passes: absent-slot and aligned counts 0..12.
 constexpr uint32_t kPlanG = 13;
+constexpr uint32_t kGraphStarts = kPlanG * kPlanG;
 
 // ---------------------------------------------------------------------------
 // Chain descriptor as the kernels see it (one per chain of a kernel group).
@@ -163,7 +164,8 @@ struct ChainDev {
     // merged-row offsets (u32, nsites + 1), off[2] neighbour positions
     // (u32), off[3] couplings a (f64 Ising, f32 Heisenberg), goff[0]
     // lower-colour couplings w, goff[1] site id of each position (u32),
-    // goff[2] colour class starts (u32, ncol + 1).  Ising parameters in f64:
+    // goff[2] colour class starts (u32, ncol + 1), the first kGraphStarts of
+    // which also stand in plan; w entries in every row, 0 when they differ.  Ising parameters in f64:
     // 1/T, |h| (0 without Zeeman) and the field's sign.
     uint64_t goff[3];
     double gbeta, ghm, ghz;
