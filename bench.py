@@ -74,8 +74,9 @@ def source_digest(kernel):
 def pass_counters(workload, kernels):
     """Counter-measured bytes per dispatch (FETCH_SIZE + WRITE_SIZE, scaled by
     a device copy of known size) and VALU instructions per dispatch of the
-    named pass kernels -- the mean over them -- from the table the rocprofv3
-    runs of this workload wrote (profiles/pass_counters.txt).  None when the
+    named pass kernels (Heisenberg ones without their item size) -- the mean
+    over them -- from the table the rocprofv3 runs of this workload wrote
+    (profiles/pass_counters.txt).  None when the
     table has no row for one of them (another tile, say) or when a kernel's
     sources differ from those the table was measured with (its "# sources"
     line holds their digests)."""

@@ -417,7 +417,7 @@ int setup_heis_resident(Group& G, int g, uint32_t max_sweeps) {
         const uint64_t nk = (uint64_t)d.rows * d.w * d.ncol;
         n = std::max(n, nk);
         sites += nk;
-        padded += (uint64_t)d.rows * d.segs * vg::kHeisSeg * d.ncol;
+        padded += (uint64_t)d.rows * ((d.w + 3u) / 4u * 4u) * d.ncol;
         random = random || d.proposal;
     }
     const uint64_t nc = n / colours_of(g);
@@ -452,12 +452,39 @@ int setup_heis_resident(Group& G, int g, uint32_t max_sweeps) {
     return VG_OK;
 }
 
+// Positions per work item of a Heisenberg lattice group: one while the waves
+// that leaves are few, else four.  A wave of items of four issues 1000
+// instructions (sc), of single ones 380: on a chip that holds all waves at
+// once the second pass is shorter, and past that the first does less work a
+// site (start-up and sums; 16-byte loads).  The line is 8 waves of single
+// items a SIMD on sc, 14 on bcc and 48 on fcc, whose items of four need the
+// registers of three waves a SIMD.  us a pass with items of four and one,
+// random proposals (waves a SIMD): sc 32^3 6.8, 4.6 (0.25); 64^3 7.0, 5.1 (2);
+// 96^3 8.5, 8.0 (6.8); 104^3 10.7, 10.0 (8.6); 128^3 12.5, 14.0 (16); bcc 40^3
+// 7.2, 4.9 (1); 80^3 9.2, 8.5 (7.8); 66^3 x 3, flip proposals, 10.5, 10.2 (13);
+// 80^3 x 2 13.4, 13.8 (16); fcc 40^3 7.2, 4.6 (1); 70^3 x 3 19.1, 15.8 (16);
+// 96^3 x 3 33.4, 29.9 (41); 128^3 x 3 79.7, 86.8 (96).  (Items of two lay
+// between the two or behind both.)
+uint32_t heis_item(const Group& G, int g) {
+    uint64_t waves = 0;
+    for (const ChainDev& d : G.host) waves += (uint64_t)d.rows * d.w / 64;
+    const uint64_t line = g == kHeisSc ? 8 : (g == kHeisBcc ? 14 : 48);
+    return waves <= line * 4u * (uint64_t)num_cus() ? 1 : 4;
+}
+
 // Work decomposition of a group for a tile (Ising sc: z planes per work item):
 // items and blocks per chain, the block -> chain map, the grid.  Replays of
 // captured graphs bake the grid in, so they are dropped.
 int layout_work(vg_batch* B, int g, uint32_t tile) {
     Group& G = B->groups[g];
     std::vector<uint32_t> block_chain;
+    if (is_heis_lattice(g)) {
+        G.item = heis_item(G, g);
+        for (ChainDev& d : G.host) {
+            d.segs = (d.w + G.item - 1) / G.item;
+            magic_div(d.segs, d.segs_m, d.segs_s);
+        }
+    }
     for (size_t k = 0; k < G.members.size(); ++k) {
         ChainDev& d = G.host[k];
         uint64_t items;
@@ -586,13 +613,22 @@ void launch_heis_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, i
     }
 }
 
-void launch_heis_fcc(const Group& G, hipStream_t st, uint32_t c, uint32_t s) {
-    const auto fn = c == 0   ? vg::heis_fcc_pass<0>
-                    : c == 1 ? vg::heis_fcc_pass<1>
-                    : c == 2 ? vg::heis_fcc_pass<2>
-                             : vg::heis_fcc_pass<3>;
-    hipLaunchKernelGGL(fn, dim3(G.grid), dim3(vg::kBlock), 0, st, G.d_chains, G.d_block_chain,
-                       (float*)G.arena, (int64_t*)G.partials, s, G.total_blocks, G.grid);
+// One colour pass of a Heisenberg lattice group.
+template <uint32_t S>
+void launch_heis_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s) {
+    const dim3 grid(G.grid), block(vg::kBlock);
+    if (g != kHeisFcc) {
+        hipLaunchKernelGGL(g == kHeisSc ? vg::heis_sc_pass<S> : vg::heis_bcc_pass<S>, grid, block, 0,
+                           st, G.d_chains, G.d_block_chain, (float*)G.arena, (int64_t*)G.partials,
+                           c, s, G.total_blocks, G.grid);
+        return;
+    }
+    const auto fn = c == 0   ? vg::heis_fcc_pass<0, S>
+                    : c == 1 ? vg::heis_fcc_pass<1, S>
+                    : c == 2 ? vg::heis_fcc_pass<2, S>
+                             : vg::heis_fcc_pass<3, S>;
+    hipLaunchKernelGGL(fn, grid, block, 0, st, G.d_chains, G.d_block_chain, (float*)G.arena,
+                       (int64_t*)G.partials, s, G.total_blocks, G.grid);
 }
 
 // The Wolff steps of the group's chains of one lattice kind: chains of at
@@ -637,17 +673,9 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
                     if (k + 2 > B->pass_events.size()) return fail(VG_ERR_DEVICE, "timing events exhausted");
                     VG_HIP(hipEventRecord(B->pass_events[k], st));
                 }
-                const dim3 grid(G.grid), block(vg::kBlock);
+                const dim3 block(vg::kBlock);
                 if (is_zmarch(g))
                     launch_zmarch_pass(G, g, st, c, s);
-                else if (g == kHeisSc)
-                    hipLaunchKernelGGL(vg::heis_sc_pass, grid, block, 0, st, G.d_chains,
-                                       G.d_block_chain, (float*)G.arena, (int64_t*)G.partials,
-                                       c, s, G.total_blocks, G.grid);
-                else if (g == kHeisBcc)
-                    hipLaunchKernelGGL(vg::heis_bcc_pass, grid, block, 0, st, G.d_chains,
-                                       G.d_block_chain, (float*)G.arena, (int64_t*)G.partials,
-                                       c, s, G.total_blocks, G.grid);
                 else if (g == kIsingGraph)
                     hipLaunchKernelGGL(vg::graph_ising_pass, dim3(G.total_blocks), block, 0, st,
                                        G.d_chains, G.members.size() > 1 ? G.d_block_chain : nullptr,
@@ -658,8 +686,10 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
                                        G.d_chains, G.members.size() > 1 ? G.d_block_chain : nullptr,
                                        (uint8_t*)G.arena, (int64_t*)G.partials, c, s,
                                        G.total_blocks, G.npass);
+                else if (G.item == 4)
+                    launch_heis_pass<4>(G, g, st, c, s);
                 else
-                    launch_heis_fcc(G, st, c, s);
+                    launch_heis_pass<1>(G, g, st, c, s);
                 if (timed) {
                     VG_HIP(hipEventRecord(B->pass_events[B->pass_events_used + 1], st));
                     B->pass_events_used += 2;

@@ -28,6 +28,7 @@ __global__ void ising_reduce(const ChainDev*, const int32_t*, uint32_t, uint32_t
 __global__ void ising_init(const ChainDev*, uint8_t*);
 __global__ void ising_scatter(const ChainDev*, uint8_t*, const int8_t*);
 __global__ void ising_gather(const ChainDev*, const uint8_t*, int8_t*, uint64_t);
+template <uint32_t S>
 __global__ void heis_sc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                              uint32_t, uint32_t, uint32_t);
 // bcc and fcc passes: one instantiation per colour A (sublattice), args as
@@ -35,6 +36,7 @@ __global__ void heis_sc_pass(const ChainDev*, const uint32_t*, float*, int64_t*,
 template <uint32_t A, uint32_t K, uint32_t MODE>
 __global__ void ising_bcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32_t*, uint32_t,
                                uint32_t, uint32_t, uint32_t, uint32_t);
+template <uint32_t S>
 __global__ void heis_bcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t, uint32_t);
 __global__ void heis_reduce(const ChainDev*, const int64_t*, uint32_t, uint32_t, uint32_t,
@@ -44,7 +46,7 @@ __global__ void ising_fcc_pass(const ChainDev*, const uint32_t*, uint8_t*, int32
                                uint32_t, uint32_t, uint32_t, uint32_t);
 // One instantiation per colour A, args (chains, block -> chain map, arena,
 // partials, sweep, total blocks, grid).
-template <uint32_t A>
+template <uint32_t A, uint32_t S>
 __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t);
 // Sweep blocks of small chains, one workgroup a chain.  Z: coordination
@@ -174,6 +176,8 @@ struct Group {
     // Lattice groups: sites of a colour per lane of the resident kernel that
     // runs the group's sweep blocks, 0 when colour passes do
     uint32_t resident = 0;
+    // Heisenberg lattice groups: positions per work item (template parameter)
+    uint32_t item = 4;
     uint32_t npass = 0;     // graph groups: passes per sweep (the most colours of a member)
     void* arena = nullptr;
     uint64_t arena_bytes = 0;

@@ -8,14 +8,16 @@
 // summed over the eight slots in the order dz, dy, dx (dx fastest) with an
 // absent slot (open boundary) adding +0.0f.
 //
-// Work item: 4 consecutive positions of one row; each of the four neighbour
-// rows is read with one aligned 16-byte load per component, plus the one
-// position beyond the item (x-1 or x+4).  Same three phases as the sc pass
-// (fields and first proposal calls, the wave's queue, updates).
+// Work item: S = 1 or 4 consecutive positions of one row; each of the four
+// neighbour rows is read at the item's positions (with four, one aligned 16-byte
+// load per component) and at the one position beyond it (x-1 or x+S).  Same
+// three phases as the sc pass (fields and first proposal calls, the wave's
+// queue, updates).
 #include "heis_common.hpp"
 
 namespace vg {
 
+template <uint32_t S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void heis_bcc_pass(const ChainDev* __restrict__ chains,
                                                      const uint32_t* __restrict__ block_chain,
                                                      float* __restrict__ arena,
@@ -60,11 +62,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
     const uint32_t z = fast_div(row, C.ly_m, C.ly_s);
     const uint32_t y = row - z * ly;
     const bool px = pbc & 1u, py = pbc & 2u, pz = pbc & 4u;
-    const uint32_t i0 = seg * kHeisSeg;
-    const uint32_t nvalid = active ? min(kHeisSeg, w - i0) : 0u;
+    const uint32_t i0 = seg * S;
+    const uint32_t nvalid = active ? min(S, w - i0) : 0u;
     const uint32_t own_off = active ? (row * pitch + i0) * 4u : kNoRow;
     uint32_t pend = 0;
-    float os[4][3], hs[4][3], ps[4][3], us[4];
+    float os[S][3], hs[S][3], ps[S][3], us[S];
     {
         bool yok, zok;
         uint32_t y2, z2;
@@ -89,22 +91,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
             xe_pos = i0 > 0 ? i0 - 1 : w - 1;
             xe_ok = i0 > 0 || px;
         } else {
-            xe_pos = i0 + kHeisSeg < w ? i0 + kHeisSeg : 0;
-            xe_ok = i0 + kHeisSeg < w || px;
+            xe_pos = i0 + S < w ? i0 + S : 0;
+            xe_ok = i0 + S < w || px;
         }
 
-        float4 so[3], v[4][3];
+        Run<S> so[3], v[4][3];
         // colour 1: the last segment's extra position is 0, the +x slot of
         // position w-1 across the periodic end (0 when x is open)
         float xe[4][3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) so[c] = bload4f(rown[c], own_off);
+        for (int c = 0; c < 3; ++c) so[c] = bload<S>(rown[c], own_off);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t ro = rows[r] * pitch * 4u;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                v[r][c] = bload4f(roth[c], rok[r] ? ro + i0 * 4u : kNoRow);
+                v[r][c] = bload<S>(roth[c], rok[r] ? ro + i0 * 4u : kNoRow);
                 xe[r][c] = bload1f(roth[c], rok[r] && xe_ok ? ro + xe_pos * 4u : kNoRow);
             }
         }
@@ -112,21 +114,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
         U4 fw = U4{0u, 0u, 0u, 0u};
         if (!C.proposal) fw = flip_words(C, i0, row, t, colour);
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) os[j][c] = f4get(so[c], j);
+            for (int c = 0; c < 3; ++c) os[j][c] = so[c].v[j];
             const uint32_t pos = i0 + j;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 float acc_h = 0.0f;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float a = f4get(v[r][c], j);
+                    const float a = v[r][c].v[j];
                     float bx;
                     if (colour == 0)
-                        bx = j == 0 ? xe[r][c] : f4get(v[r][c], j - 1);
+                        bx = j == 0 ? xe[r][c] : v[r][c].v[j - 1];
                     else
-                        bx = (pos + 1 == w || j == 3) ? xe[r][c] : f4get(v[r][c], j + 1);
+                        bx = (pos + 1 == w || j == S - 1) ? xe[r][c] : v[r][c].v[j + 1];
                     acc_h = r == 0 ? fa(a, bx) : fa(fa(acc_h, a), bx);
                 }
                 hs[j][c] = acc_h;
@@ -141,9 +143,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
 
     // Phase 3: accept or reject, store, sums.
     {
-        float ns[3][4];
+        float ns[3][S];
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
             float n[3];
             heis_update(C, colour == 1, os[j], hs[j], hs[j], us[j], ps[j], n, s32, bsum,
                         j < nvalid);
@@ -153,16 +155,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
         }
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            u32x4 vv;
-            vv.x = __float_as_uint(ns[c][0]);
-            vv.y = __float_as_uint(ns[c][1]);
-            vv.z = __float_as_uint(ns[c][2]);
-            vv.w = __float_as_uint(ns[c][3]);
-            __builtin_amdgcn_raw_buffer_store_b128(vv, rown[c], own_off, 0, 0);
+            bstore<S>(rown[c], own_off, ns[c]);
         }
     }
 
     heis_partials_sites(s32, bsum, partials, colour, 2u, s, total_blocks, b);
 }
+
+#define VG_HEIS_BCC(S)                                                                \
+    template __global__ void heis_bcc_pass<S>(const ChainDev*, const uint32_t*, float*, \
+                                              int64_t*, uint32_t, uint32_t, uint32_t,   \
+                                              uint32_t);
+VG_HEIS_BCC(1)
+VG_HEIS_BCC(4)
+#undef VG_HEIS_BCC
 
 }  // namespace vg

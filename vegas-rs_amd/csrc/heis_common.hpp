@@ -26,23 +26,37 @@ __device__ __forceinline__ int64_t fix27(float v) {
     return (int64_t)__float2int_rn(fm(v, kFixScale));
 }
 
-__device__ __forceinline__ float4 ld4(const float* p, bool present) {
-    if (!present) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    return *reinterpret_cast<const float4*>(p);
+// S consecutive fp32 values through a buffer resource (an offset past the plane
+// reads 0, and a store there is dropped).
+template <uint32_t S>
+struct Run {
+    float v[S];
+};
+template <uint32_t S>
+__device__ __forceinline__ Run<S> bload(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    Run<S> o;
+    if constexpr (S == 4) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) o.v[j] = __uint_as_float(v[j]);
+    } else {
+        o.v[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    }
+    return o;
 }
-
-// fp32 loads through a buffer resource (an offset past the plane reads 0).
-__device__ __forceinline__ float4 bload4f(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
-                       __uint_as_float(v.w));
+template <uint32_t S>
+__device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t off, const float (&n)[S]) {
+    if constexpr (S == 4) {
+        u32x4 v;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) v[j] = __float_as_uint(n[j]);
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0);
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(n[0]), r, off, 0, 0);
+    }
 }
 __device__ __forceinline__ float bload1f(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-
-__device__ __forceinline__ float f4get(const float4& v, uint32_t k) {
-    return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w));
 }
 
 // 24-bit value m (0..4) of a Philox call: bits [24m, 24m+24) of the 128-bit
@@ -130,19 +144,20 @@ struct HeisQueue {
 
 // Resolves the wave's pending sites: bit j of pend marks position i0 + j of
 // this lane's row.  Entries are numbered by an exclusive prefix sum of the
-// lanes' counts (three ballots); in rounds of 64, the owners post
+// lanes' counts (a ballot a bit); in rounds of 64, the owners post
 // (position, row), lane e computes entry e's calls 1..15, and the owners
 // read their proposals back.  LDS operations of one wave complete in order,
 // so the wave needs no barrier, only no reordering by the compiler.  Every
 // lane of the wave must call this.
+template <uint32_t S>
 __device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, uint32_t pend,
                                              uint32_t i0, uint32_t row, uint64_t t,
-                                             uint32_t colour, float p[4][3]) {
+                                             uint32_t colour, float (&p)[S][3]) {
     const uint32_t lane = __lane_id();
     const uint32_t cnt = __builtin_popcount(pend);
     uint32_t pre = 0, total = 0;
 #pragma unroll
-    for (uint32_t bit = 0; bit < 3; ++bit) {
+    for (uint32_t bit = 0; bit < (S == 4 ? 3u : 1u); ++bit) {
         const uint64_t m = __ballot((cnt >> bit) & 1u);
         pre += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))
@@ -152,7 +167,7 @@ __device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, ui
     for (uint32_t base = 0; base < total; base += 64) {  // wave-uniform
         uint32_t slot = pre;
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
             if ((pend >> j) & 1u) {
                 const uint32_t e = slot - base;  // wraps past 64 when slot < base
                 if (e < 64) {
@@ -177,7 +192,7 @@ __device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, ui
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         slot = pre;
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
             if ((pend >> j) & 1u) {
                 const uint32_t e = slot - base;
                 if (e < 64) {
@@ -238,16 +253,9 @@ __device__ __forceinline__ void heis_update(const ChainDev& C, bool bond, const 
     if (bond) bsum += fix27(dot3(n[0], n[1], n[2], hb[0], hb[1], hb[2]));
 }
 
-// The int32 site sums of a lane into the five int64 quantities.
-__device__ __forceinline__ void heis_fold(const int32_t s32[4], int64_t bsum, int64_t acc[5]) {
-    acc[0] += bsum;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) acc[1 + k] += (int64_t)s32[k];
-}
-
 // Phase 1 of a site: its acceptance uniform u and proposal p.  Random
 // proposals whose first call missed set bit j of pend (resolved by
-// heis_resolve); flip proposals take word j of fw.
+// heis_resolve); flip proposals take word pos & 3 of fw.
 __device__ __forceinline__ void heis_propose(const ChainDev& C, uint32_t colour, uint32_t pos,
                                              uint32_t row, uint64_t t, const U4& fw, uint32_t j,
                                              const float o[3], float& u, float p[3],
@@ -255,7 +263,7 @@ __device__ __forceinline__ void heis_propose(const ChainDev& C, uint32_t colour,
     if (C.proposal) {
         if (!proposal_first(C, pos, row, t, colour, u, p)) pend |= 1u << j;
     } else {
-        u = unit24(u4_word(fw, j));
+        u = unit24(u4_word(fw, pos & 3u));
         p[0] = -o[0];
         p[1] = -o[1];
         p[2] = -o[2];
@@ -321,17 +329,36 @@ __device__ __forceinline__ void heis_partials(const int32_t s32[4], int64_t bsum
 
 // Workgroup sums of the lattice passes (sc, bcc, fcc): a lane holds at most
 // four sites, each below 2^27 in every magnetisation sum and below
-// z * 2^27 <= 12 * 2^27 in its bond share, so every lane's five values are
-// below 2^40 and reduce with wave_sum_split.
+// z * 2^27 <= 12 * 2^27 in its bond share.  The lanes leave their sums in LDS;
+// wave v then adds the four waves' for its magnetisation component (axis2 for
+// wave 3, the bonds too for wave 0) and reduces it over its lanes, all below
+// 2^40 as wave_sum_split needs.  (Each wave reducing its own five sums took
+// 140 instructions of a wave's 1080, this takes 45.)
 __device__ __forceinline__ void heis_partials_sites(const int32_t s32[4], int64_t bsum,
                                                     int64_t* __restrict__ partials,
                                                     uint32_t colour, uint32_t ncol, uint32_t s,
                                                     uint32_t total_blocks, uint32_t b) {
-    int64_t w[5];
-    w[0] = wave_sum_split(bsum);
+    constexpr uint32_t kW = kBlock / 64;
+    __shared__ int32_t red[4][kBlock];
+    __shared__ int64_t redb[kBlock];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) w[1 + k] = wave_sum_split(s32[k]);
-    heis_block_partials(w, partials, colour, ncol, s, total_blocks, b);
+    for (uint32_t k = 0; k < 4; ++k) red[k][tid] = s32[k];
+    redb[tid] = bsum;
+    __syncthreads();
+    int64_t* const out = partials + ((uint64_t)(s * ncol + colour) * total_blocks + b) * 5u;
+    int64_t v = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kW; ++k) v += red[wave][64u * k + lane];
+    v = wave_sum_split(v);
+    if (lane == 0) out[1u + wave] = v;
+    if (wave == 0) {
+        v = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kW; ++k) v += redb[64u * k + lane];
+        v = wave_sum_split(v);
+        if (lane == 0) out[0] = v;
+    }
 }
 
 }  // namespace vg

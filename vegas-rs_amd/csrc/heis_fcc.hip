@@ -8,18 +8,18 @@
 // of colour a uses the same sum over the slots of the lower colours b < a
 // (the first 4a slots), so over a sweep every bond counts once.
 //
-// Work item: 4 consecutive positions of one row.  Each other sublattice b is
-// read in turn: four neighbour rows at the same x (a and b differ along y and
-// z), or two rows at x and at the x-offset position (they differ along x),
-// one aligned 16-byte load per component and row plus the one position
-// beyond the item.  Same three phases as the sc pass (fields and first
-// proposal calls, the wave's queue, updates).
+// Work item: S = 1 or 4 consecutive positions of one row.  Each other
+// sublattice b is read in turn: four neighbour rows at the same x (a and b
+// differ along y and z), or two rows at x and at the x-offset position (they
+// differ along x), at the item's positions (with four, one aligned 16-byte load
+// per component) and the one position beyond it.  Same three phases as the sc
+// pass (fields and first proposal calls, the wave's queue, updates).
 #include "fcc_common.hpp"
 #include "heis_common.hpp"
 
 namespace vg {
 
-template <uint32_t A>
+template <uint32_t A, uint32_t S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void heis_fcc_pass(const ChainDev* __restrict__ chains,
                                                      const uint32_t* __restrict__ block_chain,
                                                      float* __restrict__ arena,
@@ -52,8 +52,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
     const uint32_t z = fast_div(row, C.ly_m, C.ly_s);
     const uint32_t y = row - z * ly;
     const bool px = pbc & 1u, py = pbc & 2u, pz = pbc & 4u;
-    const uint32_t i0 = seg * kHeisSeg;
-    const uint32_t nvalid = active ? min(kHeisSeg, w - i0) : 0u;
+    const uint32_t i0 = seg * S;
+    const uint32_t nvalid = active ? min(S, w - i0) : 0u;
     const uint32_t own_off = active ? (row * pitch + i0) * 4u : kNoRow;
     const auto rsrc = [&](uint32_t sub, int c) {
         return plane_rsrc(reinterpret_cast<const uint8_t*>(arena + C.off[sub] + c * plane),
@@ -63,23 +63,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
 #pragma unroll
     for (int c = 0; c < 3; ++c) rown[c] = rsrc(A, c);
     uint32_t pend = 0;
-    float os[4][3], hs[4][3], hb[4][3], ps[4][3], us[4];
+    float os[S][3], hs[S][3], hb[S][3], ps[S][3], us[S];
     {
         // x-offset position beyond the item: i0-1 (colours 0, 1) or i0+4,
         // or position 0 across the periodic end (colours 2, 3: the +x slot
         // of position w-1, whichever j it has; 0 when x is open)
         constexpr bool kXneg = A < 2;
-        const bool xr_in = i0 + kHeisSeg < w;
-        const uint32_t xe_pos = kXneg ? (i0 > 0 ? i0 - 1 : w - 1) : (xr_in ? i0 + kHeisSeg : 0);
+        const bool xr_in = i0 + S < w;
+        const uint32_t xe_pos = kXneg ? (i0 > 0 ? i0 - 1 : w - 1) : (xr_in ? i0 + S : 0);
         const bool xe_ok = kXneg ? (i0 > 0 || px) : (xr_in || px);
 
-        float4 so[3];
+        Run<S> so[3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) so[c] = bload4f(rown[c], own_off);
+        for (int c = 0; c < 3; ++c) so[c] = bload<S>(rown[c], own_off);
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j)
+        for (uint32_t j = 0; j < S; ++j)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) os[j][c] = f4get(so[c], j);
+            for (int c = 0; c < 3; ++c) os[j][c] = so[c].v[j];
 
         uint32_t k = 0;  // slots summed so far
 #pragma unroll
@@ -96,19 +96,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
                 // y and z differ: slots (y,z), (y',z), (y,z'), (y',z') at x
                 const uint32_t rows[4] = {row, y2 + ly * z, y + ly * z2, y2 + ly * z2};
                 const bool rok[4] = {true, yok, zok, yok && zok};
-                float4 v[4][3];
+                Run<S> v[4][3];
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
                     for (int c = 0; c < 3; ++c)
-                        v[r][c] = bload4f(roth[c], rok[r] ? (rows[r] * pitch + i0) * 4u : kNoRow);
+                        v[r][c] = bload<S>(roth[c], rok[r] ? (rows[r] * pitch + i0) * 4u : kNoRow);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
 #pragma unroll
-                    for (uint32_t j = 0; j < 4; ++j)
+                    for (uint32_t j = 0; j < S; ++j)
 #pragma unroll
                         for (int c = 0; c < 3; ++c) {
-                            const float vv = f4get(v[r][c], j);
+                            const float vv = v[r][c].v[j];
                             hs[j][c] = k == 0 ? vv : fa(hs[j][c], vv);
                         }
                     ++k;
@@ -120,14 +120,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
                 const uint32_t row2 = (diff & 2u) ? y2 + ly * z : y + ly * z2;
                 const uint32_t rows[2] = {row, row2};
                 const bool rok[2] = {true, ok2};
-                float4 v[2][3];
+                Run<S> v[2][3];
                 float xe[2][3];
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
                     const uint32_t ro = rows[r] * pitch * 4u;
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        v[r][c] = bload4f(roth[c], rok[r] ? ro + i0 * 4u : kNoRow);
+                        v[r][c] = bload<S>(roth[c], rok[r] ? ro + i0 * 4u : kNoRow);
                         xe[r][c] = bload1f(roth[c], rok[r] && xe_ok ? ro + xe_pos * 4u : kNoRow);
                     }
                 }
@@ -136,17 +136,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
 #pragma unroll
                     for (int d1 = 0; d1 < 2; ++d1) {
 #pragma unroll
-                        for (uint32_t j = 0; j < 4; ++j) {
+                        for (uint32_t j = 0; j < S; ++j) {
                             const uint32_t pos = i0 + j;
 #pragma unroll
                             for (int c = 0; c < 3; ++c) {
                                 float vv;
                                 if (d1 == 0)
-                                    vv = f4get(v[r][c], j);
+                                    vv = v[r][c].v[j];
                                 else if (kXneg)
-                                    vv = j == 0 ? xe[r][c] : f4get(v[r][c], j - 1);
+                                    vv = j == 0 ? xe[r][c] : v[r][c].v[j - 1];
                                 else
-                                    vv = (pos + 1 == w || j == 3) ? xe[r][c] : f4get(v[r][c], j + 1);
+                                    vv = (pos + 1 == w || j == S - 1) ? xe[r][c] : v[r][c].v[j + 1];
                                 hs[j][c] = k == 0 ? vv : fa(hs[j][c], vv);
                             }
                         }
@@ -156,14 +156,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
             }
             if (A > 0 && ob + 1 == A) {
 #pragma unroll
-                for (uint32_t j = 0; j < 4; ++j)
+                for (uint32_t j = 0; j < S; ++j)
 #pragma unroll
                     for (int c = 0; c < 3; ++c) hb[j][c] = hs[j][c];
             }
         }
         if (A == 0) {  // no lower colour: the bond share is not summed
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j)
+            for (uint32_t j = 0; j < S; ++j)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) hb[j][c] = 0.0f;
         }
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
         U4 fw = U4{0u, 0u, 0u, 0u};
         if (!C.proposal) fw = flip_words(C, i0, row, t, A);
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j)
+        for (uint32_t j = 0; j < S; ++j)
             heis_propose(C, A, i0 + j, row, t, fw, j, os[j], us[j], ps[j], pend);
         pend &= (1u << nvalid) - 1u;  // no further calls for sites that do not exist
     }
@@ -181,9 +181,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
 
     // Phase 3: accept or reject, store, sums.
     {
-        float ns[3][4];
+        float ns[3][S];
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
             float n[3];
             heis_update(C, A > 0, os[j], hs[j], hb[j], us[j], ps[j], n, s32, bsum, j < nvalid);
             ns[0][j] = n[0];
@@ -192,25 +192,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
         }
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            u32x4 vv;
-            vv.x = __float_as_uint(ns[c][0]);
-            vv.y = __float_as_uint(ns[c][1]);
-            vv.z = __float_as_uint(ns[c][2]);
-            vv.w = __float_as_uint(ns[c][3]);
-            __builtin_amdgcn_raw_buffer_store_b128(vv, rown[c], own_off, 0, 0);
+            bstore<S>(rown[c], own_off, ns[c]);
         }
     }
 
     heis_partials_sites(s32, bsum, partials, A, 4u, s, total_blocks, b);
 }
 
-template __global__ void heis_fcc_pass<0>(const ChainDev*, const uint32_t*, float*, int64_t*,
-                                          uint32_t, uint32_t, uint32_t);
-template __global__ void heis_fcc_pass<1>(const ChainDev*, const uint32_t*, float*, int64_t*,
-                                          uint32_t, uint32_t, uint32_t);
-template __global__ void heis_fcc_pass<2>(const ChainDev*, const uint32_t*, float*, int64_t*,
-                                          uint32_t, uint32_t, uint32_t);
-template __global__ void heis_fcc_pass<3>(const ChainDev*, const uint32_t*, float*, int64_t*,
-                                          uint32_t, uint32_t, uint32_t);
+#define VG_HEIS_FCC(A, S)                                                                \
+    template __global__ void heis_fcc_pass<A, S>(const ChainDev*, const uint32_t*, float*, \
+                                                 int64_t*, uint32_t, uint32_t, uint32_t);
+#define VG_HEIS_FCC_ITEM(S) \
+    VG_HEIS_FCC(0, S)       \
+    VG_HEIS_FCC(1, S)       \
+    VG_HEIS_FCC(2, S)       \
+    VG_HEIS_FCC(3, S)
+VG_HEIS_FCC_ITEM(1)
+VG_HEIS_FCC_ITEM(4)
+#undef VG_HEIS_FCC_ITEM
+#undef VG_HEIS_FCC
 
 }  // namespace vg

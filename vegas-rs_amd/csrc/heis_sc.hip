@@ -8,13 +8,13 @@
 // (src/energy.rs:64-214): one sweep updates every colour-0 site, then every
 // colour-1 site.
 //
-// Work item: 4 consecutive positions of one row (one aligned 16-byte load per
-// component per row touched).  Random proposals draw from each site's own
-// Philox calls (counter x = i), so the four sites are independent; flip
-// proposals take word i & 3 of one call per item (counter x = i / 4).  The
-// item runs in three phases -- fields and first proposal calls, the wave's
-// queue of sites whose first call missed, then the updates -- so the rare
-// further calls cost one wave-wide call per round of 64 such sites instead
+// Work item: S = 1 or 4 consecutive positions of one row, by the number of
+// waves (four: one aligned 16-byte load per component per row touched).  Random
+// proposals draw from each site's own Philox calls (counter x = i), so the
+// sites are independent; flip proposals take word i & 3 of the call of counter
+// x = i / 4.  The item runs in three phases -- fields and first proposal calls,
+// the wave's queue of sites whose first call missed, then the updates -- so the
+// rare further calls cost one wave-wide call per round of 64 such sites instead
 // of one per site.
 // All arithmetic is single IEEE fp32 operations in a fixed order (no
 // contraction), so the CPU oracle reproduces every bit.
@@ -22,6 +22,7 @@
 
 namespace vg {
 
+template <uint32_t S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void heis_sc_pass(const ChainDev* __restrict__ chains,
                                                     const uint32_t* __restrict__ block_chain,
                                                     float* __restrict__ arena,
@@ -66,11 +67,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
     const uint32_t ly = C.ly, lz = C.lz, w = C.w, pitch = C.pitch, pbc = C.pbc;
     const uint32_t z = fast_div(row, C.ly_m, C.ly_s), y = row - z * ly;
     const uint32_t q = (colour + y + z) & 1u;
-    i0 = seg * kHeisSeg;
-    nvalid = active ? min(kHeisSeg, w - i0) : 0u;
+    i0 = seg * S;
+    nvalid = active ? min(S, w - i0) : 0u;
     const uint32_t own_off = active ? (row * pitch + i0) * 4u : kNoRow;
     const uint32_t orow = row * pitch * 4u;
-    float os[4][3], hs[4][3], ps[4][3], us[4];
+    float os[S][3], hs[S][3], ps[S][3], us[S];
     {
         const bool ym_ok = (y > 0) || (pbc & 2u);
         const bool yp_ok = (y + 1 < ly) || (pbc & 2u);
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
         const uint32_t r_zm = z > 0 ? row - ly : row + (lz - 1) * ly;
         const uint32_t r_zp = z + 1 < lz ? row + ly : row - (lz - 1) * ly;
 
-        float4 so[3], mid[3], ym[3], yp[3], zm[3], zp[3];
+        Run<S> so[3], mid[3], ym[3], yp[3], zm[3], zp[3];
         float xe[3];  // the extra x neighbour (position i0-1 or i0+4)
         bool xe_ok = true;
         uint32_t xe_pos;
@@ -89,48 +90,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
             xe_pos = i0 > 0 ? i0 - 1 : w - 1;
             xe_ok = i0 > 0 || (pbc & 1u);
         } else {
-            xe_pos = i0 + kHeisSeg < w ? i0 + kHeisSeg : 0;
-            xe_ok = i0 + kHeisSeg < w || (pbc & 1u);
+            xe_pos = i0 + S < w ? i0 + S : 0;
+            xe_ok = i0 + S < w || (pbc & 1u);
         }
         // With q = 1 the last segment's extra neighbour is position 0: the
         // +x neighbour of position w-1 across the periodic end (0 when x is
         // open), whichever j that position has.
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            so[c] = bload4f(rown[c], own_off);
-            mid[c] = bload4f(roth[c], orow + i0 * 4u);
-            ym[c] = bload4f(roth[c], ym_ok ? (r_ym * pitch + i0) * 4u : kNoRow);
-            yp[c] = bload4f(roth[c], yp_ok ? (r_yp * pitch + i0) * 4u : kNoRow);
-            zm[c] = bload4f(roth[c], zm_ok ? (r_zm * pitch + i0) * 4u : kNoRow);
-            zp[c] = bload4f(roth[c], zp_ok ? (r_zp * pitch + i0) * 4u : kNoRow);
+            so[c] = bload<S>(rown[c], own_off);
+            mid[c] = bload<S>(roth[c], orow + i0 * 4u);
+            ym[c] = bload<S>(roth[c], ym_ok ? (r_ym * pitch + i0) * 4u : kNoRow);
+            yp[c] = bload<S>(roth[c], yp_ok ? (r_yp * pitch + i0) * 4u : kNoRow);
+            zm[c] = bload<S>(roth[c], zm_ok ? (r_zm * pitch + i0) * 4u : kNoRow);
+            zp[c] = bload<S>(roth[c], zp_ok ? (r_zp * pitch + i0) * 4u : kNoRow);
             xe[c] = bload1f(roth[c], xe_ok ? orow + xe_pos * 4u : kNoRow);
         }
 
         U4 fw = U4{0u, 0u, 0u, 0u};
         if (!C.proposal) fw = flip_words(C, i0, row, t, colour);
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) os[j][c] = f4get(so[c], j);
+            for (int c = 0; c < 3; ++c) os[j][c] = so[c].v[j];
             const uint32_t pos = i0 + j;
             // x neighbours, -x then +x: positions pos-1, pos (q = 0) or
             // pos, pos+1 (q = 1) of the other plane's row.
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const float here = f4get(mid[c], j);
+                const float here = mid[c].v[j];
                 float nmx, npx;
                 if (q == 0) {
-                    nmx = j == 0 ? xe[c] : f4get(mid[c], j - 1);
+                    nmx = j == 0 ? xe[c] : mid[c].v[j - 1];
                     npx = here;
                 } else {
                     nmx = here;
-                    npx = (pos + 1 == w || j == 3) ? xe[c] : f4get(mid[c], j + 1);
+                    npx = (pos + 1 == w || j == S - 1) ? xe[c] : mid[c].v[j + 1];
                 }
                 float v = fa(nmx, npx);
-                v = fa(v, f4get(ym[c], j));
-                v = fa(v, f4get(yp[c], j));
-                v = fa(v, f4get(zm[c], j));
-                v = fa(v, f4get(zp[c], j));
+                v = fa(v, ym[c].v[j]);
+                v = fa(v, yp[c].v[j]);
+                v = fa(v, zm[c].v[j]);
+                v = fa(v, zp[c].v[j]);
                 hs[j][c] = v;
             }
             heis_propose(C, colour, pos, row, t, fw, j, os[j], us[j], ps[j], pend);
@@ -143,9 +144,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
 
     // Phase 3: accept or reject, store, sums.
     {
-        float ns[3][4];
+        float ns[3][S];
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < S; ++j) {
             float n[3];
             heis_update(C, colour == 1, os[j], hs[j], hs[j], us[j], ps[j], n, s32, bsum,
                         j < nvalid);
@@ -155,17 +156,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
         }
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            u32x4 v;
-            v.x = __float_as_uint(ns[c][0]);
-            v.y = __float_as_uint(ns[c][1]);
-            v.z = __float_as_uint(ns[c][2]);
-            v.w = __float_as_uint(ns[c][3]);
-            __builtin_amdgcn_raw_buffer_store_b128(v, rown[c], own_off, 0, 0);
+            bstore<S>(rown[c], own_off, ns[c]);
         }
     }
 
     heis_partials_sites(s32, bsum, partials, colour, 2u, s, total_blocks, b);
 }
+
+#define VG_HEIS_SC(S)                                                                           \
+    template __global__ void heis_sc_pass<S>(const ChainDev*, const uint32_t*, float*, int64_t*, \
+                                             uint32_t, uint32_t, uint32_t, uint32_t);
+VG_HEIS_SC(1)
+VG_HEIS_SC(4)
+#undef VG_HEIS_SC
 
 // record = {bond, mx, my, mz, axis2}, summed over the ncol colour passes (a
 // pass adds the bonds to lower colours only, so each bond counts once).

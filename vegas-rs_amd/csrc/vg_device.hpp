@@ -173,7 +173,7 @@ struct ChainDev {
 
 constexpr uint32_t kBlock = 256;       // threads per workgroup of a pass
 constexpr uint32_t kIsingSeg = 32;     // positions per Ising work item (one word of site bits)
-constexpr uint32_t kHeisSeg = 4;       // positions per Heisenberg work item
+constexpr uint32_t kHeisSeg = 4;       // most positions per Heisenberg work item
 constexpr uint32_t kNumXcd = 8;        // MI355X: 8 XCDs, workgroups dealt round-robin
 // Wolff chains of at most this many sites keep their spins and visit marks
 // in LDS, one bit per site each (2 x 64 KiB of the 160 KiB of a CU), and the
