@@ -46,15 +46,6 @@ struct GraphHead {
     bool go;     // a site of this class, in a sweep that the chain runs
 };
 
-__device__ __forceinline__ uint64_t loaded(uint64_t v) {
-    asm volatile("" : "+s"(v));
-    return v;
-}
-__device__ __forceinline__ uint32_t loaded(uint32_t v) {
-    asm volatile("" : "+s"(v));
-    return v;
-}
-
 __device__ __forceinline__ GraphHead graph_head(const ChainDev& C, const uint8_t* arena,
                                                 uint32_t colour, uint32_t s, uint32_t b) {
     const uint32_t* const held = &C.plan[0][0];
@@ -227,7 +218,7 @@ __global__ __launch_bounds__(256) void graph_heis_pass(const ChainDev* __restric
         const float o[3] = {xs[p], ys[p], zs[p]};
         float u, pr[3];
         if (H.proposal) {
-            if (!proposal_first(C, site, 0u, t, 0u, u, pr)) proposal_rest(C, site, 0u, t, 0u, pr);
+            if (!proposal_first(H.seed, site, 0u, t, 0u, u, pr)) proposal_rest(H.seed, site, 0u, t, 0u, pr);
         } else {
             const U4 fw = philox(U4{site, 0u, (uint32_t)t, ctr_w(t, kHeisStream, 0)},
                                  (uint32_t)H.seed, (uint32_t)(H.seed >> 32));

@@ -26,12 +26,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
                                                      uint32_t total_blocks, uint32_t grid) {
     __shared__ HeisQueue hq[kBlock / 64];
     const uint32_t b = xcd_block(blockIdx.x, grid);
-    if (b >= total_blocks) return;  // uniform over the workgroup
-    const ChainDev& C = chains[block_chain[b]];
-    if (s >= C.limit) return;  // uniform: the workgroup belongs to one chain
-    const uint32_t local = (b - C.block0) * kBlock + threadIdx.x;
-    const bool active = local < C.items;
-    const uint64_t t = C.sweep0 + s;
+    const ChainDev& C = chains[block_chain[min(b, total_blocks - 1u)]];
+    const HeisHead H = heis_head(C, b, total_blocks, s);
+    const bool active = H.active, rnd = H.proposal != 0;
+    const uint64_t t = H.t;
     int32_t s32[4] = {0, 0, 0, 0};     // mx, my, mz, axis2 of the lane's sites
     int64_t bsum = 0;                  // bond of the lane's sites
 
@@ -41,13 +39,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
     // 0 for an absent neighbour row.
     __amdgpu_buffer_rsrc_t rown[3], roth[3];
     {
-        const uint64_t plane = C.plane;
+        const uint64_t plane = H.plane;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            rown[c] = plane_rsrc(reinterpret_cast<const uint8_t*>(arena + C.off[colour] + c * plane),
+            rown[c] = plane_rsrc(reinterpret_cast<const uint8_t*>(arena + (colour ? H.off[1] : H.off[0]) + c * plane),
                                  (uint32_t)(plane * 4u));
             roth[c] = plane_rsrc(
-                reinterpret_cast<const uint8_t*>(arena + C.off[colour ^ 1u] + c * plane),
+                reinterpret_cast<const uint8_t*>(arena + (colour ? H.off[0] : H.off[1]) + c * plane),
                 (uint32_t)(plane * 4u));
         }
     }
@@ -56,11 +54,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
     // kNoRow, so it reads zeros and its stores are dropped; a site j >=
     // nvalid of a short last segment is padding, which every kernel keeps at
     // zero.  Neither is ever accepted, so both add zero to the sums.
-    const uint32_t ly = C.ly, lz = C.lz, w = C.w, pitch = C.pitch, pbc = C.pbc;
-    const uint32_t row = fast_div(local, C.segs_m, C.segs_s);
-    const uint32_t seg = local - row * C.segs;
-    const uint32_t z = fast_div(row, C.ly_m, C.ly_s);
-    const uint32_t y = row - z * ly;
+    const uint32_t ly = H.ly, lz = H.lz, w = H.w, pitch = H.pitch, pbc = H.pbc;
+    const uint32_t row = H.row;
+    const uint32_t seg = H.seg;
+    const uint32_t z = H.z, y = H.y;
     const bool px = pbc & 1u, py = pbc & 2u, pz = pbc & 4u;
     const uint32_t i0 = seg * S;
     const uint32_t nvalid = active ? min(S, w - i0) : 0u;
@@ -111,8 +108,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
             }
         }
 
-        U4 fw = U4{0u, 0u, 0u, 0u};
-        if (!C.proposal) fw = flip_words(C, i0, row, t, colour);
+        heis_propose<S>(H.seed, rnd, colour, i0, row, t, us, ps, pend);
 #pragma unroll
         for (uint32_t j = 0; j < S; ++j) {
 #pragma unroll
@@ -133,13 +129,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
                 }
                 hs[j][c] = acc_h;
             }
-            heis_propose(C, colour, pos, row, t, fw, j, os[j], us[j], ps[j], pend);
         }
         pend &= (1u << nvalid) - 1u;  // no further calls for sites that do not exist
     }
 
     // Phase 2: the wave's sites whose first proposal call missed.
-    if (C.proposal) heis_resolve(C, hq[threadIdx.x >> 6], pend, i0, row, t, colour, ps);
+    if (rnd) heis_resolve(H.seed, hq[threadIdx.x >> 6], pend, i0, row, t, colour, ps);
 
     // Phase 3: accept or reject, store, sums.
     {
@@ -147,6 +142,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
 #pragma unroll
         for (uint32_t j = 0; j < S; ++j) {
             float n[3];
+            if (!rnd) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) ps[j][c] = -os[j][c];
+            }
             heis_update(C, colour == 1, os[j], hs[j], hs[j], us[j], ps[j], n, s32, bsum,
                         j < nvalid);
             ns[0][j] = n[0];
@@ -159,7 +158,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
         }
     }
 
-    heis_partials_sites(s32, bsum, partials, colour, 2u, s, total_blocks, b);
+    heis_partials_sites(s32, bsum, partials, colour, 2u, s, total_blocks, b, H.run);
 }
 
 #define VG_HEIS_BCC(S)                                                                \

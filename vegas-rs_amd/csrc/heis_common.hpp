@@ -64,9 +64,9 @@ __device__ __forceinline__ float bload1f(__amdgpu_buffer_rsrc_t r, uint32_t off)
 __device__ __forceinline__ uint32_t v24(const U4& c, int m) {
     switch (m) {
         case 0: return c.x & 0xFFFFFFu;
-        case 1: return __builtin_amdgcn_alignbit(c.y, c.x, 24) & 0xFFFFFFu;
-        case 2: return __builtin_amdgcn_alignbit(c.z, c.y, 16) & 0xFFFFFFu;
-        case 3: return __builtin_amdgcn_alignbit(c.w, c.z, 8) & 0xFFFFFFu;
+        case 1: return __builtin_amdgcn_perm(c.y, c.x, 0x0C050403u);  // three bytes and a zero
+        case 2: return __builtin_amdgcn_perm(c.z, c.y, 0x0C040302u);
+        case 3: return c.z >> 8;
         default: return c.w & 0xFFFFFFu;
     }
 }
@@ -90,10 +90,68 @@ __device__ __forceinline__ Try mtry(uint32_t a, uint32_t b) {
 
 // A Marsaglia try inside the unit disc -> point on the sphere.
 __device__ __forceinline__ void sphere_point(const Try& a, float p[3]) {
-    const float root = sqrt_rn(fs(1.0f, a.q));
-    p[0] = fm(fm(2.0f, a.x1), root);
-    p[1] = fm(fm(2.0f, a.x2), root);
+    // twice a float is exact: (2 x) root and x (2 root) round alike
+    const float root2 = fm(2.0f, sqrt_rn(fs(1.0f, a.q)));
+    p[0] = fm(a.x1, root2);
+    p[1] = fm(a.x2, root2);
     p[2] = ff(-2.0f, a.q, 1.0f);  // 2q is exact: the same rounding as fs(1, 2q)
+}
+
+// What a colour pass's wave needs of its chain, loaded in one batch; workgroups
+// past the work and chains that run fewer sweeps in this block are not sent away
+// before it.
+struct HeisHead {
+    uint64_t off[4], plane, seed, t;
+    uint32_t segs, ly, lz, w, pitch, pbc, proposal;
+    uint32_t row, seg, y, z;  // the lane's item
+    bool run;                 // the workgroup has work in this sweep
+    bool active;              // the lane has an item
+};
+__device__ __forceinline__ HeisHead heis_head(const ChainDev& C, uint32_t b, uint32_t total_blocks,
+                                              uint32_t s) {
+    HeisHead h;
+    uint32_t limit = C.limit, block0 = C.block0, items = C.items;
+    uint32_t segs_m = C.segs_m, segs_s = C.segs_s, ly_m = C.ly_m, ly_s = C.ly_s;
+    uint64_t sweep0 = C.sweep0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) h.off[k] = C.off[k];
+    h.plane = C.plane;
+    h.seed = C.seed;
+    h.segs = C.segs;
+    h.ly = C.ly;
+    h.lz = C.lz;
+    h.w = C.w;
+    h.pitch = C.pitch;
+    h.pbc = C.pbc;
+    h.proposal = C.proposal;
+    sweep0 = loaded(sweep0);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) h.off[k] = loaded(h.off[k]);
+    h.plane = loaded(h.plane);
+    h.seed = loaded(h.seed);
+    limit = loaded(limit);
+    block0 = loaded(block0);
+    items = loaded(items);
+    segs_m = loaded(segs_m);
+    segs_s = loaded(segs_s);
+    ly_m = loaded(ly_m);
+    ly_s = loaded(ly_s);
+    h.segs = loaded(h.segs);
+    h.ly = loaded(h.ly);
+    h.lz = loaded(h.lz);
+    h.w = loaded(h.w);
+    h.pitch = loaded(h.pitch);
+    h.pbc = loaded(h.pbc);
+    h.proposal = loaded(h.proposal);
+    h.t = sweep0 + s;
+    h.run = b < total_blocks && s < limit;
+    const uint32_t local = (b - block0) * kBlock + threadIdx.x;
+    h.active = h.run && local < items;
+    h.row = fast_div(local, segs_m, segs_s);
+    h.seg = local - h.row * h.segs;
+    h.z = fast_div(h.row, ly_m, ly_s);
+    h.y = h.row - h.z * h.ly;
+    return h;
 }
 
 // Fresh uniform-sphere proposal of one site (Spin::rand -> marsaglia,
@@ -105,10 +163,10 @@ __device__ __forceinline__ void sphere_point(const Try& a, float p[3]) {
 // proposal_first does call 0 (both tries without branches) and returns
 // whether one hit (p = 0.954); proposal_rest does calls 1..15 for a site
 // whose first two tries missed.
-__device__ __forceinline__ bool proposal_first(const ChainDev& C, uint32_t pos, uint32_t row,
+__device__ __forceinline__ bool proposal_first(uint64_t seed, uint32_t pos, uint32_t row,
                                                uint64_t t, uint32_t colour, float& u, float p[3]) {
     const U4 c0 = philox(U4{pos, row, (uint32_t)t, ctr_w(t, kHeisStream, colour)},
-                         (uint32_t)C.seed, (uint32_t)(C.seed >> 32));
+                         (uint32_t)seed, (uint32_t)(seed >> 32));
     u = f24u(v24(c0, 0));
     const Try t0 = mtry(v24(c0, 1), v24(c0, 2));
     const Try t1 = mtry(v24(c0, 3), v24(c0, 4));
@@ -120,9 +178,9 @@ __device__ __forceinline__ bool proposal_first(const ChainDev& C, uint32_t pos, 
     return ok;
 }
 
-__device__ __forceinline__ void proposal_rest(const ChainDev& C, uint32_t pos, uint32_t row,
+__device__ __forceinline__ void proposal_rest(uint64_t seed, uint32_t pos, uint32_t row,
                                               uint64_t t, uint32_t colour, float p[3]) {
-    const uint32_t k0 = (uint32_t)C.seed, k1 = (uint32_t)(C.seed >> 32);
+    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
     for (uint32_t k = 1; k < kHeisMaxCalls; ++k) {
         const U4 ck = philox(U4{pos, row, (uint32_t)t, ctr_w(t, kHeisStream + k, colour)}, k0, k1);
         const Try a = mtry(v24(ck, 0), v24(ck, 1));
@@ -150,7 +208,7 @@ struct HeisQueue {
 // so the wave needs no barrier, only no reordering by the compiler.  Every
 // lane of the wave must call this.
 template <uint32_t S>
-__device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, uint32_t pend,
+__device__ __forceinline__ void heis_resolve(uint64_t seed, HeisQueue& q, uint32_t pend,
                                              uint32_t i0, uint32_t row, uint64_t t,
                                              uint32_t colour, float (&p)[S][3]) {
     const uint32_t lane = __lane_id();
@@ -182,7 +240,7 @@ __device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, ui
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (lane < total - base) {
             float r[3];
-            proposal_rest(C, q.pos[lane], q.row[lane], t, colour, r);
+            proposal_rest(seed, q.pos[lane], q.row[lane], t, colour, r);
             q.p[0][lane] = r[0];
             q.p[1][lane] = r[1];
             q.p[2][lane] = r[2];
@@ -211,10 +269,10 @@ __device__ __forceinline__ void heis_resolve(const ChainDev& C, HeisQueue& q, ui
 
 // Flip proposals (-s) take their acceptance uniform from word (i & 3) of one
 // call per 4 positions, counter (i >> 2, row, sweep, purpose 16).
-__device__ __forceinline__ U4 flip_words(const ChainDev& C, uint32_t i0, uint32_t row, uint64_t t,
+__device__ __forceinline__ U4 flip_words(uint64_t seed, uint32_t i0, uint32_t row, uint64_t t,
                                          uint32_t colour) {
-    return philox(U4{i0 >> 2, row, (uint32_t)t, ctr_w(t, kHeisStream, colour)},
-                  (uint32_t)C.seed, (uint32_t)(C.seed >> 32));
+    return philox(U4{i0 >> 2, row, (uint32_t)t, ctr_w(t, kHeisStream, colour)}, (uint32_t)seed,
+                  (uint32_t)(seed >> 32));
 }
 
 __device__ __forceinline__ int32_t fix27_32(float v) { return __float2int_rn(fm(v, kFixScale)); }
@@ -240,8 +298,7 @@ __device__ __forceinline__ void heis_update(const ChainDev& C, bool bond, const 
     const float e_an = fm(C.kk, ff(pe, pe, -fm(oe, oe)));
     const float e_ze = fm(C.hm, dot3(dx, dy, dz, C.fx, C.fy, C.fz));
     const float dE = fa(fa(e_ex, e_an), e_ze);
-    bool accept = valid && dE < 0.0f;
-    if (valid && !accept) accept = u < exp_nonpos(-fm(dE, C.beta));
+    const bool accept = valid & ((dE < 0.0f) | (u < exp_nonpos(-fm(dE, C.beta))));
     n[0] = accept ? px : ox;
     n[1] = accept ? py : oy;
     n[2] = accept ? pz : oz;
@@ -253,20 +310,48 @@ __device__ __forceinline__ void heis_update(const ChainDev& C, bool bond, const 
     if (bond) bsum += fix27(dot3(n[0], n[1], n[2], hb[0], hb[1], hb[2]));
 }
 
-// Phase 1 of a site: its acceptance uniform u and proposal p.  Random
-// proposals whose first call missed set bit j of pend (resolved by
-// heis_resolve); flip proposals take word pos & 3 of fw.
-__device__ __forceinline__ void heis_propose(const ChainDev& C, uint32_t colour, uint32_t pos,
-                                             uint32_t row, uint64_t t, const U4& fw, uint32_t j,
-                                             const float o[3], float& u, float p[3],
-                                             uint32_t& pend) {
-    if (C.proposal) {
-        if (!proposal_first(C, pos, row, t, colour, u, p)) pend |= 1u << j;
+// An item's acceptance uniforms u and, for random proposals, its proposals p
+// (bit j of pend: the first call missed, heis_resolve does the rest); flip
+// proposals take word pos & 3 of their call.  They need no spins: written after
+// an item's loads and before the loads' first use, and kept there by the empty
+// asm statements (HOLD), they are made while the loads are on their way (left
+// to itself the compiler sums the fields, and waits, first: sc 128^3 x 3, 25.8
+// us a pass, 24.6 so).  Without, for items of four on fcc, whose registers it
+// would pass: 128^3 x 3 116 us a pass, 78 so.
+template <uint32_t S, bool HOLD = true>
+__device__ __forceinline__ void heis_propose(uint64_t seed, bool random, uint32_t colour,
+                                             uint32_t i0, uint32_t row, uint64_t t, float (&u)[S],
+                                             float (&p)[S][3], uint32_t& pend) {
+    const auto first = [&](uint32_t j) {
+        if (!proposal_first(seed, i0 + j, row, t, colour, u[j], p[j])) pend |= 1u << j;
+    };
+    const auto flip = [&](const U4& fw, uint32_t j) {
+        u[j] = unit24(u4_word(fw, (i0 + j) & 3u));
+        p[j][0] = p[j][1] = p[j][2] = 0.0f;
+    };
+    if constexpr (HOLD) {
+        if (random) {
+#pragma unroll
+            for (uint32_t j = 0; j < S; ++j) first(j);
+        } else {
+            const U4 fw = flip_words(seed, i0, row, t, colour);
+#pragma unroll
+            for (uint32_t j = 0; j < S; ++j) flip(fw, j);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < S; ++j)
+            asm volatile("" : "+v"(u[j]), "+v"(p[j][0]), "+v"(p[j][1]), "+v"(p[j][2]));
     } else {
-        u = unit24(u4_word(fw, pos & 3u));
-        p[0] = -o[0];
-        p[1] = -o[1];
-        p[2] = -o[2];
+        U4 fw = U4{0u, 0u, 0u, 0u};
+        if (!random) fw = flip_words(seed, i0, row, t, colour);
+#pragma unroll
+        for (uint32_t j = 0; j < S; ++j) {
+            // (a branch a site keeps the sites' work apart, and its registers)
+            if (random)
+                first(j);
+            else
+                flip(fw, j);
+        }
     }
 }
 
@@ -337,7 +422,7 @@ __device__ __forceinline__ void heis_partials(const int32_t s32[4], int64_t bsum
 __device__ __forceinline__ void heis_partials_sites(const int32_t s32[4], int64_t bsum,
                                                     int64_t* __restrict__ partials,
                                                     uint32_t colour, uint32_t ncol, uint32_t s,
-                                                    uint32_t total_blocks, uint32_t b) {
+                                                    uint32_t total_blocks, uint32_t b, bool run) {
     constexpr uint32_t kW = kBlock / 64;
     __shared__ int32_t red[4][kBlock];
     __shared__ int64_t redb[kBlock];
@@ -351,13 +436,13 @@ __device__ __forceinline__ void heis_partials_sites(const int32_t s32[4], int64_
 #pragma unroll
     for (uint32_t k = 0; k < kW; ++k) v += red[wave][64u * k + lane];
     v = wave_sum_split(v);
-    if (lane == 0) out[1u + wave] = v;
+    if (lane == 0 && run) out[1u + wave] = v;
     if (wave == 0) {
         v = 0;
 #pragma unroll
         for (uint32_t k = 0; k < kW; ++k) v += redb[64u * k + lane];
         v = wave_sum_split(v);
-        if (lane == 0) out[0] = v;
+        if (lane == 0 && run) out[0] = v;
     }
 }
 

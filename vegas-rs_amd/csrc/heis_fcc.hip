@@ -27,12 +27,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
                                                      uint32_t total_blocks, uint32_t grid) {
     __shared__ HeisQueue hq[kBlock / 64];
     const uint32_t b = xcd_block(blockIdx.x, grid);
-    if (b >= total_blocks) return;  // uniform over the workgroup
-    const ChainDev& C = chains[block_chain[b]];
-    if (s >= C.limit) return;  // uniform: the workgroup belongs to one chain
-    const uint32_t local = (b - C.block0) * kBlock + threadIdx.x;
-    const bool active = local < C.items;
-    const uint64_t t = C.sweep0 + s;
+    const ChainDev& C = chains[block_chain[min(b, total_blocks - 1u)]];
+    const HeisHead H = heis_head(C, b, total_blocks, s);
+    const bool active = H.active, rnd = H.proposal != 0;
+    const uint64_t t = H.t;
     int32_t s32[4] = {0, 0, 0, 0};     // mx, my, mz, axis2 of the lane's sites
     int64_t bsum = 0;                  // bond of the lane's sites
 
@@ -45,18 +43,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
     // dropped; a site j >= nvalid of a short last segment is padding, which
     // every kernel keeps at zero.  Neither is ever accepted, so both add
     // zero to the sums.
-    const uint32_t ly = C.ly, lz = C.lz, w = C.w, pitch = C.pitch, pbc = C.pbc;
-    const uint64_t plane = C.plane;
-    const uint32_t row = fast_div(local, C.segs_m, C.segs_s);
-    const uint32_t seg = local - row * C.segs;
-    const uint32_t z = fast_div(row, C.ly_m, C.ly_s);
-    const uint32_t y = row - z * ly;
+    const uint32_t ly = H.ly, lz = H.lz, w = H.w, pitch = H.pitch, pbc = H.pbc;
+    const uint64_t plane = H.plane;
+    const uint32_t row = H.row;
+    const uint32_t seg = H.seg;
+    const uint32_t z = H.z, y = H.y;
     const bool px = pbc & 1u, py = pbc & 2u, pz = pbc & 4u;
     const uint32_t i0 = seg * S;
     const uint32_t nvalid = active ? min(S, w - i0) : 0u;
     const uint32_t own_off = active ? (row * pitch + i0) * 4u : kNoRow;
     const auto rsrc = [&](uint32_t sub, int c) {
-        return plane_rsrc(reinterpret_cast<const uint8_t*>(arena + C.off[sub] + c * plane),
+        return plane_rsrc(reinterpret_cast<const uint8_t*>(arena + H.off[sub] + c * plane),
                           (uint32_t)(plane * 4u));
     };
     __amdgpu_buffer_rsrc_t rown[3];
@@ -168,16 +165,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
                 for (int c = 0; c < 3; ++c) hb[j][c] = 0.0f;
         }
 
-        U4 fw = U4{0u, 0u, 0u, 0u};
-        if (!C.proposal) fw = flip_words(C, i0, row, t, A);
+        // (held in place, items of four would pass the registers)
+        heis_propose<S, S == 1>(H.seed, rnd, A, i0, row, t, us, ps, pend);
+        if (!rnd) {
 #pragma unroll
-        for (uint32_t j = 0; j < S; ++j)
-            heis_propose(C, A, i0 + j, row, t, fw, j, os[j], us[j], ps[j], pend);
+            for (uint32_t j = 0; j < S; ++j)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) ps[j][c] = -os[j][c];
+        }
         pend &= (1u << nvalid) - 1u;  // no further calls for sites that do not exist
     }
 
     // Phase 2: the wave's sites whose first proposal call missed.
-    if (C.proposal) heis_resolve(C, hq[threadIdx.x >> 6], pend, i0, row, t, A, ps);
+    if (rnd) heis_resolve(H.seed, hq[threadIdx.x >> 6], pend, i0, row, t, A, ps);
 
     // Phase 3: accept or reject, store, sums.
     {
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
         }
     }
 
-    heis_partials_sites(s32, bsum, partials, A, 4u, s, total_blocks, b);
+    heis_partials_sites(s32, bsum, partials, A, 4u, s, total_blocks, b, H.run);
 }
 
 #define VG_HEIS_FCC(A, S)                                                                \

@@ -41,10 +41,10 @@ __global__ __launch_bounds__(256) void heis_draws(const ChainDev* __restrict__ c
     float u, p[3] = {0.0f, 0.0f, 0.0f};
     const uint64_t at = (uint64_t)blockIdx.z * stride * ns + (uint64_t)blockIdx.y * nc + site;
     if (C.proposal) {
-        if (!proposal_first(C, i, row, t, c, u, p)) proposal_rest(C, i, row, t, c, p);
+        if (!proposal_first(C.seed, i, row, t, c, u, p)) proposal_rest(C.seed, i, row, t, c, p);
         out[at] = make_float4(p[0], p[1], p[2], u);
     } else {
-        u = unit24(u4_word(flip_words(C, i, row, t, c), i & 3u));
+        u = unit24(u4_word(flip_words(C.seed, i, row, t, c), i & 3u));
         out[at].w = u;
     }
 }

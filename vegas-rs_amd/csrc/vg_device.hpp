@@ -212,8 +212,8 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t grid) {
 // device results are bit-identical.  Returns 0 below -86, where e^x < 2^-124
 // (the caller compares a uniform in [0,1) against it); above, the result is
 // a normal number, so denormal modes never matter.
+// No branches: a wave nearly always has lanes on both sides.
 VG_HD float exp_nonpos(float x) {
-    if (x < -86.0f) return 0.0f;
     const float log2e = (float)1.4426950408889634;
     const float ln2_hi = 0.693145751953125f;
     const float ln2_lo = (float)(0.6931471805599453 - 0.693145751953125);
@@ -228,13 +228,12 @@ VG_HD float exp_nonpos(float x) {
     p = fmaf(p, r, 0.5f);
     p = fmaf(p, r, 1.0f);
     p = fmaf(p, r, 1.0f);
-    const int e = (int)n + 127;          // n in [-124, 0]: normal scale factor
-    union {
-        uint32_t u;
-        float f;
-    } s;
-    s.u = (uint32_t)e << 23;
-    return p * s.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+    p = __builtin_amdgcn_ldexpf(p, (int)n);  // a normal number: exact
+#else
+    if (x >= -86.0f) p = ldexpf(p, (int)n);
+#endif
+    return x < -86.0f ? 0.0f : p;
 }
 
 // e^x for x <= 0 in f64, the graph chains' acceptance: Cody and Waite's
@@ -280,11 +279,10 @@ __device__ __forceinline__ float sqrt_rn(float x) {
     float s = __builtin_amdgcn_sqrtf(x);
     const uint32_t u = __float_as_uint(s);
     const float sm = __uint_as_float(u - 1u), sp = __uint_as_float(u + 1u);
-    if (__builtin_fmaf(-sm, s, x) <= 0.0f)
-        s = sm;
-    else if (__builtin_fmaf(-sp, s, x) > 0.0f)
-        s = sp;
-    return s;
+    const bool low = __builtin_fmaf(-sm, s, x) <= 0.0f;
+    const bool high = __builtin_fmaf(-sp, s, x) > 0.0f;
+    s = high ? sp : s;
+    return low ? sm : s;
 }
 
 // Reductions over the 64 lanes of a wave (every lane active): DPP moves
@@ -324,6 +322,17 @@ __device__ __forceinline__ int32_t wave_total(int32_t s) {
     v += dpp0<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
     v += dpp0<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
     return (int32_t)v;
+}
+
+// A scalar made to be loaded by here: fields read one by one where each is used
+// are a chain of waits at the start of a pass.
+__device__ __forceinline__ uint64_t loaded(uint64_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ uint32_t loaded(uint32_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
 }
 
 // Issue priority of the calling wave, 0 (lowest) .. 3; p must fold to a
