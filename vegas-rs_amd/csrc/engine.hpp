@@ -235,6 +235,10 @@ struct vg_batch {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev2 = nullptr, ev3 = nullptr;  // the same, for the block after
     hipEvent_t done[2] = {nullptr, nullptr};  // records of a block are on the host
+    // Second stream of a sweep block with passes of several groups, and the
+    // events that part it from the context's stream and join it again.
+    hipStream_t side = nullptr;
+    hipEvent_t parted = nullptr, joined = nullptr;
     double last_ms = 0.0;
     // Per-launch timing of the colour-pass kernels (plain launches only).
     bool timing = false;
@@ -282,6 +286,9 @@ int layout_work(vg_batch* B, int g, uint32_t tile);
 bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid);
 void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s);
 int enqueue_block(vg_batch* B, uint32_t nsw);
+// The batch's second stream, made when its chains lie in several groups.
+int make_side_stream(vg_batch* B);
+void free_side_stream(vg_batch* B);
 int launch_block(vg_batch* B, uint32_t nsw);
 double sums_scale(int spin);
 void observables(const ChainHost& ch, const vg_sweep_sums& r, double* E, double* M);

@@ -245,6 +245,8 @@ int rebuild(vg_server* S) {
             G.partial_cap = cap;
         }
     }
+    const int rc = make_side_stream(&B);
+    if (rc) return rc;
     const uint64_t words = (uint64_t)S->running.size() * Q * 5;
     if (words > S->records_cap) {
         if (S->d_records) quiet(hipFree(S->d_records));
@@ -593,6 +595,7 @@ int vg_server_destroy(vg_server* S) {
         G.partials = nullptr;
         G.arena = nullptr;
     }
+    free_side_stream(&S->B);
     S->B.d_records = nullptr;
     S->B.h_records = nullptr;
     if (S->d_records) quiet(hipFree(S->d_records));
