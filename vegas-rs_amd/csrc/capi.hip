@@ -286,10 +286,23 @@ void launch_ising_init(const Group& G, const ChainDev& d, const ChainDev* dp, hi
 int upload_descriptors(vg_batch* B, int g, int slot) {
     Group& G = B->groups[g];
     if (G.members.empty()) return VG_OK;
+    std::lock_guard<std::mutex> lk(B->send_mu);
+    const size_t bytes = G.host.size() * sizeof(ChainDev);
+    if (G.sent.size() == G.host.size() && !std::memcmp(G.sent.data(), G.host.data(), bytes))
+        return VG_OK;  // the device has them
+    G.sent.clear();
     ChainDev* staging = slot ? G.h_staging2 : G.h_staging;
-    std::memcpy(staging, G.host.data(), G.host.size() * sizeof(ChainDev));
-    VG_HIP(hipMemcpyAsync(G.d_chains, staging, G.host.size() * sizeof(ChainDev),
-                          hipMemcpyHostToDevice, B->ctx->stream));
+    std::memcpy(staging, G.host.data(), bytes);
+    const uint32_t words = (uint32_t)(bytes / 4);
+    static_assert(sizeof(ChainDev) % 4 == 0, "descriptors are whole words");
+    if (bytes <= (64u << 10)) {
+        hipLaunchKernelGGL(vg::copy_words, dim3((words + 255) / 256), dim3(256), 0, B->ctx->stream,
+                           (const uint32_t*)staging, (uint32_t*)G.d_chains, words);
+        VG_HIP(hipGetLastError());
+    } else {
+        VG_HIP(hipMemcpyAsync(G.d_chains, staging, bytes, hipMemcpyHostToDevice, B->ctx->stream));
+    }
+    G.sent = G.host;
     return VG_OK;
 }
 
@@ -549,6 +562,7 @@ int free_batch(vg_batch* B) {
         if (G.draws) quiet(hipFree(G.draws));
     }
     free_side_stream(B);
+    if (B->io) quiet(hipHostFree(B->io));
     if (B->d_records) quiet(hipFree(B->d_records));
     if (B->h_records) quiet(hipHostFree(B->h_records));
     if (B->h_records2) quiet(hipHostFree(B->h_records2));
@@ -662,6 +676,29 @@ bool runs_passes(const Group& G, int g, bool timed) {
     return !G.members.empty() && g != kIsingWolff && (!G.resident || timed);
 }
 
+// The batch's pinned buffer for `bytes` of a chain's state, or null: states of
+// at most kIoBytes go through it and the layout kernel reads or writes host
+// memory itself, for larger ones the caller allocates device memory and copies.
+// us a download and an upload, allocated and copied, and so: 420 Ising sites 29
+// and 23, 15 and 17; 64000 54 and 155, 17 and 20 (with the spins checked in
+// blocks); 2.7 million 254 and 3130, 210 and 310; 1000 Heisenberg spins 38 and
+// 34, 16 and 15.
+void* state_buffer(vg_batch* B, uint64_t bytes) {
+    if (bytes > vg_batch::kIoBytes) return nullptr;
+    if (bytes > B->io_bytes) {
+        if (B->io) quiet(hipHostFree(B->io));
+        B->io = nullptr;
+        B->io_bytes = 0;
+        if (hipHostMalloc(&B->io, bytes, hipHostMallocCoherent) != hipSuccess) {
+            B->io = nullptr;
+            quiet(hipGetLastError());
+            return nullptr;
+        }
+        B->io_bytes = bytes;
+    }
+    return B->io;
+}
+
 int make_side_stream(vg_batch* B) {
     int used = 0;
     for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
@@ -692,11 +729,12 @@ void free_side_stream(vg_batch* B) {
 // sc 64^3 with bcc 40^3 18.6, 12.6 and 17.9, 16.7; a chain of 40^3 of all six
 // kinds 66, 49 and 63, 55.  (Four streams gave no more, and a block with one
 // group of passes loses by it.)
-int enqueue_block(vg_batch* B, uint32_t nsw) {
+int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records) {
     hipStream_t main = B->ctx->stream, of[kNumGroups];
     const uint64_t nrec = (uint64_t)B->chains.size() * nsw * 5u;
-    hipLaunchKernelGGL(vg::zero_i64, dim3((uint32_t)((nrec + 255) / 256)), dim3(256), 0, main,
-                       B->d_records, nrec);
+    if (!B->whole_blocks)
+        hipLaunchKernelGGL(vg::zero_i64, dim3((uint32_t)((nrec + 255) / 256)), dim3(256), 0, main,
+                           records, nrec);
     const bool timed = B->timing && !B->use_graph;  // an event pair per colour pass
     int used = 0;
     for (int g = 0; g < kNumGroups; ++g) {
@@ -709,13 +747,13 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
         Group& G = B->groups[g];
         if (G.members.empty() || runs_passes(G, g, timed)) continue;
         if (g == kIsingWolff) {
-            launch_wolff<0>(G, main, nsw, B->d_records);
-            launch_wolff<1>(G, main, nsw, B->d_records);
-            launch_wolff<2>(G, main, nsw, B->d_records);
+            launch_wolff<0>(G, main, nsw, records);
+            launch_wolff<1>(G, main, nsw, records);
+            launch_wolff<2>(G, main, nsw, records);
         } else if (is_heis_lattice(g)) {
-            launch_heis_resident(G, g, main, nsw, B->d_records);
+            launch_heis_resident(G, g, main, nsw, records);
         } else {
-            launch_resident(G, g, main, nsw, B->d_records);
+            launch_resident(G, g, main, nsw, records);
         }
     }
     if (part) {
@@ -765,11 +803,11 @@ int enqueue_block(vg_batch* B, uint32_t nsw) {
         if (is_ising(g) && !is_graph(g))
             hipLaunchKernelGGL(vg::ising_reduce, grid, dim3(vg::kBlock), 0, st, G.d_chains,
                                (const int32_t*)G.partials, G.total_blocks, colours_of(g), nsw,
-                               B->d_records);
+                               records);
         else
             hipLaunchKernelGGL(vg::heis_reduce, grid, dim3(vg::kBlock), 0, st, G.d_chains,
                                (const int64_t*)G.partials, G.total_blocks, passes_of(G, g), nsw,
-                               B->d_records);
+                               records);
     }
     VG_HIP(hipGetLastError());
     if (part) {
@@ -789,7 +827,7 @@ int block_graph(vg_batch* B, uint32_t nsw, hipGraphExec_t* out) {
         VG_HIP(hipStreamSynchronize(st));
         hipGraph_t graph = nullptr;
         VG_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        int rc = enqueue_block(B, nsw);
+        int rc = enqueue_block(B, nsw, B->d_records);
         hipError_t e = hipStreamEndCapture(st, &graph);
         if (rc != VG_OK) {
             if (graph) quiet(hipGraphDestroy(graph));
@@ -808,8 +846,8 @@ int block_graph(vg_batch* B, uint32_t nsw, hipGraphExec_t* out) {
     return VG_OK;
 }
 
-int launch_block(vg_batch* B, uint32_t nsw) {
-    if (!B->use_graph) return enqueue_block(B, nsw);
+int launch_block(vg_batch* B, uint32_t nsw, int64_t* direct) {
+    if (!B->use_graph) return enqueue_block(B, nsw, direct ? direct : B->d_records);
     hipGraphExec_t exec = nullptr;
     int rc = block_graph(B, nsw, &exec);
     if (rc) return rc;
@@ -921,11 +959,16 @@ int run_impl(vg_batch* B, uint64_t sweeps, vg_sweep_sums* sums, double* energy,
                 B->pass_events_used = 0;
             }
             VG_HIP(hipEventRecord(slot ? B->ev2 : B->ev0, st));
-            int rc = launch_block(B, nsw);
+            // A few records go straight to the host's (coherent) memory; more,
+            // and those of replays, by a copy.
+            int64_t* const to = slot ? B->h_records2 : B->h_records;
+            const bool direct = !B->use_graph && B->whole_blocks && nch * nsw <= 1024;
+            int rc = launch_block(B, nsw, direct ? to : nullptr);
             if (rc) return rc;
             VG_HIP(hipEventRecord(slot ? B->ev3 : B->ev1, st));
-            VG_HIP(hipMemcpyAsync(slot ? B->h_records2 : B->h_records, B->d_records,
-                                  nch * nsw * 5u * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+            if (!direct)
+                VG_HIP(hipMemcpyAsync(to, B->d_records, nch * nsw * 5u * sizeof(int64_t),
+                                      hipMemcpyDeviceToHost, st));
             VG_HIP(hipEventRecord(B->done[slot], st));
             inflight[(head + n_inflight) % 2] = Block{nsw, queued, slot};
             ++n_inflight;
@@ -1254,8 +1297,9 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
     }
     const uint64_t rec_bytes = (uint64_t)n_chains * B->max_block_sweeps * 5u * sizeof(int64_t);
     hipError_t e = hipMalloc(&B->d_records, rec_bytes);
-    if (e == hipSuccess) e = hipHostMalloc(&B->h_records, rec_bytes);
-    if (e == hipSuccess) e = hipHostMalloc(&B->h_records2, rec_bytes);
+    if (e == hipSuccess) e = hipHostMalloc(&B->h_records, rec_bytes, hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostMalloc(&B->h_records2, rec_bytes, hipHostMallocCoherent);
+    B->whole_blocks = true;
     for (hipEvent_t* ev : {&B->ev0, &B->ev1, &B->ev2, &B->ev3, &B->done[0], &B->done[1]})
         if (e == hipSuccess) e = hipEventCreate(ev);
     if (e != hipSuccess) {
@@ -1393,10 +1437,15 @@ int vg_batch_set_ising(vg_batch* batch, uint32_t chain, const int8_t* spins) {
     if (!spins) return fail(VG_ERR_INVALID_ARGUMENT, "null spins");
     ChainHost& ch = batch->chains[chain];
     if (!is_ising(ch.group)) return fail(VG_ERR_INVALID_ARGUMENT, "chain %u is not Ising", chain);
-    for (uint64_t n = 0; n < ch.n_sites; ++n)
-        if (spins[n] != 1 && spins[n] != -1)
-            return fail(VG_ERR_INVALID_ARGUMENT, "spin %llu is %d, not +1 or -1",
-                        (unsigned long long)n, (int)spins[n]);
+    for (uint64_t first = 0; first < ch.n_sites; first += 4096) {  // (blocks: vector compares)
+        const uint64_t end = std::min<uint64_t>(first + 4096, ch.n_sites);
+        uint8_t bad = 0;
+        for (uint64_t n = first; n < end; ++n) bad |= (uint8_t)((spins[n] != 1) & (spins[n] != -1));
+        for (uint64_t n = first; bad && n < end; ++n)
+            if (spins[n] != 1 && spins[n] != -1)
+                return fail(VG_ERR_INVALID_ARGUMENT, "spin %llu is %d, not +1 or -1",
+                            (unsigned long long)n, (int)spins[n]);
+    }
     Group& G = batch->groups[ch.group];
     hipStream_t st = batch->ctx->stream;
     VG_HIP(hipSetDevice(batch->ctx->device));
@@ -1416,6 +1465,17 @@ int vg_batch_set_ising(vg_batch* batch, uint32_t chain, const int8_t* spins) {
         VG_HIP(hipStreamSynchronize(st));
         return VG_OK;
     }
+    std::unique_lock<std::mutex> lk(batch->io_mu);
+    if (void* const io = state_buffer(batch, ch.n_sites)) {
+        std::memcpy(io, spins, ch.n_sites);
+        const uint64_t nb = (uint64_t)G.host[ch.index].ncol * G.host[ch.index].plane;
+        hipLaunchKernelGGL(vg::ising_scatter, dim3((uint32_t)((nb + 255) / 256)), dim3(256), 0, st,
+                           G.d_chains + ch.index, (uint8_t*)G.arena, (const int8_t*)io);
+        VG_HIP(hipGetLastError());
+        VG_HIP(hipStreamSynchronize(st));
+        return VG_OK;
+    }
+    lk.unlock();
     int8_t* tmp = nullptr;
     VG_HIP(hipMalloc(&tmp, ch.n_sites));
     hipError_t e = hipMemcpyAsync(tmp, spins, ch.n_sites, hipMemcpyHostToDevice, st);
@@ -1456,6 +1516,17 @@ int vg_batch_get_ising(vg_batch* batch, uint32_t chain, int8_t* spins) {
         for (uint64_t i = 0; i < ch.n_sites; ++i) spins[i] = v[ch.graph_pos[i]] ? 1 : -1;
         return VG_OK;
     }
+    std::unique_lock<std::mutex> lk(batch->io_mu);
+    if (void* const io = state_buffer(batch, ch.n_sites)) {
+        hipLaunchKernelGGL(vg::ising_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256),
+                           0, st, G.d_chains + ch.index, (const uint8_t*)G.arena, (int8_t*)io,
+                           ch.n_sites);
+        VG_HIP(hipGetLastError());
+        VG_HIP(hipStreamSynchronize(st));
+        std::memcpy(spins, io, ch.n_sites);
+        return VG_OK;
+    }
+    lk.unlock();
     int8_t* tmp = nullptr;
     VG_HIP(hipMalloc(&tmp, ch.n_sites));
     hipLaunchKernelGGL(vg::ising_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256), 0,
@@ -1492,6 +1563,17 @@ int vg_batch_set_heisenberg(vg_batch* batch, uint32_t chain, const double* xyz) 
     }
     double* tmp = nullptr;
     const uint64_t bytes = ch.n_sites * 3 * sizeof(double);
+    std::unique_lock<std::mutex> lk(batch->io_mu);
+    if (void* const io = state_buffer(batch, bytes)) {
+        std::memcpy(io, xyz, bytes);
+        hipLaunchKernelGGL(vg::heis_scatter, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256),
+                           0, st, G.d_chains + ch.index, (float*)G.arena, (const double*)io,
+                           ch.n_sites);
+        VG_HIP(hipGetLastError());
+        VG_HIP(hipStreamSynchronize(st));
+        return VG_OK;
+    }
+    lk.unlock();
     VG_HIP(hipMalloc(&tmp, bytes));
     hipError_t e = hipMemcpyAsync(tmp, xyz, bytes, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {
@@ -1529,6 +1611,17 @@ int vg_batch_get_heisenberg(vg_batch* batch, uint32_t chain, double* xyz) {
     }
     double* tmp = nullptr;
     const uint64_t bytes = ch.n_sites * 3 * sizeof(double);
+    std::unique_lock<std::mutex> lk(batch->io_mu);
+    if (void* const io = state_buffer(batch, bytes)) {
+        hipLaunchKernelGGL(vg::heis_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256), 0,
+                           st, G.d_chains + ch.index, (const float*)G.arena, (double*)io,
+                           ch.n_sites);
+        VG_HIP(hipGetLastError());
+        VG_HIP(hipStreamSynchronize(st));
+        std::memcpy(xyz, io, bytes);
+        return VG_OK;
+    }
+    lk.unlock();
     VG_HIP(hipMalloc(&tmp, bytes));
     hipLaunchKernelGGL(vg::heis_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256), 0,
                        st, G.d_chains + ch.index, (const float*)G.arena, tmp, ch.n_sites);

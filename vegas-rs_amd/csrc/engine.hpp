@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -69,6 +70,7 @@ __global__ void heis_init(const ChainDev*, float*);
 __global__ void heis_scatter(const ChainDev*, float*, const double*, uint64_t);
 __global__ void heis_gather(const ChainDev*, const float*, double*, uint64_t);
 __global__ void zero_i64(int64_t*, uint64_t);
+__global__ void copy_words(const uint32_t*, uint32_t*, uint32_t);
 // Graph chains (an arbitrary exchange matrix): one pass per colour class,
 // args (chains, block -> chain map, arena, partials, colour, sweep, total
 // blocks, passes per sweep); initial states.
@@ -153,6 +155,7 @@ inline uint64_t sites_of(const vg_lattice& L) {
 struct Group {
     std::vector<uint32_t> members;  // batch chain indices
     std::vector<ChainDev> host;     // descriptors, uploaded each sweep block
+    std::vector<ChainDev> sent;     // what d_chains holds
     ChainDev* d_chains = nullptr;
     ChainDev* h_staging = nullptr;  // pinned copy used for the upload
     ChainDev* h_staging2 = nullptr;  // second one, for the block after (batches)
@@ -230,6 +233,16 @@ struct vg_batch {
     int64_t* d_records = nullptr;  // [chain][sweep][5]
     int64_t* h_records = nullptr;  // pinned
     int64_t* h_records2 = nullptr;  // pinned, for the block after (batches)
+    // Every chain runs every sweep of a block, so that the kernels write every
+    // record (not in the job server, whose chains stop within a block).
+    bool whole_blocks = false;
+    // Pinned buffer for the states of small chains, at most kIoBytes
+    static constexpr uint64_t kIoBytes = 4 << 20;
+    void* io = nullptr;
+    uint64_t io_bytes = 0;
+    // Held while io is used, and while descriptors are compared and sent: states
+    // of one batch may be read from several threads.
+    std::mutex io_mu, send_mu;
     bool use_graph = false;
     std::map<uint32_t, hipGraphExec_t> graphs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -285,11 +298,14 @@ int layout_work(vg_batch* B, int g, uint32_t tile);
 // resident at once (the falling wave priorities are used only then).
 bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid);
 void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s);
-int enqueue_block(vg_batch* B, uint32_t nsw);
+// A block of nsw sweeps on the batch's stream, its records to `records`.
+int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records);
 // The batch's second stream, made when its chains lie in several groups.
 int make_side_stream(vg_batch* B);
 void free_side_stream(vg_batch* B);
-int launch_block(vg_batch* B, uint32_t nsw);
+// The same to the device's records, or, where the caller has a pinned buffer
+// for them (direct) and no graph is replayed, straight there.
+int launch_block(vg_batch* B, uint32_t nsw, int64_t* direct = nullptr);
 double sums_scale(int spin);
 void observables(const ChainHost& ch, const vg_sweep_sums& r, double* E, double* M);
 // Geometry and parameters of chain `ch` as member `slot` of group g (sizes,

@@ -206,7 +206,10 @@ __global__ __launch_bounds__(kResidentBlock, Z < 12 && R == 1 ? 8 : 4) void isin
         for (uint32_t s = tid; s < ns; s += kResidentBlock) {
             int64_t* const rec = records + ((uint64_t)C.slot * nsw + done + s) * 5u;
             rec[0] = sums[2u * s + 1u];
+            rec[1] = 0;
+            rec[2] = 0;
             rec[3] = sums[2u * s];
+            rec[4] = 0;
         }
         __syncthreads();
     }

@@ -225,6 +225,7 @@ int rebuild(vg_server* S) {
             if (G.h_staging) quiet(hipHostFree(G.h_staging));
             G.d_chains = nullptr;
             G.h_staging = nullptr;
+            G.sent.clear();
             G.chains_cap = 0;
             const uint32_t cap = (uint32_t)std::max<size_t>(16, G.host.size() * 2);
             VG_HIP(hipMalloc(&G.d_chains, cap * sizeof(ChainDev)));
