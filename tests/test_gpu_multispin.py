@@ -110,3 +110,14 @@ def test_noalloc_packs_and_unpacks_byte_rows(vg, orc, ctx, kind, w, ly, lz, pbc,
     assert np.array_equal(got[:, :4], want[:, :4])
     assert np.array_equal(_from_planes(L, False, out), st)
     assert np.array_equal(out, _to_planes(L, False, st))  # padding zero again
+
+
+@pytest.mark.parametrize("ly,lz", [(512, 512), (512, 514)])  # 1024 and 1028 workgroups of short rows
+def test_sums_of_many_workgroups(vg, orc, ctx, ly, lz):
+    L, d, OL, OM = _chain(vg, orc, "sc", 1, ly, lz, (1, 1, 1), 0.0, 91)
+    st = orc.ising_init(OL, 91)
+    with vg.Batch(ctx, [d]) as b:
+        b.randomize()
+        b.set_thermostat(0, T["sc"])
+        b.set_tile(1)
+        assert np.array_equal(b.run_sums(3)[0], orc.ising_sweeps(OL, OM, 91, 0, 3, st))

@@ -801,7 +801,9 @@ int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records) {
         const hipStream_t st = of[g];
         const dim3 grid((uint32_t)G.members.size(), nsw);
         if (is_ising(g) && !is_graph(g))
-            hipLaunchKernelGGL(vg::ising_reduce, grid, dim3(vg::kBlock), 0, st, G.d_chains,
+            hipLaunchKernelGGL(vg::ising_reduce, grid,
+                               dim3(reduce_block(G.total_blocks / (uint32_t)G.members.size())), 0,
+                               st, G.d_chains,
                                (const int32_t*)G.partials, G.total_blocks, colours_of(g), nsw,
                                records);
         else

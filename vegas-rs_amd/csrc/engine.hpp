@@ -298,6 +298,8 @@ int layout_work(vg_batch* B, int g, uint32_t tile);
 // resident at once (the falling wave priorities are used only then).
 bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid);
 void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint32_t s);
+// Threads of ising_reduce for a group of `blocks` pass workgroups.
+inline uint32_t reduce_block(uint32_t blocks) { return blocks > 1024 ? 1024u : vg::kBlock; }
 // A block of nsw sweeps on the batch's stream, its records to `records`.
 int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records);
 // The batch's second stream, made when its chains lie in several groups.

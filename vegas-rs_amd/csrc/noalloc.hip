@@ -219,7 +219,8 @@ extern "C" int vg_run_sums_noalloc(const vg_chain_desc* desc, double temperature
                                G.d_chains, static_cast<uint8_t*>(spins));
         for (uint32_t s = 0; s < nsw; ++s)
             for (uint32_t c = 0; c < d.ncol; ++c) launch_zmarch_pass(G, g, st, c, s);
-        hipLaunchKernelGGL(vg::ising_reduce, dim3(1, nsw), dim3(vg::kBlock), 0, st, G.d_chains,
+        hipLaunchKernelGGL(vg::ising_reduce, dim3(1, nsw), dim3(reduce_block(G.total_blocks)), 0,
+                           st, G.d_chains,
                            (const int32_t*)G.partials, G.total_blocks, d.ncol, nsw,
                            sums + 5 * done);
         VG_HIP(hipGetLastError());
