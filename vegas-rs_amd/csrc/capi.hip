@@ -380,12 +380,12 @@ bool all_resident(int g, const Group& G, uint32_t tile, uint32_t grid) {
 // Otherwise the cheaper by the measured cost of a sweep, in ns.  Resident: one
 // workgroup a chain, 300 a colour + n / 1.75 for n sites, and a CU's chains one
 // after the other.  Passes: 3200 each in replays + 1 for 64 words of 32
-// positions, all chains together.  us a sweep, resident and passes, for 1, 256,
-// 512 and 1024 chains: sc 8^3 0.9/5.9, 1.3/7.9, 1.8/9.1, 3.2/10.6; sc 16^3
-// 2.4/7.0, 2.8/8.9, 5.4/10.6, 10.4/14.6; sc 20^3 4.9/7.3, 5.3/9.7, 10.2/13.6,
-// 20.3/19.4; sc 64 x 16 x 8 6.3/7.0, 6.7/9.0, 13.0/10.6, 25.9/12.3; bcc 16^3
-// 4.7/7.8, 5.1/9.8, 9.9/12.1, 19.5/16.9; fcc 12^3 4.0/15.9, 4.4/20.0, 8.6/23.4,
-// 16.9/29.0.
+// positions, all chains together.  us a sweep, resident and passes, for 1, 256
+// and 1024 chains: sc 8^3 0.9/5.9, 1.2/7.9, 3.1/10.6; sc 16^3 2.3/7.0, 2.7/8.9,
+// 10.1/14.6; fcc 12^3 3.7/15.8, 4.2/20.0, 15.6/28.9; and where the passes take
+// 1024 chains (the resident times there of a form 4% slower): sc 20^3 4.7/7.3,
+// 5.3/9.7, 20.3/19.4; sc 64 x 16 x 8 6.1/6.9, 6.5/9.0, 25.9/12.3; bcc 16^3
+// 4.6/7.8, 5.1/9.8, 19.5/16.9.
 uint32_t resident_sites(const Group& G, int g) {
     if (G.tile_set || G.tie_cap != 128 || G.host.empty()) return 0;
     const double ncol = colours_of(g);
@@ -590,14 +590,20 @@ void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint3
 // A block of nsw sweeps of an Ising lattice group in the resident kernel.
 void launch_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_t* records) {
     const uint32_t r = G.resident;
-    const auto fn = g == kIsingSc    ? (r == 1   ? vg::ising_resident<6, 1>
-                                        : r == 2 ? vg::ising_resident<6, 2>
-                                                 : vg::ising_resident<6, 4>)
-                    : g == kIsingBcc ? (r == 1   ? vg::ising_resident<8, 1>
-                                        : r == 2 ? vg::ising_resident<8, 2>
-                                                 : vg::ising_resident<8, 4>)
-                                     : (r == 1 ? vg::ising_resident<12, 1>
-                                               : vg::ising_resident<12, 2>);
+    uint64_t most = 0;
+    for (const ChainDev& d : G.host) most = std::max<uint64_t>(most, (uint64_t)d.rows * d.w);
+    const bool solo = most <= 64;
+    const auto fn = g == kIsingSc    ? (solo     ? vg::ising_resident<6, 1, true>
+                                        : r == 1 ? vg::ising_resident<6, 1, false>
+                                        : r == 2 ? vg::ising_resident<6, 2, false>
+                                                 : vg::ising_resident<6, 4, false>)
+                    : g == kIsingBcc ? (solo     ? vg::ising_resident<8, 1, true>
+                                        : r == 1 ? vg::ising_resident<8, 1, false>
+                                        : r == 2 ? vg::ising_resident<8, 2, false>
+                                                 : vg::ising_resident<8, 4, false>)
+                                     : (solo     ? vg::ising_resident<12, 1, true>
+                                        : r == 1 ? vg::ising_resident<12, 1, false>
+                                                 : vg::ising_resident<12, 2, false>);
     hipLaunchKernelGGL(fn, dim3((uint32_t)G.members.size()), dim3(vg::kResidentBlock),
                        vg::kResidentLds, st, G.d_chains, (uint8_t*)G.arena, nsw, vg::kResidentLds,
                        records);

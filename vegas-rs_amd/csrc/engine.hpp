@@ -51,8 +51,8 @@ template <uint32_t A, uint32_t S>
 __global__ void heis_fcc_pass(const ChainDev*, const uint32_t*, float*, int64_t*, uint32_t,
                               uint32_t, uint32_t);
 // Sweep blocks of small chains, one workgroup a chain.  Z: coordination
-// number; R: sites of a colour per lane.
-template <uint32_t Z, uint32_t R>
+// number; R: sites of a colour per lane; SOLO: at most 64, one wave's.
+template <uint32_t Z, uint32_t R, bool SOLO>
 __global__ void ising_resident(const ChainDev*, uint8_t*, uint32_t, uint32_t, int64_t*);
 // Heisenberg: the draws of sweeps s0 .. of a block, and the sweeps on them.
 __global__ void heis_draws(const ChainDev*, uint32_t, uint32_t, uint32_t, float4*);
