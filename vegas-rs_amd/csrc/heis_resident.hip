@@ -96,8 +96,10 @@ __global__ __launch_bounds__(kResidentBlock) void heis_resident(
     __syncthreads();
 
     for (uint32_t s = 0; s < run; ++s) {
-        int32_t s32[4] = {0, 0, 0, 0};
-        int64_t bsum = 0;
+        // A lane's share of a sweep is up to eight sites', and with spins or an
+        // anisotropy axis longer than 1 a site's terms reach 16 * 2^27: summed
+        // in 64 bits (the passes' items hold four sites).
+        int64_t sums4[4] = {0, 0, 0, 0}, bsum = 0;
 #pragma unroll
         for (uint32_t c = 0; c < NCOL; ++c) {
             float4 d[R];
@@ -130,16 +132,20 @@ __global__ __launch_bounds__(kResidentBlock) void heis_resident(
                 const float p[3] = {rnd ? d[r].x : -o[0], rnd ? d[r].y : -o[1],
                                     rnd ? d[r].z : -o[2]};
                 float m[3];
+                int32_t s32[4] = {0, 0, 0, 0};
                 heis_update(C, c > 0, o, h, Z == 12 ? hb : h, d[r].w, p, m, s32, bsum);
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) sums4[k] += s32[k];
                 spin[c * nc + site] = make_float4(m[0], m[1], m[2], 0.0f);
             }
             __syncthreads();
         }
-        // At most R * NCOL sites a lane: within wave_sum_split's bounds.
+        // At most R * NCOL sites a lane, each below 2^31: within wave_sum_split's
+        // bounds.
         int64_t v[5];
         v[0] = wave_sum_split(bsum);
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) v[1 + k] = wave_sum_split(s32[k]);
+        for (uint32_t k = 0; k < 4; ++k) v[1 + k] = wave_sum_split(sums4[k]);
         if ((tid & 63u) == 0u)
 #pragma unroll
             for (uint32_t k = 0; k < 5; ++k)
