@@ -1,0 +1,42 @@
+"""What the engine's host code leaves behind when a HIP call fails part way: on the
+stand-in for the HIP runtime."""
+import pytest
+
+import _fake
+
+
+@pytest.mark.parametrize("failing", [1, 2, 3, 5, 7])
+def test_noalloc_unpacks_after_an_error(failing):
+    """int8 planes packed in place are unpacked again when a launch of the sweeps
+    (3, 5) or their reduction (7) fails, and left alone when the set-up or the
+    packing itself (1, 2) does."""
+    out = _fake.run(f"""
+d = sc(800)
+fake.fake_error_at_launch({failing})
+try:
+    vg.run_sums_noalloc(d, 4.5, 0.0, (0.0, 0.0, 1.0), 0, 2, 4096, 8192, 0)
+except vg.VegasError:
+    print("refused")
+print(launches()[-1])
+""")
+    assert out.startswith("refused")
+    last = out.split()[-1]
+    assert ("noalloc_bitsILb0E" in last) == (failing > 2), last
+    if failing <= 2:
+        assert ("noalloc_setup", "noalloc_bitsILb1E")[failing - 1] in last, last
+
+
+def test_noalloc_enqueues_nothing_after_an_older_error():
+    """An error that an earlier call left behind fails the call before it has
+    touched the caller's planes."""
+    out = _fake.run("""
+fake.fake_fail(b"hipMalloc", 1)
+p = C.c_void_p()
+assert fake.hipMalloc(C.byref(p), C.c_size_t(16)) != 0
+try:
+    vg.run_sums_noalloc(sc(800), 4.5, 0.0, (0.0, 0.0, 1.0), 0, 2, 4096, 8192, 0)
+except vg.VegasError:
+    print("refused")
+print(len(launches()))
+""")
+    assert out.split() == ["refused", "0"]

@@ -209,27 +209,37 @@ extern "C" int vg_run_sums_noalloc(const vg_chain_desc* desc, double temperature
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint64_t rows_per_block = (vg::kBlock / 64u) * (d.segs < 64u ? 64u / d.segs : 1u);
     const dim3 convert((uint32_t)(((uint64_t)d.ncol * d.rows + rows_per_block - 1) / rows_per_block));
-    for (uint64_t done = 0; done < sweeps;) {
+    // An error from before the call, and one of the set-up or the packing: the
+    // caller's planes are as they were.  After that a failure still unpacks them.
+    VG_HIP(hipGetLastError());
+    hipError_t e = hipSuccess;
+    for (uint64_t done = 0; done < sweeps && e == hipSuccess;) {
         const uint32_t nsw = (uint32_t)std::min<uint64_t>(chunk, sweeps - done);
         d.sweep0 = sweep0 + done;
         hipLaunchKernelGGL(vg::noalloc_setup, dim3((d.nblocks + 255) / 256), dim3(256), 0, st, d,
                            G.d_chains, G.d_block_chain, d.nblocks);
-        if (ch.byte_planes && done == 0)
+        if (done == 0) VG_HIP(hipGetLastError());
+        if (ch.byte_planes && done == 0) {
             hipLaunchKernelGGL(vg::noalloc_bits<true>, convert, dim3(vg::kBlock), 0, st,
                                G.d_chains, static_cast<uint8_t*>(spins));
+            VG_HIP(hipGetLastError());
+        }
         for (uint32_t s = 0; s < nsw; ++s)
             for (uint32_t c = 0; c < d.ncol; ++c) launch_zmarch_pass(G, g, st, c, s);
         hipLaunchKernelGGL(vg::ising_reduce, dim3(1, nsw), dim3(reduce_block(G.total_blocks)), 0,
                            st, G.d_chains,
                            (const int32_t*)G.partials, G.total_blocks, d.ncol, nsw,
                            sums + 5 * done);
-        VG_HIP(hipGetLastError());
+        e = hipGetLastError();
         done += nsw;
     }
     if (ch.byte_planes) {
         hipLaunchKernelGGL(vg::noalloc_bits<false>, convert, dim3(vg::kBlock), 0, st, G.d_chains,
                            static_cast<uint8_t*>(spins));
-        VG_HIP(hipGetLastError());
+        if (e == hipSuccess) e = hipGetLastError();
     }
+    if (e != hipSuccess)
+        return fail(e == hipErrorOutOfMemory ? VG_ERR_OUT_OF_MEMORY : VG_ERR_DEVICE,
+                    "launching the sweeps: %s", hipGetErrorString(e));
     return VG_OK;
 }
