@@ -290,17 +290,21 @@ int vg_batch_pass_stats(const vg_batch* batch, int32_t spin, double* total_ms, u
 /*     x = i on bcc and fcc; w = lx / 2 (sc) or lx positions.  int8: one  */
 /*     byte per position, 1 = Up, 0 = Down, pitch = round_up(w, 64).      */
 /*     Bit-packed: bit (i & 7) of byte i >> 3, pitch = round_up(2 *       */
-/*     ceil(w / 16), 16).  Padding bytes zero.  Updated in place; while    */
-/*     the call's sweeps run, int8 rows hold their bits in their first w/8 */
-/*     bytes.                                                              */
+/*     ceil(w / 16), 16).  Padding bytes zero.  Updated in place; until    */
+/*     the call's last sweep has run, int8 planes hold the old spins or, of */
+/*     chains past some 300 million sites, each row's bits in its first     */
+/*     eighth.  After an error they are bytes too: as they were, or with    */
+/*     the sweeps that were launched.                                       */
 /*   sums: sweeps * 5 int64, per sweep {bond, 0, 0, mag, 0} as in          */
 /*     vg_sweep_sums (the batch path reports N as the fifth).             */
 /*   sweep0: the chain's sweep counter before the first sweep (Philox).   */
 /* The thermostat follows vg_batch_set_thermostat.  Descriptor, block map */
-/* and pass partials live in a 16 MiB device array that each GPU holds    */
-/* until the process ends.  A sweep's partials take colours x workgroups  */
-/* x 32 bytes (N / 512 bytes on sc, cells / 128 on fcc); a chain whose    */
-/* partials for one sweep do not fit is refused (VG_ERR_INVALID_ARGUMENT):*/
+/* and pass partials live in 16 MiB, and the bits of int8 planes in 40    */
+/* more, of a device array that each GPU holds until the process ends.    */
+/* A sweep is charged colours x workgroups x 32 bytes of partials, for    */
+/* workgroups of 256 items of four planes (N / 512 bytes on sc, cells /   */
+/* 128 on fcc), whatever the tile that it runs with; a chain for which    */
+/* that does not fit is refused (VG_ERR_INVALID_ARGUMENT):                */
 /* every sc and bcc chain a batch accepts fits, fcc up to about 2 x 10^9  */
 /* cells.                                                                 */
 /* Calls on one GPU share that array: calls that overlap on one GPU race */

@@ -40,3 +40,24 @@ except vg.VegasError:
 print(len(launches()))
 """)
     assert out.split() == ["refused", "0"]
+
+
+@pytest.mark.parametrize("sweeps,failing", [(2, 1), (2, 3), (2, 6), (5000, 3), (5000, 8194)])
+def test_noalloc_writes_bytes_after_an_error(sweeps, failing):
+    """The same of a chain whose bits are held apart: its bytes are written after
+    a failure behind the packing, in the first chunk of sweeps (4096) and later."""
+    out = _fake.run(f"""
+fake.fake_error_at_launch({failing})
+try:
+    vg.run_sums_noalloc(sc(32), 4.5, 0.0, (0.0, 0.0, 1.0), 0, {sweeps}, 4096, 8192, 0)
+except vg.VegasError:
+    print("refused")
+l = launches()
+print(len(l), l[-1])
+""")
+    assert out.startswith("refused")
+    count, last = out.split()[1:]
+    if failing == 1:
+        assert count == "1"
+    else:
+        assert "noalloc_finish" in last, last

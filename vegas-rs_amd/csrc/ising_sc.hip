@@ -209,71 +209,12 @@ VG_SC_PASS(4, kPeriodic)
 VG_SC_PASS(8, kPeriodic)
 #undef VG_SC_PASS
 
-// Sums the pass partials of each (chain, sweep) over its ncol colour passes
-// into its record: record = {bond, 0, 0, mag, 0} (int64).  A pass adds the
-// bonds to lower colours only (none in colour 0), so each bond counts once.
 // grid = (chains, sweeps).
 __global__ __launch_bounds__(1024) void ising_reduce(const ChainDev* __restrict__ chains,
                                                     const int32_t* __restrict__ partials,
                                                     uint32_t total_blocks, uint32_t ncol,
                                                     uint32_t nsw, int64_t* __restrict__ records) {
-    __shared__ int64_t red[2][16];
-    const uint32_t block = blockDim.x;  // 256, or 1024 where a chain has many workgroups
-    const ChainDev& C = chains[blockIdx.x];
-    const uint32_t s = blockIdx.y;
-    if (s >= C.limit) return;  // this chain ran fewer sweeps in the block
-    int64_t mm = 0, bb = 0;
-    // Four workgroups' partials at a time, in 16-byte loads, by 1024 threads where
-    // there are many: one workgroup sums a chain's sweep, and with 256 threads and
-    // eight loads one after the other that was 22 us for sc 1024^3, now 8.8.
-    constexpr uint32_t kAhead = 4;
-    static_assert(kWaves == 4, "a workgroup's partials are two 16-byte words");
-    for (uint32_t c = 0; c < ncol; ++c) {
-        const int4* const from = reinterpret_cast<const int4*>(partials) +
-                                 ((uint64_t)(s * ncol + c) * total_blocks + C.block0) * 2u;
-        for (uint32_t k = threadIdx.x; k < C.nblocks; k += kAhead * block) {
-            int4 v[kAhead][2];
-#pragma unroll
-            for (uint32_t j = 0; j < kAhead; ++j) {
-                const uint32_t at = min(k + j * block, C.nblocks - 1u);
-                v[j][0] = from[2u * at];
-                v[j][1] = from[2u * at + 1u];
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < kAhead; ++j) {
-                if (k + j * block >= C.nblocks) break;
-#pragma unroll
-                for (uint32_t h = 0; h < 2; ++h) {
-                    mm += (int64_t)v[j][h].x + v[j][h].z;
-                    bb += (int64_t)v[j][h].y + v[j][h].w;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        mm += __shfl_xor(mm, o, 64);
-        bb += __shfl_xor(bb, o, 64);
-    }
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        red[0][wave] = mm;
-        red[1][wave] = bb;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t m = 0, bo = 0;
-        for (uint32_t k = 0; k < block / 64; ++k) {
-            m += red[0][k];
-            bo += red[1][k];
-        }
-        int64_t* r = records + ((uint64_t)C.slot * nsw + s) * 5u;
-        r[0] = bo;
-        r[1] = 0;
-        r[2] = 0;
-        r[3] = m;
-        r[4] = 0;
-    }
+    reduce_sweep(chains[blockIdx.x], partials, total_blocks, ncol, nsw, blockIdx.y, records);
 }
 
 }  // namespace vg

@@ -697,4 +697,69 @@ __device__ __forceinline__ void align_all(const uint32_t u[4], uint32_t o, uint3
     }
 }
 
+// Sums the pass partials of one chain's sweep s over its ncol colour passes
+// into its record: record = {bond, 0, 0, mag, 0} (int64).  A pass adds the
+// bonds to lower colours only (none in colour 0), so each bond counts once.
+// One workgroup's work, of 256 or 1024 threads.
+__device__ __forceinline__ void reduce_sweep(const ChainDev& C,
+                                             const int32_t* __restrict__ partials,
+                                             uint32_t total_blocks, uint32_t ncol, uint32_t nsw,
+                                             uint32_t s, int64_t* __restrict__ records) {
+    __shared__ int64_t red[2][16];
+    const uint32_t block = blockDim.x;  // 256, or 1024 where a chain has many workgroups
+    if (s >= C.limit) return;  // this chain ran fewer sweeps in the block
+    int64_t mm = 0, bb = 0;
+    // Four workgroups' partials at a time, in 16-byte loads, by 1024 threads where
+    // there are many: one workgroup sums a chain's sweep, and with 256 threads and
+    // eight loads one after the other that was 22 us for sc 1024^3, now 8.8.
+    constexpr uint32_t kAhead = 4;
+    static_assert(kWaves == 4, "a workgroup's partials are two 16-byte words");
+    for (uint32_t c = 0; c < ncol; ++c) {
+        const int4* const from = reinterpret_cast<const int4*>(partials) +
+                                 ((uint64_t)(s * ncol + c) * total_blocks + C.block0) * 2u;
+        for (uint32_t k = threadIdx.x; k < C.nblocks; k += kAhead * block) {
+            int4 v[kAhead][2];
+#pragma unroll
+            for (uint32_t j = 0; j < kAhead; ++j) {
+                const uint32_t at = min(k + j * block, C.nblocks - 1u);
+                v[j][0] = from[2u * at];
+                v[j][1] = from[2u * at + 1u];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kAhead; ++j) {
+                if (k + j * block >= C.nblocks) break;
+#pragma unroll
+                for (uint32_t h = 0; h < 2; ++h) {
+                    mm += (int64_t)v[j][h].x + v[j][h].z;
+                    bb += (int64_t)v[j][h].y + v[j][h].w;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        mm += __shfl_xor(mm, o, 64);
+        bb += __shfl_xor(bb, o, 64);
+    }
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+        red[0][wave] = mm;
+        red[1][wave] = bb;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t m = 0, bo = 0;
+        for (uint32_t k = 0; k < block / 64; ++k) {
+            m += red[0][k];
+            bo += red[1][k];
+        }
+        int64_t* r = records + ((uint64_t)C.slot * nsw + s) * 5u;
+        r[0] = bo;
+        r[1] = 0;
+        r[2] = 0;
+        r[3] = m;
+        r[4] = 0;
+    }
+}
+
 }  // namespace vg
