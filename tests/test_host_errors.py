@@ -61,3 +61,40 @@ print(len(l), l[-1])
         assert count == "1"
     else:
         assert "noalloc_finish" in last, last
+
+
+TWO_GROUPS = """
+b = vg.Batch(ctx, [sc(64), sc(64, spin=vg.HEISENBERG)])
+b.run(1)
+fake.fake_clear()
+"""
+
+
+@pytest.mark.parametrize("how,last", [
+    ("fake_error_at_launch(3)", "wait"), ("fake_error_at_launch(7)", "wait"),
+    ('fake_fail(b"hipEventRecord", 3)', "sync"), ('fake_fail(b"hipStreamWaitEvent", 2)', "sync"),
+])
+def test_side_stream_joins_after_an_error(how, last):
+    """A block of two groups whose launch fails: whatever the second stream was
+    given lies before the next work of the main stream, by its event or, if that
+    fails, by waiting."""
+    out = _fake.run(TWO_GROUPS + f"""
+fake.{how}
+try:
+    b.run(1)
+except vg.VegasError:
+    print("refused")
+print(";".join(log()))
+""")
+    refused, lines = out.strip().split("\n")
+    assert refused == "refused"
+    lines = lines.split(";")
+    streams = [l.split()[l.split().index("stream") + 1] for l in lines if l.startswith("launch")]
+    main = streams[0]
+    side = next(s for s in streams if s != main)
+    tail = lines[max(i for i, l in enumerate(lines) if f"stream {side} " in l and "launch" in l) + 1:]
+    if last == "wait":
+        assert any(l.startswith("record event") and l.endswith(f"stream {side}") for l in tail), tail
+        assert any(l.startswith(f"wait stream {main} ") for l in tail), tail
+    else:
+        assert f"sync stream {side}" in tail, tail

@@ -817,11 +817,16 @@ int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records) {
                                (const int64_t*)G.partials, G.total_blocks, passes_of(G, g), nsw,
                                records);
     }
-    VG_HIP(hipGetLastError());
-    if (part) {
-        VG_HIP(hipEventRecord(B->joined, B->side));
-        VG_HIP(hipStreamWaitEvent(main, B->joined, 0));
+    hipError_t e = hipGetLastError();
+    if (part) {  // after an error too: what follows on the main stream waits for the side's
+        hipError_t j = hipEventRecord(B->joined, B->side);
+        if (j == hipSuccess) j = hipStreamWaitEvent(main, B->joined, 0);
+        if (j != hipSuccess) quiet(hipStreamSynchronize(B->side));
+        if (e == hipSuccess) e = j;
     }
+    if (e != hipSuccess)
+        return fail(e == hipErrorOutOfMemory ? VG_ERR_OUT_OF_MEMORY : VG_ERR_DEVICE,
+                    "launching a sweep block: %s", hipGetErrorString(e));
     return VG_OK;
 }
 
