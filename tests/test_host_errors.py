@@ -98,3 +98,27 @@ print(";".join(log()))
         assert any(l.startswith(f"wait stream {main} ") for l in tail), tail
     else:
         assert f"sync stream {side}" in tail, tail
+
+
+@pytest.mark.parametrize("spin,call", [
+    ("ISING", "set_ising(0, [1] * 64)"), ("ISING", "get_ising(0)"),
+    ("HEISENBERG", "set_heisenberg(0, [[0.0, 0.0, 1.0]] * 64)"), ("HEISENBERG", "get_heisenberg(0)"),
+])
+def test_state_buffer_is_waited_for_after_an_error(spin, call):
+    """A kernel that reads or writes the pinned state buffer has ended before the
+    call returns an error: the next call writes there."""
+    out = _fake.run(f"""
+b = vg.Batch(ctx, [sc(4, spin=vg.{spin})])
+fake.fake_clear()
+fake.fake_error_at_launch(1)
+try:
+    b.{call}
+except vg.VegasError:
+    print("refused")
+print(";".join(log()))
+""")
+    refused, lines = out.strip().split("\n")
+    assert refused == "refused"
+    lines = lines.split(";")
+    assert any(l.startswith("launch") for l in lines), lines
+    assert lines[-1].startswith("sync stream"), lines

@@ -705,6 +705,14 @@ void* state_buffer(vg_batch* B, uint64_t bytes) {
     return B->io;
 }
 
+// The end of a call that gave a kernel the buffer: after an error too the kernel is
+// through with it before the next call writes there.
+int state_done(hipStream_t st) {
+    const hipError_t e = hipGetLastError(), w = hipStreamSynchronize(st);
+    if (e == hipSuccess && w == hipSuccess) return VG_OK;
+    return fail(VG_ERR_DEVICE, "moving a state: %s", hipGetErrorString(e != hipSuccess ? e : w));
+}
+
 int make_side_stream(vg_batch* B) {
     int used = 0;
     for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
@@ -1484,9 +1492,7 @@ int vg_batch_set_ising(vg_batch* batch, uint32_t chain, const int8_t* spins) {
         const uint64_t nb = (uint64_t)G.host[ch.index].ncol * G.host[ch.index].plane;
         hipLaunchKernelGGL(vg::ising_scatter, dim3((uint32_t)((nb + 255) / 256)), dim3(256), 0, st,
                            G.d_chains + ch.index, (uint8_t*)G.arena, (const int8_t*)io);
-        VG_HIP(hipGetLastError());
-        VG_HIP(hipStreamSynchronize(st));
-        return VG_OK;
+        return state_done(st);
     }
     lk.unlock();
     int8_t* tmp = nullptr;
@@ -1534,8 +1540,8 @@ int vg_batch_get_ising(vg_batch* batch, uint32_t chain, int8_t* spins) {
         hipLaunchKernelGGL(vg::ising_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256),
                            0, st, G.d_chains + ch.index, (const uint8_t*)G.arena, (int8_t*)io,
                            ch.n_sites);
-        VG_HIP(hipGetLastError());
-        VG_HIP(hipStreamSynchronize(st));
+        rc = state_done(st);
+        if (rc) return rc;
         std::memcpy(spins, io, ch.n_sites);
         return VG_OK;
     }
@@ -1582,9 +1588,7 @@ int vg_batch_set_heisenberg(vg_batch* batch, uint32_t chain, const double* xyz) 
         hipLaunchKernelGGL(vg::heis_scatter, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256),
                            0, st, G.d_chains + ch.index, (float*)G.arena, (const double*)io,
                            ch.n_sites);
-        VG_HIP(hipGetLastError());
-        VG_HIP(hipStreamSynchronize(st));
-        return VG_OK;
+        return state_done(st);
     }
     lk.unlock();
     VG_HIP(hipMalloc(&tmp, bytes));
@@ -1629,8 +1633,8 @@ int vg_batch_get_heisenberg(vg_batch* batch, uint32_t chain, double* xyz) {
         hipLaunchKernelGGL(vg::heis_gather, dim3((uint32_t)((ch.n_sites + 255) / 256)), dim3(256), 0,
                            st, G.d_chains + ch.index, (const float*)G.arena, (double*)io,
                            ch.n_sites);
-        VG_HIP(hipGetLastError());
-        VG_HIP(hipStreamSynchronize(st));
+        rc = state_done(st);
+        if (rc) return rc;
         std::memcpy(xyz, io, bytes);
         return VG_OK;
     }
