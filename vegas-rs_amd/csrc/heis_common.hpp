@@ -97,9 +97,9 @@ __device__ __forceinline__ void sphere_point(const Try& a, float p[3]) {
     p[2] = ff(-2.0f, a.q, 1.0f);  // 2q is exact: the same rounding as fs(1, 2q)
 }
 
-// What a colour pass's wave needs of its chain, loaded in one batch; workgroups
-// past the work and chains that run fewer sweeps in this block are not sent away
-// before it.
+// What a colour pass's wave needs of its chain, loaded in one batch: workgroups
+// past the work and of chains that run fewer sweeps in this block are sent away
+// behind it, by `run`, not field by field before it.
 struct HeisHead {
     uint64_t off[4], plane, seed, t;
     uint32_t segs, ly, lz, w, pitch, pbc, proposal;
@@ -422,7 +422,7 @@ __device__ __forceinline__ void heis_partials(const int32_t s32[4], int64_t bsum
 __device__ __forceinline__ void heis_partials_sites(const int32_t s32[4], int64_t bsum,
                                                     int64_t* __restrict__ partials,
                                                     uint32_t colour, uint32_t ncol, uint32_t s,
-                                                    uint32_t total_blocks, uint32_t b, bool run) {
+                                                    uint32_t total_blocks, uint32_t b) {
     constexpr uint32_t kW = kBlock / 64;
     __shared__ int32_t red[4][kBlock];
     __shared__ int64_t redb[kBlock];
@@ -436,13 +436,13 @@ __device__ __forceinline__ void heis_partials_sites(const int32_t s32[4], int64_
 #pragma unroll
     for (uint32_t k = 0; k < kW; ++k) v += red[wave][64u * k + lane];
     v = wave_sum_split(v);
-    if (lane == 0 && run) out[1u + wave] = v;
+    if (lane == 0) out[1u + wave] = v;
     if (wave == 0) {
         v = 0;
 #pragma unroll
         for (uint32_t k = 0; k < kW; ++k) v += redb[64u * k + lane];
         v = wave_sum_split(v);
-        if (lane == 0 && run) out[0] = v;
+        if (lane == 0) out[0] = v;
     }
 }
 

@@ -29,6 +29,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
     const uint32_t b = xcd_block(blockIdx.x, grid);
     const ChainDev& C = chains[block_chain[min(b, total_blocks - 1u)]];
     const HeisHead H = heis_head(C, b, total_blocks, s);
+    if (!H.run) return;  // uniform: the workgroup belongs to one chain
     const bool active = H.active, rnd = H.proposal != 0;
     const uint64_t t = H.t;
     int32_t s32[4] = {0, 0, 0, 0};     // mx, my, mz, axis2 of the lane's sites
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void h
         }
     }
 
-    heis_partials_sites(s32, bsum, partials, A, 4u, s, total_blocks, b, H.run);
+    heis_partials_sites(s32, bsum, partials, A, 4u, s, total_blocks, b);
 }
 
 #define VG_HEIS_FCC(A, S)                                                                \
