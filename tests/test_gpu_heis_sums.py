@@ -38,3 +38,23 @@ def test_long_anisotropy_axis(vg, orc, ctx, kind, dims, axis):
 def test_long_spins(vg, orc, ctx, proposal):
     """Length 2.7: two neighbours keep a site's bonds below 16."""
     _run(vg, orc, ctx, "sc", (8192, 1, 1), (1, 0, 0), (0.0, 0.0, 1.0), 2.7, proposal)
+
+
+def test_long_spins_under_replays(vg, orc, ctx):
+    """A captured block follows the lengths of the spins: unit, long, unit again."""
+    L = vg.lattice(vg.SC, 8192, 1, 1, pbc=(True, False, False))
+    d = vg.chain(L, vg.HEISENBERG, vg.FLIP, vg.hamiltonian(exchange=1.0), 11)
+    OL = orc.lattice("sc", 8192, 1, 1, pbc=(1, 0, 0))
+    OM = orc.model(spin="heisenberg", terms=("exchange",), temperature=0.2)
+    with vg.Batch(ctx, [d]) as b:
+        b.set_graph(True)
+        b.set_thermostat(0, 0.2)
+        for length in (1.0, 2.7, 1.0):
+            b.randomize()
+            st = orc.heis_init(OL, 11)
+            if length != 1.0:
+                st = np.tile(np.array([0.0, 0.0, length], dtype=np.float32), (8192, 1))
+                b.set_heisenberg(0, st.astype(np.float64))
+            for k in range(2):
+                assert np.array_equal(b.run_sums(3)[0],
+                                      orc.heis_sweeps(OL, OM, 11, 3 * k, 3, st)), (length, k)

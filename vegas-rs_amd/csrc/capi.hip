@@ -407,6 +407,22 @@ uint32_t resident_sites(const Group& G, int g) {
 
 bool is_heis_lattice(int g) { return g == kHeisSc || g == kHeisBcc || g == kHeisFcc; }
 
+template <uint32_t Z>
+auto heis_resident_of(uint32_t r, bool wide) {
+    if constexpr (Z == 12)
+        return r == 1 ? (wide ? vg::heis_resident<12, 1, true> : vg::heis_resident<12, 1, false>)
+                      : (wide ? vg::heis_resident<12, 2, true> : vg::heis_resident<12, 2, false>);
+    else
+        return r == 1   ? (wide ? vg::heis_resident<Z, 1, true> : vg::heis_resident<Z, 1, false>)
+               : r == 2 ? (wide ? vg::heis_resident<Z, 2, true> : vg::heis_resident<Z, 2, false>)
+                        : (wide ? vg::heis_resident<Z, 4, true> : vg::heis_resident<Z, 4, false>);
+}
+auto heis_resident_fn(int g, uint32_t r, bool wide) {
+    return g == kHeisSc    ? heis_resident_of<6>(r, wide)
+           : g == kHeisBcc ? heis_resident_of<8>(r, wide)
+                           : heis_resident_of<12>(r, wide);
+}
+
 // The same for a Heisenberg lattice group, with its workspace for the draws of
 // at most max_sweeps sweeps and 64 MiB.
 //
@@ -447,13 +463,10 @@ int setup_heis_resident(Group& G, int g, uint32_t max_sweeps) {
     const double passes = std::max((random ? 6500.0 : 4600.0) * ncol,
                                    (random ? 5000.0 : 3800.0) * ncol + slope * (double)padded);
     if (resident > passes) return VG_OK;
-    const void* fns[] = {(const void*)&vg::heis_resident<6, 1>, (const void*)&vg::heis_resident<6, 2>,
-                         (const void*)&vg::heis_resident<6, 4>, (const void*)&vg::heis_resident<8, 1>,
-                         (const void*)&vg::heis_resident<8, 2>, (const void*)&vg::heis_resident<8, 4>,
-                         (const void*)&vg::heis_resident<12, 1>,
-                         (const void*)&vg::heis_resident<12, 2>};
-    for (const void* fn : fns)  // past the 64 KiB default
-        VG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
+    const uint32_t r = nc <= vg::kResidentBlock ? 1u : (nc <= 2 * vg::kResidentBlock ? 2u : 4u);
+    for (bool wide : {false, true})  // past the 64 KiB default
+        VG_HIP(hipFuncSetAttribute((const void*)heis_resident_fn(g, r, wide),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
     if (hipMalloc(&G.draws, per_sweep * held) != hipSuccess) {
         G.draws = nullptr;  // no room for the workspace: passes
         quiet(hipGetLastError());
@@ -461,8 +474,27 @@ int setup_heis_resident(Group& G, int g, uint32_t max_sweeps) {
     }
     G.draw_sweeps = held;
     G.draw_stride = (uint32_t)n;
-    G.resident = nc <= vg::kResidentBlock ? 1u : (nc <= 2 * vg::kResidentBlock ? 2u : 4u);
+    G.resident = r;
     return VG_OK;
+}
+
+// Whether a site's magnetisation or squared axis component may reach 2 (with a
+// margin for fp32): what the resident kernel's sums must be wide for.
+bool long_terms(const ChainHost& ch) {
+    const double* const a = ch.desc.hamiltonian.anisotropy_axis;
+    const double a2 = std::max(1.0, a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
+    return !(std::max(1.0, ch.spin2) * a2 < 1.99);
+}
+
+// Sets Group::wide of a resident Heisenberg group; captured graphs hold the kernel.
+void refresh_wide(vg_batch* B, Group& G) {
+    if (!G.draws) return;
+    bool wide = false;
+    for (uint32_t i : G.members) wide = wide || long_terms(B->chains[i]);
+    if (wide == G.wide) return;
+    G.wide = wide;
+    for (auto& kv : B->graphs) quiet(hipGraphExecDestroy(kv.second));
+    B->graphs.clear();
 }
 
 // Positions per work item of a Heisenberg lattice group: one while the waves
@@ -612,16 +644,8 @@ void launch_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_
 // The same of a Heisenberg lattice group: draws, then the sweeps on them, as
 // many at a time as the workspace holds.
 void launch_heis_resident(const Group& G, int g, hipStream_t st, uint32_t nsw, int64_t* records) {
-    const uint32_t r = G.resident, z = g == kHeisSc ? 6u : (g == kHeisBcc ? 8u : 12u);
-    const auto fn = g == kHeisSc    ? (r == 1   ? vg::heis_resident<6, 1>
-                                       : r == 2 ? vg::heis_resident<6, 2>
-                                                : vg::heis_resident<6, 4>)
-                    : g == kHeisBcc ? (r == 1   ? vg::heis_resident<8, 1>
-                                       : r == 2 ? vg::heis_resident<8, 2>
-                                                : vg::heis_resident<8, 4>)
-                                    : (r == 1 ? vg::heis_resident<12, 1>
-                                              : vg::heis_resident<12, 2>);
-    const uint32_t ncol = z == 12 ? 4u : 2u, nc = G.draw_stride / ncol;
+    const auto fn = heis_resident_fn(g, G.resident, G.wide);
+    const uint32_t ncol = colours_of(g), nc = G.draw_stride / ncol;
     const uint32_t block = std::min<uint32_t>((nc + 63u) / 64u * 64u, vg::kResidentBlock);
     const uint32_t chains = (uint32_t)G.members.size();
     for (uint32_t s0 = 0; s0 < nsw; s0 += G.draw_sweeps) {
@@ -1300,6 +1324,7 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
                 free_batch(B);
                 return rc;
             }
+            refresh_wide(B, G);
         }
         if (is_zmarch(g)) {
             int rc = layout_work(B, g, default_tile(G.host.data(), G.host.size()));
@@ -1449,6 +1474,8 @@ int vg_batch_randomize(vg_batch* batch) {
     }
     VG_HIP(hipGetLastError());
     VG_HIP(hipStreamSynchronize(st));
+    for (ChainHost& ch : batch->chains) ch.spin2 = 1.0;
+    for (Group& G : batch->groups) refresh_wide(batch, G);
     return VG_OK;
 }
 
@@ -1579,6 +1606,14 @@ int vg_batch_set_heisenberg(vg_batch* batch, uint32_t chain, const double* xyz) 
                               v.size() * sizeof(float), hipMemcpyHostToDevice, st));
         VG_HIP(hipStreamSynchronize(st));
         return VG_OK;
+    }
+    if (G.draws) {
+        for (uint64_t i = 0; i < ch.n_sites; ++i) {
+            const double* const s = xyz + 3 * i;
+            const double s2 = s[0] * s[0] + s[1] * s[1] + s[2] * s[2];
+            ch.spin2 = std::max(ch.spin2, std::isnan(s2) ? HUGE_VAL : s2);
+        }
+        refresh_wide(batch, G);
     }
     double* tmp = nullptr;
     const uint64_t bytes = ch.n_sites * 3 * sizeof(double);

@@ -56,7 +56,7 @@ template <uint32_t Z, uint32_t R, bool SOLO>
 __global__ void ising_resident(const ChainDev*, uint8_t*, uint32_t, uint32_t, int64_t*);
 // Heisenberg: the draws of sweeps s0 .. of a block, and the sweeps on them.
 __global__ void heis_draws(const ChainDev*, uint32_t, uint32_t, uint32_t, float4*);
-template <uint32_t Z, uint32_t R>
+template <uint32_t Z, uint32_t R, bool WIDE>
 __global__ void heis_resident(const ChainDev*, float*, uint32_t, uint32_t, uint32_t,
                               const float4*, uint32_t, int64_t*);
 // Wolff steps of the chains of one lattice kind (0 sc, 1 bcc, 2 fcc).
@@ -190,6 +190,7 @@ struct Group {
     // sweeps, draw_stride of them a sweep and chain (the largest chain's sites)
     float4* draws = nullptr;
     uint32_t draw_sweeps = 0, draw_stride = 0;
+    bool wide = false;  // resident Heisenberg chains: a member's terms may pass 2 (long_terms)
     // Capacities of d_chains / h_staging (descriptors) and of partials
     // (bytes), for batches whose membership changes (the job server).
     uint32_t chains_cap = 0;
@@ -206,6 +207,9 @@ struct ChainHost {
     double field_dir[3] = {0.0, 0.0, 1.0};
     int group = 0;
     uint32_t index = 0;  // index in its group
+    // Chains of resident Heisenberg groups: the largest squared length of a spin
+    // set by the caller since the last random state (drawn spins have length 1)
+    double spin2 = 1.0;
     // The planes are the caller's, with rows of one byte per site (the
     // allocation-free entry point, which keeps a row's bits at its start).
     bool byte_planes = false;
