@@ -177,7 +177,10 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t* e) { return handle(e); }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return handle(e); }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    if (fails("hipEventCreateWithFlags")) return bad(hipErrorOutOfMemory);
+    return handle(e);
+}
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     if (fails("hipEventRecord")) return bad(hipErrorUnknown);

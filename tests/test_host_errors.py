@@ -122,3 +122,23 @@ print(";".join(log()))
     lines = lines.split(";")
     assert any(l.startswith("launch") for l in lines), lines
     assert lines[-1].startswith("sync stream"), lines
+
+
+@pytest.mark.parametrize("failing,of_server", [("hipStreamCreateWithFlags", 2),
+                                               ("hipEventCreateWithFlags", 1)])
+def test_one_stream_where_a_second_cannot_be_made(failing, of_server):
+    """Batches and servers with chains of two groups run on one stream then."""
+    out = _fake.run(f"""
+fake.fake_fail(b"{failing}", 1)
+b = vg.Batch(ctx, [sc(64), sc(64, spin=vg.HEISENBERG)])
+b.run(1)
+s1 = {{l.split()[3] for l in log() if l.startswith("launch")}}
+fake.fake_fail(b"{failing}", {of_server})  # (the server's first stream is made before)
+s = vg.Server(ctx, quantum_sweeps=10)
+fake.fake_clear()
+ids = [s.submit(sc(64, spin=k), vg.relax(10, 2.0)) for k in (vg.ISING, vg.HEISENBERG)]
+states = [s.wait(j).state for j in ids]
+s2 = {{l.split()[3] for l in log() if l.startswith("launch")}}
+print(len(s1), len(s2), states == [vg.JOB_DONE] * 2)
+""")
+    assert out.split() == ["1", "1", "True"]

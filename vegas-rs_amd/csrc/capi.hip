@@ -737,16 +737,17 @@ int state_done(hipStream_t st) {
     return fail(VG_ERR_DEVICE, "moving a state: %s", hipGetErrorString(e != hipSuccess ? e : w));
 }
 
-int make_side_stream(vg_batch* B) {
+void make_side_stream(vg_batch* B) {
     int used = 0;
     for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
-    if (used < 2 || B->side) return VG_OK;
+    if (used < 2 || B->side) return;
     hipError_t e = hipEventCreateWithFlags(&B->parted, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&B->joined, hipEventDisableTiming);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&B->side, hipStreamNonBlocking);
-    if (e == hipSuccess) return VG_OK;
+    if (e == hipSuccess) return;
+    quiet(hipGetLastError());
+    B->side = nullptr;
     free_side_stream(B);
-    return fail(VG_ERR_DEVICE, "second stream: %s", hipGetErrorString(e));
 }
 
 void free_side_stream(vg_batch* B) {
@@ -1334,13 +1335,7 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             }
         }
     }
-    {
-        const int rc = make_side_stream(B);
-        if (rc) {
-            free_batch(B);
-            return rc;
-        }
-    }
+    make_side_stream(B);
     const uint64_t rec_bytes = (uint64_t)n_chains * B->max_block_sweeps * 5u * sizeof(int64_t);
     hipError_t e = hipMalloc(&B->d_records, rec_bytes);
     if (e == hipSuccess) e = hipHostMalloc(&B->h_records, rec_bytes, hipHostMallocCoherent);

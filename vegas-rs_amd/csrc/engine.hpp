@@ -306,8 +306,9 @@ void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint3
 inline uint32_t reduce_block(uint32_t blocks) { return blocks > 1024 ? 1024u : vg::kBlock; }
 // A block of nsw sweeps on the batch's stream, its records to `records`.
 int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records);
-// The batch's second stream, made when its chains lie in several groups.
-int make_side_stream(vg_batch* B);
+// The batch's second stream, made when its chains lie in several groups; without
+// one (none can be made) every group runs on the first.
+void make_side_stream(vg_batch* B);
 void free_side_stream(vg_batch* B);
 // The same to the device's records, or, where the caller has a pinned buffer
 // for them (direct) and no graph is replayed, straight there.

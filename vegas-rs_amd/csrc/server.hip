@@ -246,8 +246,7 @@ int rebuild(vg_server* S) {
             G.partial_cap = cap;
         }
     }
-    const int rc = make_side_stream(&B);
-    if (rc) return rc;
+    make_side_stream(&B);
     const uint64_t words = (uint64_t)S->running.size() * Q * 5;
     if (words > S->records_cap) {
         if (S->d_records) quiet(hipFree(S->d_records));
