@@ -1,0 +1,51 @@
+"""What the engine's host code asks of the HIP runtime, and when: on the stand-in
+for it."""
+import pytest
+
+import _fake
+
+
+@pytest.mark.parametrize("spin", ["ISING", "HEISENBERG"])
+def test_state_buffer_is_made_with_the_batch(spin):
+    """The first download and upload allocate nothing; nor does a chain of another
+    size in the batch."""
+    out = _fake.run(f"""
+b = vg.Batch(ctx, [sc(8, spin=vg.{spin}), sc(20, spin=vg.{spin})])
+fake.fake_clear()
+if vg.{spin} == vg.ISING:
+    import numpy as np
+    b.set_ising(0, np.ones(512, dtype=np.int8)); b.set_ising(1, np.ones(8000, dtype=np.int8))
+    b.get_ising(0); b.get_ising(1)
+else:
+    b.set_heisenberg(0, [[0.0, 0.0, 1.0]] * 512); b.set_heisenberg(1, [[0.0, 0.0, 1.0]] * 8000)
+    b.get_heisenberg(0); b.get_heisenberg(1)
+print(sum(l.startswith("hostmalloc") for l in log()), sum(l.startswith("copy") for l in log()))
+""")
+    assert out.split() == ["0", "0"]
+
+
+def test_batch_without_a_state_buffer():
+    """Where the pinned memory for it cannot be had, states are copied."""
+    out = _fake.run("""
+fake.fake_fail(b"hipHostMalloc", 3)   # (after the two of the group's descriptors)
+b = vg.Batch(ctx, [sc(8)])
+fake.fake_clear()
+import numpy as np
+b.set_ising(0, np.ones(512, dtype=np.int8))
+b.run(2)
+print(sum(l.startswith("copy") for l in log()))
+""")
+    assert out.split() == ["1"]
+
+
+def test_server_makes_its_streams_at_creation():
+    out = _fake.run("""
+s = vg.Server(ctx, quantum_sweeps=10)
+fake.fake_clear()
+ids = [s.submit(sc(64, spin=k), vg.relax(10, 2.0)) for k in (vg.ISING, vg.HEISENBERG)]
+for j in ids: s.wait(j)
+s.close()
+print(sum(l.startswith("stream") for l in log()),
+      len({l.split()[3] for l in log() if l.startswith("launch")}))
+""")
+    assert out.split() == ["0", "2"]

@@ -594,10 +594,8 @@ int free_batch(vg_batch* B) {
         if (G.draws) quiet(hipFree(G.draws));
     }
     free_side_stream(B);
-    if (B->io) quiet(hipHostFree(B->io));
     if (B->d_records) quiet(hipFree(B->d_records));
     if (B->h_records) quiet(hipHostFree(B->h_records));
-    if (B->h_records2) quiet(hipHostFree(B->h_records2));
     for (hipEvent_t e : {B->ev0, B->ev1, B->ev2, B->ev3, B->done[0], B->done[1]})
         if (e) quiet(hipEventDestroy(e));
     delete B;
@@ -709,24 +707,13 @@ bool runs_passes(const Group& G, int g, bool timed) {
 // The batch's pinned buffer for `bytes` of a chain's state, or null: states of
 // at most kIoBytes go through it and the layout kernel reads or writes host
 // memory itself, for larger ones the caller allocates device memory and copies.
+// Made with the batch, so that no call pays for it.
 // us a download and an upload, allocated and copied, and so: 420 Ising sites 29
 // and 23, 15 and 17; 64000 54 and 155, 17 and 20 (with the spins checked in
 // blocks); 2.7 million 254 and 3130, 210 and 310; 1000 Heisenberg spins 38 and
 // 34, 16 and 15.
 void* state_buffer(vg_batch* B, uint64_t bytes) {
-    if (bytes > vg_batch::kIoBytes) return nullptr;
-    if (bytes > B->io_bytes) {
-        if (B->io) quiet(hipHostFree(B->io));
-        B->io = nullptr;
-        B->io_bytes = 0;
-        if (hipHostMalloc(&B->io, bytes, hipHostMallocCoherent) != hipSuccess) {
-            B->io = nullptr;
-            quiet(hipGetLastError());
-            return nullptr;
-        }
-        B->io_bytes = bytes;
-    }
-    return B->io;
+    return bytes <= B->io_bytes ? B->io : nullptr;
 }
 
 // The end of a call that gave a kernel the buffer: after an error too the kernel is
@@ -738,9 +725,7 @@ int state_done(hipStream_t st) {
 }
 
 void make_side_stream(vg_batch* B) {
-    int used = 0;
-    for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
-    if (used < 2 || B->side) return;
+    if (B->side) return;
     hipError_t e = hipEventCreateWithFlags(&B->parted, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&B->joined, hipEventDisableTiming);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&B->side, hipStreamNonBlocking);
@@ -1335,11 +1320,33 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             }
         }
     }
-    make_side_stream(B);
+    int used = 0;
+    for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
+    if (used > 1) make_side_stream(B);
     const uint64_t rec_bytes = (uint64_t)n_chains * B->max_block_sweeps * 5u * sizeof(int64_t);
     hipError_t e = hipMalloc(&B->d_records, rec_bytes);
-    if (e == hipSuccess) e = hipHostMalloc(&B->h_records, rec_bytes, hipHostMallocCoherent);
-    if (e == hipSuccess) e = hipHostMalloc(&B->h_records2, rec_bytes, hipHostMallocCoherent);
+    // One pinned allocation: both blocks' records and the state buffer (each
+    // allocation takes 12 us, its end 12 to 40, whatever the size).
+    uint64_t io = 0;
+    for (const ChainHost& ch : B->chains) {
+        const uint64_t bytes = ch.n_sites * (is_heis_lattice(ch.group) ? 3 * sizeof(double) : 1);
+        if ((is_zmarch(ch.group) || is_heis_lattice(ch.group)) && bytes <= vg_batch::kIoBytes)
+            io = std::max(io, bytes);
+    }
+    const uint64_t step = round_up(rec_bytes, 256);
+    if (e == hipSuccess && io &&
+        hipHostMalloc(&B->h_records, 2 * step + io, hipHostMallocCoherent) != hipSuccess) {
+        B->h_records = nullptr;
+        quiet(hipGetLastError());
+        io = 0;
+    }
+    if (e == hipSuccess && !B->h_records)
+        e = hipHostMalloc(&B->h_records, 2 * step, hipHostMallocCoherent);
+    if (e == hipSuccess) {
+        B->h_records2 = B->h_records + step / sizeof(int64_t);
+        B->io = B->h_records + 2 * step / sizeof(int64_t);
+        B->io_bytes = io;
+    }
     B->whole_blocks = true;
     for (hipEvent_t* ev : {&B->ev0, &B->ev1, &B->ev2, &B->ev3, &B->done[0], &B->done[1]})
         if (e == hipSuccess) e = hipEventCreate(ev);

@@ -235,12 +235,12 @@ struct vg_batch {
     vgi::Group groups[vgi::kNumGroups];
     uint32_t max_block_sweeps = 256;
     int64_t* d_records = nullptr;  // [chain][sweep][5]
-    int64_t* h_records = nullptr;  // pinned
-    int64_t* h_records2 = nullptr;  // pinned, for the block after (batches)
+    int64_t* h_records = nullptr;  // pinned; batches: h_records2 and io behind them
+    int64_t* h_records2 = nullptr;  // for the block after (batches)
     // Every chain runs every sweep of a block, so that the kernels write every
     // record (not in the job server, whose chains stop within a block).
     bool whole_blocks = false;
-    // Pinned buffer for the states of small chains, at most kIoBytes
+    // For the states of small chains, at most kIoBytes
     static constexpr uint64_t kIoBytes = 4 << 20;
     void* io = nullptr;
     uint64_t io_bytes = 0;
@@ -306,8 +306,8 @@ void launch_zmarch_pass(const Group& G, int g, hipStream_t st, uint32_t c, uint3
 inline uint32_t reduce_block(uint32_t blocks) { return blocks > 1024 ? 1024u : vg::kBlock; }
 // A block of nsw sweeps on the batch's stream, its records to `records`.
 int enqueue_block(vg_batch* B, uint32_t nsw, int64_t* records);
-// The batch's second stream, made when its chains lie in several groups; without
-// one (none can be made) every group runs on the first.
+// The batch's second stream, for chains in several groups; without one (none can
+// be made) every group runs on the first.
 void make_side_stream(vg_batch* B);
 void free_side_stream(vg_batch* B);
 // The same to the device's records, or, where the caller has a pinned buffer

@@ -246,7 +246,6 @@ int rebuild(vg_server* S) {
             G.partial_cap = cap;
         }
     }
-    make_side_stream(&B);
     const uint64_t words = (uint64_t)S->running.size() * Q * 5;
     if (words > S->records_cap) {
         if (S->d_records) quiet(hipFree(S->d_records));
@@ -557,6 +556,7 @@ int vg_server_create(vg_ctx* ctx, const vg_server_config* config, vg_server** ou
         quiet(hipStreamDestroy(S->own_ctx.stream));
         return fail(VG_ERR_DEVICE, "hipEventCreate: %s", hipGetErrorString(e));
     }
+    make_side_stream(&S->B);  // here, with no job waiting
     S->stats.pool_bytes = c.memory_bytes;
     S->t0 = std::chrono::steady_clock::now();
     vg_server* raw = S.release();
