@@ -49,3 +49,19 @@ print(sum(l.startswith("stream") for l in log()),
       len({l.split()[3] for l in log() if l.startswith("launch")}))
 """)
     assert out.split() == ["0", "2"]
+
+
+@pytest.mark.parametrize("change", ["set_tile(2)", "set_tie_capacity(3)"])
+def test_second_stream_for_groups_that_turn_to_passes(change):
+    """Small chains of two lattices run a block in one launch each; made to run
+    passes, they do so side by side."""
+    out = _fake.run(f"""
+b = vg.Batch(ctx, [sc(8), sc(8, kind=vg.BCC)])
+b.run(2)
+one = {{l.split()[3] for l in log() if l.startswith("launch")}}
+b.{change}
+fake.fake_clear()
+b.run(2)
+print(len(one), len({{l.split()[3] for l in log() if "_pass" in l}}))
+""")
+    assert out.split() == ["1", "2"]

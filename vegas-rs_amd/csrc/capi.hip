@@ -735,6 +735,13 @@ void make_side_stream(vg_batch* B) {
     free_side_stream(B);
 }
 
+// Makes a batch's second stream once several of its groups run passes.
+void side_stream_if_used(vg_batch* B) {
+    int used = 0;
+    for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
+    if (used > 1) make_side_stream(B);
+}
+
 void free_side_stream(vg_batch* B) {
     for (hipEvent_t* e : {&B->parted, &B->joined}) {
         if (*e) quiet(hipEventDestroy(*e));
@@ -1320,9 +1327,7 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             }
         }
     }
-    int used = 0;
-    for (int g = 0; g < kNumGroups; ++g) used += runs_passes(B->groups[g], g, false);
-    if (used > 1) make_side_stream(B);
+    side_stream_if_used(B);
     const uint64_t rec_bytes = (uint64_t)n_chains * B->max_block_sweeps * 5u * sizeof(int64_t);
     hipError_t e = hipMalloc(&B->d_records, rec_bytes);
     // One pinned allocation: both blocks' records and the state buffer (each
@@ -1770,6 +1775,7 @@ int vg_batch_set_tile(vg_batch* batch, uint32_t tile) {
         int rc = layout_work(batch, g, tile);
         if (rc) return rc;
     }
+    side_stream_if_used(batch);
     return VG_OK;
 }
 
@@ -1896,6 +1902,7 @@ int vg_batch_set_tie_capacity(vg_batch* batch, uint32_t records) {
         G.tie_cap = records;
         if (!G.members.empty()) G.resident = resident_sites(G, g);
     }
+    side_stream_if_used(batch);
     // captured graphs hold the old kernel arguments
     for (auto& kv : batch->graphs) quiet(hipGraphExecDestroy(kv.second));
     batch->graphs.clear();
