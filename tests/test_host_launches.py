@@ -65,3 +65,24 @@ b.run(2)
 print(len(one), len({{l.split()[3] for l in log() if "_pass" in l}}))
 """)
     assert out.split() == ["1", "2"]
+
+
+def test_draws_take_no_memory_from_the_rest():
+    """A batch that fits without the workspace for the draws of its small Heisenberg
+    chains is made, and runs passes: here one byte short of all."""
+    out = _fake.run("""
+descs = [sc(16, spin=vg.HEISENBERG, seed=k) for k in range(4)]
+descs.append(sc(16, proposal=vg.WOLFF))
+before = fake.fake_used()
+b = vg.Batch(ctx, descs)
+used = fake.fake_used() - before
+b.run(2)
+print(any("heis_draws" in l for l in launches()))
+b.close()
+fake.fake_limit(fake.fake_used() + used - 1)
+b = vg.Batch(ctx, descs)
+fake.fake_clear()
+b.run(2)
+print(any("heis_draws" in l for l in launches()), any("heis_sc_pass" in l for l in launches()))
+""")
+    assert out.split() == ["True", "False", "True"]

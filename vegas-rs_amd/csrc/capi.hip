@@ -1311,14 +1311,6 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             free_batch(B);
             return fail(VG_ERR_OUT_OF_MEMORY, "allocating partial sums: %s", hipGetErrorString(e));
         }
-        if (is_heis_lattice(g)) {
-            int rc = setup_heis_resident(G, g, B->max_block_sweeps);
-            if (rc) {
-                free_batch(B);
-                return rc;
-            }
-            refresh_wide(B, G);
-        }
         if (is_zmarch(g)) {
             int rc = layout_work(B, g, default_tile(G.host.data(), G.host.size()));
             if (rc) {
@@ -1327,7 +1319,6 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
             }
         }
     }
-    side_stream_if_used(B);
     const uint64_t rec_bytes = (uint64_t)n_chains * B->max_block_sweeps * 5u * sizeof(int64_t);
     hipError_t e = hipMalloc(&B->d_records, rec_bytes);
     // One pinned allocation: both blocks' records and the state buffer (each
@@ -1359,6 +1350,19 @@ int create_impl(vg_ctx* ctx, uint32_t n_chains, const vg_chain_desc* descs, cons
         free_batch(B);
         return fail(VG_ERR_DEVICE, "allocating records: %s", hipGetErrorString(e));
     }
+    // Workspaces that a batch can do without come last: they take no memory from
+    // what it cannot.
+    for (int g : {kHeisSc, kHeisBcc, kHeisFcc}) {
+        Group& G = B->groups[g];
+        if (G.members.empty()) continue;
+        int rc = setup_heis_resident(G, g, B->max_block_sweeps);
+        if (rc) {
+            free_batch(B);
+            return rc;
+        }
+        refresh_wide(B, G);
+    }
+    side_stream_if_used(B);
     for (int g = 0; g < kNumGroups; ++g) {
         int rc = upload_descriptors(B, g);
         if (rc) {
