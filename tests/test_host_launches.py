@@ -86,3 +86,25 @@ b.run(2)
 print(any("heis_draws" in l for l in launches()), any("heis_sc_pass" in l for l in launches()))
 """)
     assert out.split() == ["True", "False", "True"]
+
+
+def test_blocks_send_sweep_counters_only():
+    """Descriptors go to the device when something but the sweep counters has
+    changed: a thermostat, a tile."""
+    out = _fake.run("""
+b = vg.Batch(ctx, [sc(4, seed=k) for k in range(2000)])
+def sent(n):
+    fake.fake_clear()
+    b.run(n)
+    most = max(int(l.split()[-1]) for l in log() if l.startswith("copy"))
+    return int(most > 2000 * n * 40), sum("set_sweeps" in l for l in launches())
+print(*sent(1), *sent(1), *sent(2), *sent(300))
+b.set_thermostat(7, 2.0)
+print(*sent(1), *sent(1))
+b.set_tile(2)
+print(*sent(1), *sent(1))
+b.set_sweep_count(3, 77)
+print(*sent(1))
+""")
+    # (descriptors sent, launches for counters)
+    assert out.split("\n")[:4] == ["0 0 0 1 0 1 0 2", "1 0 0 1", "1 0 0 1", "0 1"]

@@ -71,6 +71,7 @@ __global__ void heis_scatter(const ChainDev*, float*, const double*, uint64_t);
 __global__ void heis_gather(const ChainDev*, const float*, double*, uint64_t);
 __global__ void zero_i64(int64_t*, uint64_t);
 __global__ void copy_words(const uint32_t*, uint32_t*, uint32_t);
+__global__ void set_sweeps(const uint64_t*, ChainDev*, uint32_t);
 // Graph chains (an arbitrary exchange matrix): one pass per colour class,
 // args (chains, block -> chain map, arena, partials, colour, sweep, total
 // blocks, passes per sweep); initial states.
@@ -155,7 +156,10 @@ inline uint64_t sites_of(const vg_lattice& L) {
 struct Group {
     std::vector<uint32_t> members;  // batch chain indices
     std::vector<ChainDev> host;     // descriptors, uploaded each sweep block
-    std::vector<ChainDev> sent;     // what d_chains holds
+    // What d_chains holds: descriptors as in host (`stale`: or not, whatever sets
+    // anything in host but sweep0 says so), with these sweep0
+    bool stale = true;
+    std::vector<uint64_t> sent_sweeps;
     ChainDev* d_chains = nullptr;
     ChainDev* h_staging = nullptr;  // pinned copy used for the upload
     ChainDev* h_staging2 = nullptr;  // second one, for the block after (batches)

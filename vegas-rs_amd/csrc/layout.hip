@@ -189,6 +189,13 @@ __global__ void copy_words(const uint32_t* __restrict__ from, uint32_t* __restri
     if (i < n) to[i] = from[i];
 }
 
+// The chains' sweep counters, from pinned host memory.
+__global__ void set_sweeps(const uint64_t* __restrict__ from, ChainDev* __restrict__ chains,
+                           uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) chains[i].sweep0 = from[i];
+}
+
 // Zero n int64 words (used for per-block records; a kernel rather than a
 // memset so the sweep block can be captured in a graph).
 __global__ void zero_i64(int64_t* __restrict__ p, uint64_t n) {

@@ -225,7 +225,6 @@ int rebuild(vg_server* S) {
             if (G.h_staging) quiet(hipHostFree(G.h_staging));
             G.d_chains = nullptr;
             G.h_staging = nullptr;
-            G.sent.clear();
             G.chains_cap = 0;
             const uint32_t cap = (uint32_t)std::max<size_t>(16, G.host.size() * 2);
             VG_HIP(hipMalloc(&G.d_chains, cap * sizeof(ChainDev)));
@@ -297,6 +296,7 @@ int quantum(vg_server* S, uint32_t& nsw_out) {
     for (int g = 0; g < kNumGroups; ++g) {
         Group& G = B.groups[g];
         for (size_t k = 0; k < G.members.size(); ++k) G.host[k] = S->running[G.members[k]]->dev;
+        G.stale = true;
         int rc = upload_descriptors(&B, g);
         if (rc) return rc;
     }
