@@ -288,7 +288,6 @@ def run_batched(vg, ctx, sweeps, baseline_sweeps, n_chains=512, cpu=None):
         for i, (T, h, d) in enumerate(therm):
             b.set_thermostat(i, T, h, d)
         tile = b.autotune(30)  # 30 trial sweeps per tile: a stable pick
-        b.set_tile(tile)
         b.set_graph(True)
         b.run(10)
         b.prepare(sweeps)
@@ -340,7 +339,6 @@ def run_bitpacked(vg, ctx, side, sweeps):
         for i, T in enumerate(temps):
             b.set_thermostat(i, T)
         tile = b.autotune(50)
-        b.set_tile(tile)
         b.set_graph(True)
         b.run(10)
         b.prepare(sweeps)
@@ -370,14 +368,13 @@ def run_bitpacked(vg, ctx, side, sweeps):
 def run_resident(vg, ctx, side, sweeps):
     """One int8 Ising chain of sc side^3 at T_c = 4.5115 (J = 1, h = 0, seed
     7), held one bit per site like every Ising chain: 134 MB at 1024^3.
-    Attempts/s and the pass kernel's roofline at 2 B per attempt."""
+    Attempts/s and the pass kernel's roofline at 0.25 B per attempt."""
     L = vg.lattice(vg.SC, side, side, side)
     n = side ** 3
     with vg.Batch(ctx, [vg.chain(L, vg.ISING, vg.FLIP, vg.hamiltonian(exchange=1.0), 7)]) as b:
         b.randomize()
         b.set_thermostat(0, 4.5115)
         tile = b.autotune(4)
-        b.set_tile(tile)
         b.set_graph(True)
         b.run(4)
         b.prepare(sweeps)
@@ -388,7 +385,7 @@ def run_resident(vg, ctx, side, sweeps):
     value = n * sweeps / wall
     per_launch = n // 2
     avg_ms = dev_ms / (2 * sweeps)
-    achieved = 2 * per_launch / (avg_ms * 1e-3) / 1e9
+    achieved = 0.25 * per_launch / (avg_ms * 1e-3) / 1e9
     log(f"resident sc {side}^3: {value:.4e} attempts/s, pass {avg_ms * 1e3:.1f} us, tile {tile}")
     return {
         "workload": (f"ising-sc{side}-i8: one chain sc {side}^3 at T=4.5115 (int8 chain, one bit "
@@ -400,7 +397,7 @@ def run_resident(vg, ctx, side, sweeps):
         "roofline": with_counters(
             {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
              "frac": achieved / HBM_PEAK_GBS, "kernel": "ising_sc_pass",
-             "algorithmic_bytes_per_launch": 2 * per_launch, "mean_launch_us": avg_ms * 1e3},
+             "algorithmic_bytes_per_launch": per_launch // 4, "mean_launch_us": avg_ms * 1e3},
             "resident", [f"ising_sc_pass<{tile},2>"], ising_mads(per_launch)),
     }
 
@@ -477,7 +474,8 @@ def run_fcc(vg, ctx, cells, heis_cells, sweeps, kind=None):
     and 3 Heisenberg chains of heis_cells^3 cells (J = 1, K = 0.1 z, B = 0.05
     z, uniform-sphere proposals; T = 1.5, 3.2, 5), random starts from seed 7.
     The Ising chains run again stored one bit per site.  Attempts/s and each
-    pass kernel's roofline (2 B / 0.25 B / 24 B per attempt).
+    pass kernel's roofline (0.25 B an Ising attempt, whichever spin kind,
+    24 B a Heisenberg one).
     With kind = vg.BCC the same on bcc lattices (2 sites per cell, two colour
     passes; Ising T = 5, 6.35, 8 around T_c ~ 6.35, Heisenberg T = 1, 2.1, 3.5)."""
     bcc = kind == vg.BCC
@@ -512,7 +510,7 @@ def run_fcc(vg, ctx, cells, heis_cells, sweeps, kind=None):
         value = n * len(temps) * sweeps / wall
         per_launch = n * len(temps) // passes
         avg_ms = dev_ms / (passes * sweeps)
-        bpa = {"ising": 2, "ising_bits": 0.25, "heisenberg": 24}[spin]
+        bpa = 0.25 if ising else 24  # (both Ising kinds are held one bit per site)
         achieved = bpa * per_launch / (avg_ms * 1e-3) / 1e9
         log(f"{name} {spin}: {value:.4e} attempts/s, pass {avg_ms * 1e3:.1f} us -> "
             f"{achieved:.0f} GB/s")
@@ -842,8 +840,9 @@ def main():
     batch.randomize()
     for i, T in enumerate(temps):
         batch.set_thermostat(i, T)
-    tile = batch.autotune(50) if args.tile == 0 else args.tile
-    batch.set_tile(tile)
+    if args.tile:
+        batch.set_tile(args.tile)
+    tile = args.tile or batch.autotune(50)  # (autotune keeps its pick)
     batch.set_graph(args.graph)
     log(f"bench: {len(temps)} chains sc {side}^3 int8, warmup {args.warmup}")
     if args.warmup:
@@ -873,7 +872,8 @@ def main():
     ev_ms, ev_launches = batch.pass_stats(vg.ISING)
     batch.set_timing(False)
     attempts_per_launch = attempts_per_step // 2
-    alg_bytes = 2 * attempts_per_launch  # read + write of each site once per sweep
+    # each site's bit read and written once per sweep (int8 spins are held so)
+    alg_bytes = attempts_per_launch // 4
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
     log(f"bench: pass kernel {avg_ms * 1e3:.1f} us/launch -> {achieved:.0f} GB/s algorithmic")
 
