@@ -258,7 +258,10 @@ int vg_batch_get_tile(const vg_batch* batch, uint32_t* tile);
  * beforehand, five rounds over the tiles, the median of each) and keeps the
  * fastest, for each of the three groups.  The chains' spins and sweep counters are
  * restored after every trial, so tuning does not change any trajectory.
- * Groups of small chains that run without passes are left as they are. */
+ * Groups of small chains that run without passes are left as they are.  The
+ * tile returned is that of the first group, for the caller's information:
+ * every group has its own already, and setting it with vg_batch_set_tile
+ * would give all groups the one and put small chains on passes. */
 int vg_batch_autotune(vg_batch* batch, uint32_t trial_sweeps, uint32_t* chosen_tile);
 /* Records (0..128, default 128) the per-wave tie queue of the Ising sc, bcc
  * and fcc passes may hold before a wave settles further tied rows in the
@@ -271,7 +274,10 @@ int vg_batch_last_run_ms(const vg_batch* batch, double* ms);
 /* Per-launch timing of the colour-pass kernels: when enabled (plain launches
  * only), every pass launch is bracketed by a hipEvent pair on the batch
  * stream; vg_batch_pass_stats returns the accumulated kernel time and launch
- * count of the pass kernel used by `spin` chains.  Enabling resets them. */
+ * count of the pass kernel used by `spin` chains.  Enabling resets them.
+ * Small chains, whose sweep blocks are otherwise one launch or two, run as
+ * passes while it is enabled, and every group on the batch's one stream: the
+ * times are those of the pass kernels, not a part of an untimed run's. */
 int vg_batch_set_timing(vg_batch* batch, int enabled);
 int vg_batch_pass_stats(const vg_batch* batch, int32_t spin, double* total_ms, uint64_t* launches);
 

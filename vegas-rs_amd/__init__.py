@@ -394,6 +394,7 @@ class Batch:
         _check(_lib.vg_batch_set_tie_capacity(self.h, records))
 
     def set_timing(self, enabled: bool) -> None:
+        """Times every colour pass; small chains run as passes meanwhile."""
         _check(_lib.vg_batch_set_timing(self.h, 1 if enabled else 0))
 
     def pass_stats(self, spin: int = ISING):

@@ -166,9 +166,8 @@ struct Group {
     uint32_t* d_block_chain = nullptr;
     uint32_t block_chain_cap = 0;
     uint32_t tile = 4;  // Ising sc/bcc/fcc: z planes per work item (template parameter)
-    // Ising sc/bcc/fcc: the pass's form (vg::IsingMode) -- one bit per site,
-    // with every chain periodic along every axis or not, or the caller's byte
-    // planes (the allocation-free entry point)
+    // Ising sc/bcc/fcc: the pass's form (vg::IsingMode), with every chain
+    // periodic along every axis or not
     uint32_t mode = 1;
     uint32_t total_blocks = 0;
     uint32_t grid = 0;  // total_blocks rounded up to a multiple of 8

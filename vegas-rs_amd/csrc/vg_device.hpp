@@ -380,10 +380,6 @@ __device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off)
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
 
-__device__ __forceinline__ uint32_t bload8(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    return __builtin_amdgcn_raw_buffer_load_b8(r, off, 0, 0);
-}
-
 // 24-bit uniform in [0,1) and in [-1,1) from a 32-bit draw (exact in fp32).
 VG_HD float unit24(uint32_t w) { return (float)(w >> 8) * 5.9604644775390625e-08f; }
 VG_HD float sym24(uint32_t w) { return (float)(w >> 8) * 1.1920928955078125e-07f - 1.0f; }
