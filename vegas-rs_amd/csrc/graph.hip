@@ -23,6 +23,8 @@
 // 2 x 4 for Heisenberg) and its neighbours' spins by gather; this path is
 // for generality (any lattice or coupling set), the stencil passes are the
 // fast path for sc, bcc and fcc.
+#include <type_traits>
+
 #include "heis_common.hpp"
 
 namespace vg {
@@ -36,6 +38,10 @@ namespace vg {
 // left is the launch, the descriptor, entries, spins, the f64 arithmetic and
 // the sums, one after the other.
 constexpr uint32_t kGather = 8;
+// Ising rows all of at most this many entries take so many at once: reading the last
+// one again costs what eight do.  us a pass, a loop over entries, eight and two at
+// once: 200000 sites in pairs 4.9, 5.0, 4.1; a ring of 2^20 11.2, 10.9, 7.8.
+constexpr uint32_t kShort = 2;
 
 // What a pass's wave needs of its chain, loaded in one batch before anything
 // is decided: field by field where each is used, the scalar loads were a chain
@@ -118,27 +124,34 @@ __global__ __launch_bounds__(256) void graph_ising_pass(const ChainDev* __restri
             e0 = ptr[p];
             e1 = ptr[p + 1];
         }
-        for (; e0 < e1; e0 += kGather) {
-            uint32_t j[kGather], bj[kGather];
-            double aj[kGather], wj[kGather];
+        const auto gather = [&](auto width) {
+            constexpr uint32_t N = decltype(width)::value;
+            for (; e0 < e1; e0 += N) {
+                uint32_t j[N], bj[N];
+                double aj[N], wj[N];
 #pragma unroll
-            for (uint32_t k = 0; k < kGather; ++k) {
-                const uint32_t e = min(e0 + k, e1 - 1u);
-                j[k] = nbr[e];
-                aj[k] = a[e];
-                wj[k] = w[e];
+                for (uint32_t k = 0; k < N; ++k) {
+                    const uint32_t e = min(e0 + k, e1 - 1u);
+                    j[k] = nbr[e];
+                    aj[k] = a[e];
+                    wj[k] = w[e];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < N; ++k) bj[k] = spin[j[k]];
+#pragma unroll
+                for (uint32_t k = 0; k < N; ++k) {
+                    const double sj = bj[k] ? 1.0 : -1.0;
+                    const double hk = __dadd_rn(h, __dmul_rn(aj[k], sj));
+                    const double hbk = __dadd_rn(hb, __dmul_rn(wj[k], sj));
+                    h = e0 + k < e1 ? hk : h;
+                    hb = e0 + k < e1 ? hbk : hb;
+                }
             }
-#pragma unroll
-            for (uint32_t k = 0; k < kGather; ++k) bj[k] = spin[j[k]];
-#pragma unroll
-            for (uint32_t k = 0; k < kGather; ++k) {
-                const double sj = bj[k] ? 1.0 : -1.0;
-                const double hk = __dadd_rn(h, __dmul_rn(aj[k], sj));
-                const double hbk = __dadd_rn(hb, __dmul_rn(wj[k], sj));
-                h = e0 + k < e1 ? hk : h;
-                hb = e0 + k < e1 ? hbk : hb;
-            }
-        }
+        };
+        if (H.w - 1u < kShort)
+            gather(std::integral_constant<uint32_t, kShort>{});
+        else
+            gather(std::integral_constant<uint32_t, kGather>{});
         // The decision is computed without branches and applied by one
         // select: written as `if (dE <= 0 || u < p) flip`, the accept
         // block has two predecessors, and hipcc for gfx950 (ROCm 7.2)
