@@ -294,7 +294,7 @@ int upload_descriptors(vg_batch* B, int g, int slot) {
     if (!G.stale) {
         // Only sweep counters can differ: from block to block they alone are sent
         // (whole descriptors of 16384 chains of 4^3, 19 MB: 810 us for one sweep,
-        // FIG so).
+        // 240 so).
         bool same = true;
         for (size_t k = 0; k < n; ++k) same = same && G.sent_sweeps[k] == G.host[k].sweep0;
         if (same) return VG_OK;
